@@ -27,6 +27,7 @@
  */
 #include <hip/hip_runtime.h>
 #include <climits>
+#include <type_traits>
 #include "lxs_kernels.h"
 #include "lxs_mfma.h"
 
@@ -251,19 +252,31 @@ __global__ void __launch_bounds__(64 * NWI) smm_mfma(T* __restrict__ cdata, cons
 }
 
 /*
- * Entry-parallel form for short runs: the EP wavefronts of a work-group share each C-run. Wavefront q
- * takes the run's entries h+q, h+q+EP, ... (each wavefront covers the whole C block with TI x TJ tiles, the
- * same rolling fragment loads as smm_mfma), then the EP partial blocks meet in LDS and are added in a
- * fixed order (wavefront 0 first), the tiles of the block shared out among the wavefronts for that sum
- * and the flush. So a run that is not cut gives the same bits on every call whatever the timing, and a
- * run of L entries costs each wavefront about L/EP entries instead of L (runs of ~30 entries and a few
- * thousand of them leave one wavefront per run too little memory parallelism).
+ * Entry-parallel form for short runs: the EP wavefronts of a work-group share each C-run, then the EP
+ * partial blocks meet in LDS and are added in a fixed order (wavefront 0 first), the tiles of the block
+ * shared out among the wavefronts for that sum and the flush. So a run that is not cut gives the same bits on
+ * every call whatever the timing, and a run of L entries costs each wavefront about L/EP entries instead of L
+ * (runs of ~30 entries and a few thousand of them leave one wavefront per run too little memory parallelism).
+ * The work is split along one flat k: the k of the run's entries form one sequence of L k terms, cut into steps
+ * of one matrix-core instruction (4 of k, or 16 with B4 = 2); wavefront q takes a contiguous 1/EP of the steps,
+ * and each lane finds its own entry and k (f / K by a 24-bit multiplication, the entries' A and B offsets in a
+ * table of 64 in LDS). So k is padded once per run instead of once per entry, the wavefronts' shares
+ * differ by at most one step, and a stage of KB steps is full of loads whatever K is. What bounds these kernels
+ * is the latency of that chain of stages and, for the larger stacks, the operand bytes behind L2.
+ * Against whole entries per wavefront (each entry its own stages, its last one partly empty), us:
+ *   f64 20x46x42 S=9839 73.5 -> 44.7, 25x5x6 S=99306 45.1 -> 30.2, 5^3 S=500000 70.2 -> 45.8, 45x45x13 S=100000
+ *   234 -> 201, 64^3 S=100000 1315 -> 1250, 13^3 S=30000 18.5 -> 16.6, 23^3 S=30000 45.7 -> 44.8, S=500000 636 -> 625;
+ *   f32 14x30x8 S=205558 80.1 -> 56.7, 60x50x40 S=20000 201 -> 150, 5^3 S=500000 68.6 -> 53.7; 32^3 f64 unchanged
+ *   (241: every stage was full before), 4x9x22 f64 S=500000 unchanged (163: 7 TB/s of operands).
+ * Steps past a wavefront's share are loaded from its last k (one column, so the loads cost little) and not
+ * multiplied: loads under branches there cost 64^3 17% and 13^3 11%, since the compiler then waits for all of them.
+ * Ranges of a run are counted from its start, in 64 entries (1 entry for k above 512), so the split, and with it
+ * the bits, do not depend on where the run lies in the work-group's share.
  * Run ownership and cuts as in smm_mfma: the work-group owns the runs whose first entry lies in
  * [w*bs, (w+1)*bs); a run continues past that range until its C block changes or a segment boundary
  * past it cuts the run (lxs_cut). The end of a run is found by a 64-wide ballot over the C indices
  * (every wavefront computes it, so all take the same path through the barriers).
- * Barriers wait for LDS only (a fence restricted to the local address space), so fragment loads of the
- * next run stay in flight across them.
+ * Barriers wait for LDS only (a fence restricted to the local address space).
  *
  * B4 (FP64, smm_mfma_eb): the same run protocol on 4x4 blocks instead of 16x16 tiles. v_mfma_f64_4x4x4_4b
  * multiplies four independent 4x4x4 blocks at the FP64 matrix-core rate of the 16x16x4 form (a quarter of
@@ -291,35 +304,49 @@ __device__ __forceinline__ void ep_body(T* __restrict__ cdata, const T* __restri
   constexpr int SEG_LEN = 16; /* entries per matrix-core accumulation before the fold into the run total */
   constexpr int NTILE = TI * TJ; /* 16x16 tiles, or (B4) 4x4-block instructions per k-step */
   const int M = (0 < MC ? MC : m_rt), N = (0 < NC ? NC : n_rt), K = (0 < KC ? KC : k_rt);
-  const int KS = (2 == B4 ? (K + 15) >> 4 : (K + 3) >> 2); /* k-steps of 4 (B4 = 2: of 16, 4 per block) */
-  const int NS = (KS + KB - 1) / KB; /* k-stages per entry */
+  constexpr int KW = (2 == B4 ? 16 : 4); /* k per k-step */
+  const int SEG = SEG_LEN * ((K + KW - 1) / KW); /* k-steps per matrix-core accumulation */
+  /* f / K = (f kinv) >> ksh for the flat indices f of a table: f < we K and f (K kinv - 2^ksh) < we K^2 <= 2^ksh */
+  constexpr int WE = 64; /* entries of a table */
+  const int ksh = (K <= 128 ? 20 : 24), we = (K <= 512 ? WE : 1);
+  const unsigned int kinv = (K <= 512 ? ((1u << ksh) + (unsigned int)K - 1) / (unsigned int)K : 0u);
   const int lane = threadIdx.x & 63;
   const int q = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int li = lane & 15, lk = lane >> 4;
   extern __shared__ double lxs_smem[];
   /* partial blocks: [EP][NTILE][4][64] (16x16 tiles), [EP][NTILE][64] (B4 = 1), [EP][NTILE][16] (B4 = 2) */
   T* const red = reinterpret_cast<T*>(lxs_smem);
+  /* A and B offsets of the entries tb .. tb + we - 1, each wavefront its own copy (no barrier) */
+  __shared__ int2 tab[EP][WE];
+  int tb;
   (void)kt_unused;
 
   const int begin = blockIdx.x * bs;
   const int end = min(begin + bs, stack_size);
-  /* WIN: the stack around the work-group's entries is held in registers: lane l has the C, A and B offsets of
+  /* WIN: the stack around the work-group's entries is held in registers: lane l has the C offset of
      entry begin + l and the C offset of entry begin - 64 + l (NONE outside the stack). The head and run-end
-     scans, the cut tests and the entries' A and B offsets then come from these registers (shuffles and
-     readlanes in wave-uniform code) instead of chains of dependent loads; entries outside the window are
-     loaded. Kernels of 16 tiles or more keep loading: their accumulators leave no registers for the window
-     (a spilled window register reloaded under a partial EXEC mask would feed the readlanes stale lanes). */
+     scans and the cut tests then come from these registers (shuffles and readlanes in wave-uniform code) instead
+     of chains of dependent loads; entries outside the window are loaded. Kernels of 16 tiles or more keep
+     loading: their accumulators leave no registers for the window (a spilled window register reloaded under a
+     partial EXEC mask would feed the readlanes stale lanes). */
   constexpr bool WIN = (NTILE < 16) || (2 == B4 && NTILE <= 16); /* B4 = 2: one register pair per instruction */
   constexpr int NONE = INT_MIN; /* no C block: differs from every offset */
   const int wi = begin + lane, pi = begin - 64 + lane;
   const bool win = (wi < stack_size);
-  int wc = NONE, wa = 0, wb = 0, pc = NONE;
+  int wc = NONE, pc = NONE;
+  const auto load_tab = [&](int x) {
+    const int e = x + lane;
+    const bool in = (e < stack_size);
+    tab[q][lane] = make_int2(in ? stack[ps * e + 0] - pz : 0, in ? stack[ps * e + 1] - pz : 0);
+    tb = x;
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  };
   if constexpr (WIN) {
     wc = (win ? stack[ps * wi + 2] : NONE);
-    wa = (win ? stack[ps * wi + 0] - pz : 0);
-    wb = (win ? stack[ps * wi + 1] - pz : 0);
     pc = (0 <= pi ? stack[ps * pi + 2] : NONE);
   }
+  load_tab(begin);
   /* C offset of a wave-uniform entry j (NONE outside the stack) */
   const auto c_uni = [&](int j) -> int {
     if constexpr (WIN) {
@@ -327,19 +354,6 @@ __device__ __forceinline__ void ep_body(T* __restrict__ cdata, const T* __restri
       if (begin - 64 <= j && j < begin) return __builtin_amdgcn_readlane(pc, j - begin + 64);
     }
     return (0 <= j && j < stack_size) ? stack[ps * j + 2] : NONE;
-  };
-  /* A and B offsets of a wave-uniform entry e of the stack */
-  const auto a_uni = [&](int e) -> int {
-    if constexpr (WIN) {
-      if (begin <= e && e < begin + 64) return __builtin_amdgcn_readlane(wa, e - begin);
-    }
-    return stack[ps * e + 0] - pz;
-  };
-  const auto b_uni = [&](int e) -> int {
-    if constexpr (WIN) {
-      if (begin <= e && e < begin + 64) return __builtin_amdgcn_readlane(wb, e - begin);
-    }
-    return stack[ps * e + 1] - pz;
   };
   /* first piece head in [begin, end): a run head, or begin where it cuts a long run (lxs_cut) */
   int h = end;
@@ -489,123 +503,121 @@ __device__ __forceinline__ void ep_body(T* __restrict__ cdata, const T* __restri
     folded = true;
   };
 
-#define LXS_LOAD_KSTEP(KBI, A0, B0, KSTEP) \
-  do { \
-    const int k_ = (2 == B4 ? 16 * (KSTEP) + lxs::mfma4<T>::klane(lane) : 4 * (KSTEP) + lk); \
-    const bool kv_ = (k_ < K); \
-    if constexpr (0 != B4) { \
-      _Pragma("unroll") for (int p_ = 0; p_ < TI2; ++p_) { \
-        qa[KBI][p_] = lxs::gload2(kv_ ? (adata + ((A0) + k_ * M + min(r4 + 2 * p_, M - 2))) : zeros); \
-      } \
-      if constexpr (0 != TI % 2) fa[KBI][0] = gload(kv_ ? (adata + ((A0) + k_ * M + min(r4 + TI - 1, M - 1))) : zeros); \
-      _Pragma("unroll") for (int p_ = 0; p_ < TJ2; ++p_) { \
-        qb[KBI][p_] = lxs::gload2(kv_ ? (bdata + ((B0) + k_ * N + min(c4 + 2 * p_, N - 2))) : zeros); \
-      } \
-      if constexpr (0 != TJ % 2) fb[KBI][0] = gload(kv_ ? (bdata + ((B0) + k_ * N + min(c4 + TJ - 1, N - 1))) : zeros); \
-    } \
-    else if constexpr (PAIR) { \
-      _Pragma("unroll") for (int p_ = 0; p_ < PI; ++p_) { \
-        pa[KBI][p_] = lxs::gload2(kv_ ? (adata + ((A0) + k_ * M + aoff[2 * p_])) : zeros); \
-      } \
-      _Pragma("unroll") for (int p_ = 0; p_ < PJ; ++p_) { \
-        pb[KBI][p_] = lxs::gload2(kv_ ? (bdata + ((B0) + k_ * N + boff[2 * p_])) : zeros); \
-      } \
-    } \
-    else { \
-      _Pragma("unroll") for (int ti = 0; ti < TI; ++ti) { \
-        fa[KBI][ti] = gload(kv_ ? (adata + ((A0) + k_ * M + aoff[ti])) : zeros); \
-      } \
-      _Pragma("unroll") for (int tj = 0; tj < TJ; ++tj) { \
-        fb[KBI][tj] = gload(kv_ ? (bdata + ((B0) + k_ * N + boff[tj])) : zeros); \
-      } \
-    } \
-  } while (0)
+  /* loads of one k-step into slot kb: this lane's k of the step is the flat index f of the piece's entries from x0
+     on (entry f / K, k = f % K), clamped to the last one; the caller zeroes what lies past it */
+  const int kl = (2 == B4 ? lxs::mfma4<T>::klane(lane) : lk);
+  int x0 = 0, flast = 0; /* first entry of the range being summed, last flat index of this wavefront's part */
+  const auto load_step = [&](int kb, int f) {
+    const int fc = min(f, flast);
+    const int en = (int)(__umul24(fc, kinv) >> ksh);
+    const int k = fc - (int)__umul24(en, K);
+    const int2 ab = tab[q][(x0 - tb + en) & (WE - 1)];
+    const T* const ap = adata + (ab.x + (int)__umul24(k, M));
+    const T* const bp = bdata + (ab.y + (int)__umul24(k, N));
+    if constexpr (0 != B4) {
+#pragma unroll
+      for (int p = 0; p < TI2; ++p) qa[kb][p] = lxs::gload2(ap + min(r4 + 2 * p, M - 2));
+      if constexpr (0 != TI % 2) fa[kb][0] = gload(ap + min(r4 + TI - 1, M - 1));
+#pragma unroll
+      for (int p = 0; p < TJ2; ++p) qb[kb][p] = lxs::gload2(bp + min(c4 + 2 * p, N - 2));
+      if constexpr (0 != TJ % 2) fb[kb][0] = gload(bp + min(c4 + TJ - 1, N - 1));
+    }
+    else if constexpr (PAIR) {
+#pragma unroll
+      for (int p = 0; p < PI; ++p) pa[kb][p] = lxs::gload2(ap + aoff[2 * p]);
+#pragma unroll
+      for (int p = 0; p < PJ; ++p) pb[kb][p] = lxs::gload2(bp + boff[2 * p]);
+    }
+    else {
+#pragma unroll
+      for (int ti = 0; ti < TI; ++ti) fa[kb][ti] = gload(ap + aoff[ti]);
+#pragma unroll
+      for (int tj = 0; tj < TJ; ++tj) fb[kb][tj] = gload(bp + boff[tj]);
+    }
+  };
+  /* the k-step in slot kb; MASK: operands are zeroed where this lane's k lies past the range (not valid) */
+  const auto mma_step = [&](auto mask, int kb, bool valid) {
+    constexpr bool MASK = decltype(mask)::value;
+    T av[TI], bv[TJ];
+    if constexpr (0 != B4) {
+#pragma unroll
+      for (int p = 0; p < TI2; ++p) {
+        av[2 * p] = (a4x[p] ? qa[kb][p][1] : qa[kb][p][0]);
+        av[2 * p + 1] = qa[kb][p][1];
+      }
+      if constexpr (0 != TI % 2) av[TI - 1] = fa[kb][0];
+#pragma unroll
+      for (int p = 0; p < TJ2; ++p) {
+        bv[2 * p] = (b4x[p] ? qb[kb][p][1] : qb[kb][p][0]);
+        bv[2 * p + 1] = qb[kb][p][1];
+      }
+      if constexpr (0 != TJ % 2) bv[TJ - 1] = fb[kb][0];
+    }
+    else {
+#pragma unroll
+      for (int ti = 0; ti < TI; ++ti) {
+        if constexpr (PAIR) av[ti] = pa[kb][ti >> 1][ti & 1];
+        else av[ti] = fa[kb][ti];
+      }
+#pragma unroll
+      for (int tj = 0; tj < TJ; ++tj) {
+        if constexpr (PAIR) bv[tj] = pb[kb][tj >> 1][tj & 1];
+        else bv[tj] = fb[kb][tj];
+      }
+    }
+    if constexpr (MASK) {
+#pragma unroll
+      for (int ti = 0; ti < TI; ++ti) av[ti] = (valid ? av[ti] : T(0));
+#pragma unroll
+      for (int tj = 0; tj < TJ; ++tj) bv[tj] = (valid ? bv[tj] : T(0));
+    }
+#pragma unroll
+    for (int ti = 0; ti < TI; ++ti) {
+#pragma unroll
+      for (int tj = 0; tj < TJ; ++tj) {
+        if constexpr (0 != B4) prod4[ti][tj] = lxs::mfma4<T>::mma(av[ti], bv[tj], prod4[ti][tj]);
+        else prod[ti][tj] = mfma<T>::mma(av[ti], bv[tj], prod[ti][tj]);
+      }
+    }
+  };
 
-  int e = -1, a0 = 0, b0 = 0; /* entry whose first k-stage is in flight in the fragment registers */
-  for (;;) {                  /* one run (or piece of a cut run) [h, r) per iteration */
+  for (;;) { /* one run (or piece of a cut run) [h, r) per iteration */
     const int c0 = c_uni(h);
     const int r = run_end(h, c0);
     /* a piece that starts or ends inside a run shares its C block with another work-group */
     const bool flush_atomic = atomic || (0 < h && c_uni(h - 1) == c0) || (r < stack_size && c_uni(r) == c0);
     const bool own_next = (r < end);
-    int cur = h + q;
-    if (cur < r) {
-      if (cur != e) { /* not prefetched: load the first k-stage now */
-        a0 = a_uni(cur);
-        b0 = b_uni(cur);
+    int nseg = 0; /* k-steps since the last fold */
+    for (int x = h; x < r; x += we) { /* ranges of up to we entries, counted from the run's start */
+      const int nent = min(r - x, we);
+      if (x < tb || tb + we < x + nent) load_tab(x);
+      x0 = x;
+      const int flen = nent * K;
+      /* this wavefront's k-steps [s0, s1) of the range */
+      const int steps = (flen + KW - 1) / KW;
+      const int s0 = steps * q / EP, s1 = steps * (q + 1) / EP;
+      if (s0 < s1) {
+        flast = min(KW * s1, flen) - 1;
+        int f = KW * s0 + kl, n = s1 - s0;
 #pragma unroll
-        for (int kb = 0; kb < KB; ++kb) {
-          if (kb < KS) LXS_LOAD_KSTEP(kb, a0, b0, kb);
-        }
-      }
-      int nent = 0;
-      for (;;) { /* one entry of this wavefront per iteration */
-        const int nx = cur + EP;
-        const bool in_run = (nx < r);
-        /* after the run: this wavefront's first entry of the next run, if the work-group owns it */
-        const int cand = r + q;
-        const bool pre = !in_run && own_next && cand < stack_size;
-        const int nxt = (in_run ? nx : (pre ? cand : -1));
-        const int na = (0 <= nxt ? a_uni(nxt) : a0), nb = (0 <= nxt ? b_uni(nxt) : b0);
-        for (int s = 0; s < NS; ++s) {
-          const bool last = (s + 1 == NS);
-          const int la = (last ? na : a0), lb = (last ? nb : b0), ns = (last ? 0 : s + 1);
+        for (int kb = 0; kb < KB; ++kb) load_step(kb, f + KW * kb);
+        for (; KB < n; n -= KB, f += KW * KB) { /* every k of these steps is in the range */
 #pragma unroll
           for (int kb = 0; kb < KB; ++kb) {
-            const int ks = s * KB + kb;
-            if constexpr (0 != B4) {
-              if (ks < KS) {
-                T av[TI], bv[TJ];
-#pragma unroll
-                for (int p = 0; p < TI2; ++p) {
-                  av[2 * p] = (a4x[p] ? qa[kb][p][1] : qa[kb][p][0]);
-                  av[2 * p + 1] = qa[kb][p][1];
-                }
-                if constexpr (0 != TI % 2) av[TI - 1] = fa[kb][0];
-#pragma unroll
-                for (int p = 0; p < TJ2; ++p) {
-                  bv[2 * p] = (b4x[p] ? qb[kb][p][1] : qb[kb][p][0]);
-                  bv[2 * p + 1] = qb[kb][p][1];
-                }
-                if constexpr (0 != TJ % 2) bv[TJ - 1] = fb[kb][0];
-#pragma unroll
-                for (int ti = 0; ti < TI; ++ti) {
-#pragma unroll
-                  for (int tj = 0; tj < TJ; ++tj) {
-                    prod4[ti][tj] = lxs::mfma4<T>::mma(av[ti], bv[tj], prod4[ti][tj]);
-                  }
-                }
-              }
-            }
-            else if (ks < KS) {
-#pragma unroll
-              for (int ti = 0; ti < TI; ++ti) {
-#pragma unroll
-                for (int tj = 0; tj < TJ; ++tj) {
-                  if constexpr (PAIR) {
-                    prod[ti][tj] = mfma<T>::mma(pa[kb][ti >> 1][ti & 1], pb[kb][tj >> 1][tj & 1], prod[ti][tj]);
-                  }
-                  else {
-                    prod[ti][tj] = mfma<T>::mma(fa[kb][ti], fb[kb][tj], prod[ti][tj]);
-                  }
-                }
-              }
-            }
-            /* refill the slot with the next unit while the matrix core works */
-            if (ns * KB + kb < KS) LXS_LOAD_KSTEP(kb, la, lb, ns * KB + kb);
+            mma_step(std::false_type(), kb, true);
+            load_step(kb, f + KW * (KB + kb)); /* refill the slot while the matrix core works */
+          }
+          nseg += KB;
+          if (SEG <= nseg) { /* fold the segment into the run total */
+            fold();
+            nseg = 0;
           }
         }
-        if (SEG_LEN == ++nent) { /* fold the segment into the run total */
-          fold();
-          nent = 0;
+#pragma unroll
+        for (int kb = 0; kb < KB; ++kb) {
+          if (kb < n) mma_step(std::true_type(), kb, f + KW * kb <= flast);
         }
-        a0 = na;
-        b0 = nb;
-        if (!in_run) {
-          e = nxt;
-          break;
-        }
-        cur = nx;
+        nseg += n;
       }
     }
     /* this wavefront's partial block (run total plus the open segment) in LDS, then the fixed-order sum and
@@ -700,12 +712,12 @@ __device__ __forceinline__ void ep_body(T* __restrict__ cdata, const T* __restri
 #define LXS_EP_PASS cdata, adata, bdata, stack, stack_size, bs, m_rt, n_rt, k_rt, kt_unused, atomic, ps, pz, tsplit
 
 template <typename T, int TI, int TJ, int EP, int KB, int MC, int NC, int KC>
-__global__ void __launch_bounds__(64 * EP, (TI * TJ <= 4 ? 4 : 1)) smm_mfma_ep(LXS_EP_ARGS) {
+__global__ void __launch_bounds__(64 * EP, (TI * TJ <= 4 ? (2 == EP && 6 == KB ? 3 : 4) : 1)) smm_mfma_ep(LXS_EP_ARGS) {
   ep_body<T, TI, TJ, EP, KB, MC, NC, KC, 0>(LXS_EP_PASS);
 }
 /* FP64 on 4x4 blocks: C blocks up to 8 TI x 8 TJ */
 template <typename T, int TI, int TJ, int EP, int KB, int MC, int NC, int KC>
-__global__ void __launch_bounds__(64 * EP, 4) smm_mfma_eb(LXS_EP_ARGS) {
+__global__ void __launch_bounds__(64 * EP, (6 == KB && 9 == TI * TJ ? 3 : 4)) smm_mfma_eb(LXS_EP_ARGS) {
   ep_body<T, TI, TJ, EP, KB, MC, NC, KC, 1>(LXS_EP_PASS);
 }
 /* FP64 on 4x4 blocks that split k: C blocks up to 4 TI x 4 TJ, KB k-steps of 16 per stage */
