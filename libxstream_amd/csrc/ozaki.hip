@@ -25,10 +25,11 @@
  *               bounded).
  *   oz_recombine   per element: S_L = exact int64 sum of the level's partials, cd = sum over
  *               L = cutoff .. 0 of 2^(-7(L+2)) S_L in FP64, C = fma(alpha, 2^(ea+eb) cd, beta C).
- *   dgemm_f64   128x128 tiles with v_mfma_f64_16x16x4f64 on FP64 operands (the comparator).
+ *   dgemm_f64   128x128 or 64x64 tiles with v_mfma_f64_16x16x4f64 on FP64 operands (the comparator).
  */
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+#include <type_traits>
 #include <string.h>
 #include <stdlib.h>
 #include <pthread.h>
@@ -200,8 +201,6 @@ __global__ void __launch_bounds__(256) oz_scale_c(T* __restrict__ c, int ldc, in
 }
 
 /* ---- int8 level GEMM ------------------------------------------------------------------------- */
-
-constexpr int GT = 128;        /* output tile of the FP64 comparator */
 
 /*
  * One work item of the int8 GEMM, in units of 64 k:
@@ -842,79 +841,206 @@ __global__ void __launch_bounds__(256) oz_crt_recombine(const uint8_t* __restric
 /* ---- native FP64 GEMM (comparator) ----------------------------------------------------------- */
 
 constexpr int DK = 16; /* k per LDS stage */
+constexpr long DGEMM_LD_MAX = 1L << 21; /* 128 rows of ld elements stay within 32-bit byte offsets */
 
-/* v_mfma_f64_16x16x4f64: A lane l -> A[l%16][l/16], B lane l -> B[l/16][l%16], D lane l reg r -> (l/16 + 4r, l%16) */
-__global__ void __launch_bounds__(256) dgemm_f64(const double* __restrict__ a, long ars, long aks,
-  const double* __restrict__ b, long bks, long bcs, int M, int N, int K, double alpha, double beta,
-  double* __restrict__ c, int ldc) {
-  __shared__ double la[2][DK][GT], lb[2][DK][GT]; /* [buffer][k][row / column] */
-  const int tid = threadIdx.x, lane = tid & 63;
+/*
+ * v_mfma_f64_16x16x4f64: first operand lane l -> row l%16, k l/16; second l -> column l%16, k l/16; result lane l
+ * register r -> (l/16 + 4r, l%16). The first operand is op(B), so a lane's results are one row of C in four
+ * columns and 16 lanes store 16 consecutive rows.
+ * A work-group computes a DT x DT tile of C (DT = 32 WT) with KG groups of 4 wavefronts; each wavefront holds WT x WT
+ * tiles of 16 x 16. Group g takes the k-stages g, g + KG, ... of DK, its operands double-buffered in its own LDS; the
+ * groups' sums are added in order at the end. Operand stages go through registers (16-byte loads of two elements along
+ * the contiguous dimension, issued one stage ahead): AK / BK tell that k is contiguous in A / B. LDS holds
+ * [k][row] with 8 elements of padding, or [row][k] with 2 (k contiguous): stores of both are 16 bytes, fragment
+ * reads (k = 2 (l/16) and the one after it, for two instructions) hit every bank pair once per half-wavefront.
+ * Stages that are not full, and matrices of one row or column, go through LDS element by element.
+ * Bound: the matrix cores (64 cycles per instruction, 64 or 16 of them per stage and wavefront; two wavefronts per
+ * SIMD cover each other's waits). 4096^3: NN 3884 -> 2046 us, TN 4565 -> 1961, NT 3614 -> 2056, TT 3900 -> 2030 (67 to
+ * 70 TFLOP/s of 78.6; before: one wavefront per SIMD that stopped for LDS stores with 16-way bank conflicts and for
+ * loads under branches). The issue order is fixed by sched_group_barrier: left to itself the compiler read the second
+ * half's fragments late in some layouts (NN 2526 us).
+ */
+template <int WT, int KG, bool AK, bool BK>
+__global__ void __launch_bounds__(256 * KG, (1 == KG ? 2 : 1)) dgemm_f64(const double* __restrict__ a, long lda,
+  const double* __restrict__ b, long ldb, int M, int N, int K, int tiles_m, int tiles_n, double alpha, double beta,
+  double* __restrict__ c, long ldc) {
+  constexpr int DT = 32 * WT, RS = DT + 8, KS = DK + 2; /* rows of a tile; LDS strides of the two layouts */
+  constexpr int NX = DT * DK / 512;                     /* pairs per thread, operand and stage */
+  constexpr int SA = (AK ? DT * KS : DK * RS), SB = (BK ? DT * KS : DK * RS);
+  extern __shared__ __attribute__((aligned(16))) double dgemm_lds[];
+  typedef double v2_t __attribute__((ext_vector_type(2)));
+  typedef double v2u_t __attribute__((ext_vector_type(2), aligned(8)));
+  const int tid = threadIdx.x & 255, lane = tid & 63;
+  const int grp = (1 == KG ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 8));
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wr = wave >> 1, wc = wave & 1;
-  const int row0 = blockIdx.x * GT, col0 = blockIdx.y * GT;
-  const int nkb = (K + DK - 1) / DK;
-  d4_t acc[4][4];
-#pragma unroll
-  for (int x = 0; x < 4; ++x) {
-#pragma unroll
-    for (int y = 0; y < 4; ++y) acc[x][y] = d4_t{0, 0, 0, 0};
+  const int wr = wave >> 1, wc = wave & 1, li = lane & 15, lk = lane >> 4;
+  double* const lds = dgemm_lds + grp * 2 * (SA + SB);
+  /* work-groups go to the 8 XCDs in turn: each XCD takes one contiguous part of the tiles, in bands of 8 tile rows, so
+     that the operands of its resident work-groups meet in its L2 */
+  int t = blockIdx.x;
+  {
+    const int total = tiles_m * tiles_n, per = total / 8;
+    if (t < 8 * per) t = (t & 7) * per + (t >> 3);
   }
-  /* staging: 128 x 16 elements per operand, 8 per thread; element e = tid + 256 x */
-  double ra[8], rb[8];
-  auto fetch = [&](int kb) {
-    const int k0 = kb * DK;
+  const int band = t / (8 * tiles_n), rows = min(8, tiles_m - 8 * band), tb = t - 8 * tiles_n * band;
+  const int row0 = (8 * band + tb % rows) * DT, col0 = (tb / rows) * DT;
+  const int nst = (K + DK - 1) / DK;
+  typedef std::integral_constant<bool, AK> ak_t;
+  typedef std::integral_constant<bool, BK> bk_t;
+  /* operand element (row r of op(A) / column of op(B), k): p[r + k ld] or p[r ld + k]. A full stage is loaded from a
+     uniform address plus 32-bit byte offsets that do not change from stage to stage; rows past the matrix load its
+     last ones, they feed results that are not stored */
+  const bool fulla = (2 <= M && lda <= DGEMM_LD_MAX), fullb = (2 <= N && ldb <= DGEMM_LD_MAX);
+  unsigned int offa[NX], offb[NX];
 #pragma unroll
-    for (int x = 0; x < 8; ++x) {
-      const int e = tid + 256 * x;
-      const int r = (1 == ars ? (e & 127) : (e >> 4)), k = (1 == ars ? (e >> 7) : (e & 15));
-      const int gi = row0 + r, gk = k0 + k;
-      ra[x] = (gi < M && gk < K) ? a[(long)gi * ars + (long)gk * aks] : 0.0;
-      const int cc = (1 == bcs ? (e & 127) : (e >> 4)), kc = (1 == bcs ? (e >> 7) : (e & 15));
-      const int gj = col0 + cc, gk2 = k0 + kc;
-      rb[x] = (gj < N && gk2 < K) ? b[(long)gk2 * bks + (long)gj * bcs] : 0.0;
-    }
+  for (int x = 0; x < NX; ++x) {
+    const int e = tid + 256 * x;
+    const int ka = (AK ? 2 * (e & 7) : e / (DT / 2)), ra = row0 + (AK ? e >> 3 : 2 * (e % (DT / 2)));
+    const int kb = (BK ? 2 * (e & 7) : e / (DT / 2)), rb = col0 + (BK ? e >> 3 : 2 * (e % (DT / 2)));
+    offa[x] = 8u * (AK ? (unsigned int)(min(ra, M - 1) - row0) * (unsigned int)lda + ka
+                       : (unsigned int)(min(ra, M - 2) - min(row0, M - 2)) + ka * (unsigned int)lda);
+    offb[x] = 8u * (BK ? (unsigned int)(min(rb, N - 1) - col0) * (unsigned int)ldb + kb
+                       : (unsigned int)(min(rb, N - 2) - min(col0, N - 2)) + kb * (unsigned int)ldb);
+  }
+  const auto fetch = [&](v2_t* v, const double* __restrict__ p, long ld, int r0, int R, int st, const unsigned int* off,
+                       auto kc) {
+    constexpr bool KC = decltype(kc)::value;
+    const char* const base = (const char*)(p + (KC ? (long)r0 * ld + st * DK : min(r0, R - 2) + (long)st * DK * ld));
+#pragma unroll
+    for (int x = 0; x < NX; ++x) v[x] = *(const __attribute__((address_space(1))) v2u_t*)(base + off[x]);
   };
-  auto store = [&](int buf) {
+  const auto store = [&](double* dst, v2_t* v, int r0, int R, auto kc) {
+    constexpr bool KC = decltype(kc)::value;
 #pragma unroll
-    for (int x = 0; x < 8; ++x) {
+    for (int x = 0; x < NX; ++x) {
       const int e = tid + 256 * x;
-      if (1 == ars) la[buf][e >> 7][e & 127] = ra[x];
-      else la[buf][e & 15][e >> 4] = ra[x];
-      if (1 == bcs) lb[buf][e >> 7][e & 127] = rb[x];
-      else lb[buf][e & 15][e >> 4] = rb[x];
-    }
-  };
-  fetch(0);
-  store(0);
-  __syncthreads();
-  for (int kb = 0; kb < nkb; ++kb) {
-    const int buf = kb & 1;
-    if (kb + 1 < nkb) fetch(kb + 1);
-#pragma unroll
-    for (int ks = 0; ks < DK; ks += 4) {
-      double fa[4], fb[4];
-#pragma unroll
-      for (int x = 0; x < 4; ++x) {
-        fa[x] = la[buf][ks + (lane >> 4)][64 * wr + 16 * x + (lane & 15)];
-        fb[x] = lb[buf][ks + (lane >> 4)][64 * wc + 16 * x + (lane & 15)];
+      if (KC) {
+        *(v2_t*)(dst + (e >> 3) * KS + 2 * (e & 7)) = v[x];
       }
-#pragma unroll
-      for (int x = 0; x < 4; ++x) {
-#pragma unroll
-        for (int y = 0; y < 4; ++y) acc[x][y] = __builtin_amdgcn_mfma_f64_16x16x4f64(fa[x], fb[y], acc[x][y], 0, 0, 0);
+      else {
+        const int rl = 2 * (e % (DT / 2));
+        /* a pair that would start at the last row was loaded one row early */
+        v[x][0] = (r0 + rl == R - 1 ? v[x][1] : v[x][0]);
+        *(v2_t*)(dst + (e / (DT / 2)) * RS + rl) = v[x];
       }
     }
-    if (kb + 1 < nkb) store(buf ^ 1);
+  };
+  /* a stage that is not full, or any stage of a matrix of one row or column: element by element, zero outside */
+  const auto edge = [&](double* dst, const double* __restrict__ p, long ld, int r0, int R, int st, auto kc) {
+    constexpr bool KC = decltype(kc)::value;
+    for (int e = tid; e < DT * DK; e += 256) {
+      const int rl = (KC ? e / DK : e % DT), kl = (KC ? e % DK : e / DT), r = r0 + rl, k = st * DK + kl;
+      dst[KC ? rl * KS + kl : kl * RS + rl] = (r < R && k < K) ? p[KC ? (long)r * ld + k : r + (long)k * ld] : 0.0;
+    }
+  };
+  d4_t acc[WT][WT];
+#pragma unroll
+  for (int x = 0; x < WT; ++x) {
+#pragma unroll
+    for (int y = 0; y < WT; ++y) acc[x][y] = d4_t{0, 0, 0, 0};
+  }
+  const auto multiply = [&](const double* la, const double* lb) {
+#pragma unroll
+    for (int k8 = 0; k8 < DK; k8 += 8) {
+      v2_t fa[WT], fb[WT];
+#pragma unroll
+      for (int x = 0; x < WT; ++x) {
+        const int i = 16 * (WT * wr + x) + li, j = 16 * (WT * wc + x) + li, k = k8 + 2 * lk;
+        if (AK) fa[x] = *(const v2_t*)(la + i * KS + k);
+        else fa[x] = v2_t{la[k * RS + i], la[(k + 1) * RS + i]};
+        if (BK) fb[x] = *(const v2_t*)(lb + j * KS + k);
+        else fb[x] = v2_t{lb[k * RS + j], lb[(k + 1) * RS + j]};
+      }
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+#pragma unroll
+        for (int x = 0; x < WT; ++x) {
+#pragma unroll
+          for (int y = 0; y < WT; ++y) {
+            acc[x][y] = __builtin_amdgcn_mfma_f64_16x16x4f64(fb[y][h], fa[x][h], acc[x][y], 0, 0, 0);
+          }
+        }
+      }
+    }
+  };
+  /* the full stages without a branch around a load, so that the compiler waits for them only where they are stored;
+     a group past its last stage loads that one again */
+  const int nfull = (fulla && fullb ? K / DK : 0);
+  double *la = lds, *ln = lds + SA + SB;
+  if (0 < nfull) {
+    v2_t ra[NX], rb[NX];
+    fetch(ra, a, lda, row0, M, min(grp, nfull - 1), offa, ak_t());
+    fetch(rb, b, ldb, col0, N, min(grp, nfull - 1), offb, bk_t());
+    store(la, ra, row0, M, ak_t());
+    store(la + SA, rb, col0, N, bk_t());
+    __syncthreads();
+    for (int s0 = 0; s0 < nfull; s0 += KG) { /* the same trip count for every group */
+      const int next = min(s0 + grp + KG, nfull - 1);
+      fetch(ra, a, lda, row0, M, next, offa, ak_t());
+      fetch(rb, b, ldb, col0, N, next, offb, bk_t());
+      if (1 == KG || s0 + grp < nfull) multiply(la, la + SA);
+      store(ln, ra, row0, M, ak_t());
+      store(ln + SA, rb, col0, N, bk_t());
+      if constexpr (1 == KG) { /* issue order: the first half's fragments, its products with the next stage's loads
+                                  and the second half's fragments between them, then the second half's products */
+        __builtin_amdgcn_sched_group_barrier(0x100, 2 * WT, 0); /* DS read */
+#pragma unroll
+        for (int i = 0; i < 2 * WT; ++i) {
+          __builtin_amdgcn_sched_group_barrier(0x008, WT / 2, 0); /* MFMA */
+          __builtin_amdgcn_sched_group_barrier(0x020, NX / WT, 0); /* VMEM read */
+        }
+#pragma unroll
+        for (int i = 0; i < 2 * WT; ++i) {
+          __builtin_amdgcn_sched_group_barrier(0x008, WT / 2, 0);
+          __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+        }
+        __builtin_amdgcn_sched_group_barrier(0x008, 2 * WT * WT, 0);
+        __builtin_amdgcn_sched_group_barrier(0x200, 2 * NX, 0); /* DS write */
+      }
+      __syncthreads();
+      double* const x = la;
+      la = ln;
+      ln = x;
+    }
+  }
+  for (int s0 = nfull; s0 < nst; s0 += KG) {
+    const int st = s0 + grp;
+    if (st < nst) {
+      edge(la, a, lda, row0, M, st, ak_t());
+      edge(la + SA, b, ldb, col0, N, st, bk_t());
+    }
+    __syncthreads();
+    if (st < nst) multiply(la, la + SA);
     __syncthreads();
   }
+  if (1 < KG) { /* the groups' sums in order: group 0 adds those of 1, 2, ... from LDS */
+    static_assert(1 == KG || (KG - 1) * WT * WT * 4 * 256 <= KG * 2 * (SA + SB), "partial tiles fit the stages' LDS");
+    double* const part = dgemm_lds + tid;
+    if (0 != grp) {
 #pragma unroll
-  for (int x = 0; x < 4; ++x) {
+      for (int x = 0; x < WT * WT; ++x) {
 #pragma unroll
-    for (int y = 0; y < 4; ++y) {
-      const int j = col0 + 64 * wc + 16 * y + (lane & 15);
+        for (int r = 0; r < 4; ++r) part[(((grp - 1) * WT * WT + x) * 4 + r) * 256] = acc[x / WT][x % WT][r];
+      }
+    }
+    __syncthreads();
+    if (0 != grp) return;
+    for (int g = 0; g < KG - 1; ++g) {
+#pragma unroll
+      for (int x = 0; x < WT * WT; ++x) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) acc[x / WT][x % WT][r] += part[((g * WT * WT + x) * 4 + r) * 256];
+      }
+    }
+  }
+#pragma unroll
+  for (int x = 0; x < WT; ++x) {
+    const int i = row0 + 16 * (WT * wr + x) + li;
+#pragma unroll
+    for (int y = 0; y < WT; ++y) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const int i = row0 + 64 * wr + 16 * x + (lane >> 4) + 4 * r;
+        const int j = col0 + 16 * (WT * wc + y) + lk + 4 * r;
         if (i < M && j < N) {
           double* const pc = c + i + (long)j * ldc;
           *pc = (0 != beta ? fma(alpha, acc[x][y][r], beta * *pc) : alpha * acc[x][y][r]);
@@ -922,6 +1048,28 @@ __global__ void __launch_bounds__(256) dgemm_f64(const double* __restrict__ a, l
       }
     }
   }
+}
+
+template <int WT, int KG, bool AK, bool BK>
+int dgemm_launch(const double* a, long lda, const double* b, long ldb, int M, int N, int K, double alpha, double beta,
+  double* c, int ldc, hipStream_t st) {
+  constexpr int DT = 32 * WT;
+  constexpr size_t lds = sizeof(double) * KG * 2 * ((AK ? DT * (DK + 2) : DK * (DT + 8)) + (BK ? DT * (DK + 2) : DK * (DT + 8)));
+  const int tm = (M + DT - 1) / DT, tn = (N + DT - 1) / DT;
+  if ((double)tm * tn > 2147483647.0) return LXS_ELIMIT;
+  dgemm_f64<WT, KG, AK, BK><<<(unsigned int)(tm * tn), 256 * KG, lds, st>>>(a, lda, b, ldb, M, N, K, tm, tn, alpha, beta,
+    c, (long)ldc);
+  return (int)hipGetLastError();
+}
+template <int WT, int KG>
+int dgemm_launch(bool ak, bool bk, const double* a, long lda, const double* b, long ldb, int M, int N, int K, double alpha,
+  double beta, double* c, int ldc, hipStream_t st) {
+  if (ak) {
+    return bk ? dgemm_launch<WT, KG, true, true>(a, lda, b, ldb, M, N, K, alpha, beta, c, ldc, st)
+              : dgemm_launch<WT, KG, true, false>(a, lda, b, ldb, M, N, K, alpha, beta, c, ldc, st);
+  }
+  return bk ? dgemm_launch<WT, KG, false, true>(a, lda, b, ldb, M, N, K, alpha, beta, c, ldc, st)
+            : dgemm_launch<WT, KG, false, false>(a, lda, b, ldb, M, N, K, alpha, beta, c, ldc, st);
 }
 
 /* ---- complex 3M helpers ---------------------------------------------------------------------- */
@@ -1160,12 +1308,20 @@ extern "C" int lxs_oz_scale(int dtype, void* c, int ldc, int M, int N, double be
 /* native FP64: C = alpha op(A) op(B) + beta C; op(A)(i, k) at a[i * ars + k * aks], op(B)(k, j) at b[k * bks + j * bcs] */
 extern "C" int lxs_dgemm(const double* a, long ars, long aks, const double* b, long bks, long bcs, int M, int N, int K,
   double alpha, double beta, double* c, int ldc, void* hip_stream) {
+  const bool ak = (1 != ars), bk = (1 != bcs); /* k contiguous */
+  const long lda = (ak ? ars : aks), ldb = (bk ? bcs : bks);
+  const long t128 = (long)((M + 127) / 128) * ((N + 127) / 128), t64 = (long)((M + 63) / 64) * ((N + 63) / 64);
+  const hipStream_t st = (hipStream_t)hip_stream;
   if (!((1 == ars) || (1 == aks)) || !((1 == bks) || (1 == bcs))) return LXS_ELIMIT;
   if (0 >= M || 0 >= N) return 0;
   if (0 >= K) return lxs_oz_scale(3, c, ldc, M, N, beta, hip_stream);
-  dgemm_f64<<<dim3((unsigned int)((M + GT - 1) / GT), (unsigned int)((N + GT - 1) / GT)), 256, 0,
-    (hipStream_t)hip_stream>>>(a, ars, aks, b, bks, bcs, M, N, K, alpha, beta, c, ldc);
-  return (int)hipGetLastError();
+  /* 128 x 128 tiles need the fewest operand bytes, but two work-groups per CU to keep the matrix cores fed: 2048^3 (256
+     such tiles) ran 285 us on 64 x 64 tiles; 1500^3 (144) 146 us. Few 64 x 64 tiles leave CUs idle, so four groups of
+     wavefronts share a tile's k: 159x433x3000 (21 tiles) 114 us, 300^3 (25) 18 us, 64x64x4096 (1) 156 us; at 81 to 288
+     tiles one group is as fast (700^3, 121 tiles: 35.1 us against 34.6 on two, 1000x1100x900: 63.8 against 77 on four) */
+  if (384 <= t128) return dgemm_launch<4, 1>(ak, bk, a, lda, b, ldb, M, N, K, alpha, beta, c, ldc, st);
+  if (100 <= t64) return dgemm_launch<2, 1>(ak, bk, a, lda, b, ldb, M, N, K, alpha, beta, c, ldc, st);
+  return dgemm_launch<2, 4>(ak, bk, a, lda, b, ldb, M, N, K, alpha, beta, c, ldc, st);
 }
 
 extern "C" int lxs_oz_csplit(int dtype, const void* z, int ld, int rows, int cols, int conj, void* re, void* im,
