@@ -6,8 +6,9 @@
  * 4 / 9; Scheme 1 cutoff 2(nslices-1) - oztrim; Scheme 2 drops 2 oztrim mantissa bits) and the
  * adaptive choice as in samples/ozaki/ozaki_gemm.c:520-587 (Scheme 1 while its pair count is below
  * the prime count plus the reconstruction's share). The device work is ozaki.hip: per-operand
- * preprocessing into int8 planes (digits or residues), one int8 GEMM launch per K pass, then the FP64
- * recombination (Scheme 1) or the CRT reconstruction (Scheme 2).
+ * preprocessing into int8 planes (digits or residues), then per K pass one kernel for all pairs and the recombination
+ * (Scheme 1 over the triangle or all pairs, ozaki_pairs.hip), or one int8 GEMM launch followed by the FP64 recombination
+ * (other trims, or K too long for int32 level sums) or the CRT reconstruction (Scheme 2).
  */
 #include "lxs_internal.h"
 #include "../../include/ozaki.h"
@@ -452,7 +453,8 @@ static int oz_gemm_real(ozaki_context_t* ctx, hipStream_t hs, int ta, int tb, in
       const int Kp = (int)oz_up((size_t)kk, OZ_TILE_K);
       /* the last pass may need fewer primes */
       const int np = (0 != l.crt ? oz_crt_primes(l.np, mb - trim, kk) : 0);
-      const int nitems = oz_plan(ctx, l.crt, np, Kp / OZ_UNIT_K, tiles, impl->items, zb);
+      const int pairs = (0 == l.crt && 0 != lxs_oz_pairs_fits(s, cutoff, Kp));
+      const int nitems = (0 == pairs ? oz_plan(ctx, l.crt, np, Kp / OZ_UNIT_K, tiles, impl->items, zb) : 0);
       const double nprod = (0 != l.crt ? np : ozaki_count_pairs(s, cutoff, 0));
       const int nplanes = (0 != l.crt ? np : s);
       void* token = (NULL == fixed ? lxs_profile_begin(hs) : NULL);
@@ -473,6 +475,15 @@ static int oz_gemm_real(ozaki_context_t* ctx, hipStream_t hs, int ta, int tb, in
         }
       }
       lxs_profile_end(token, hs, "ozaki_pre", 0.0, (double)ts * ((double)M + N) * kk + (double)nplanes * (l.Mp + l.Np) * Kp);
+      if (0 == result && 0 != pairs) { /* every pair, level and the recombination in one kernel */
+        token = (NULL == fixed ? lxs_profile_begin(hs) : NULL);
+        result = lxs_oz_pairs(dtype, (const signed char*)(base + l.planes_a), (const signed char*)(base + l.planes_b), occ,
+          occ + 8, s, cutoff, l.Mp, l.Np, Kp, (const int*)(base + l.ea), (const int*)(base + l.eb), M, N, alpha,
+          (0 == k0 ? beta : 1.0), dc, ldc, lxs_oz_pairs_split(s, cutoff, M, N, Kp, l.nitems), (int*)(base + l.out), hs);
+        lxs_profile_end(token, hs, "ozaki_i8", 2.0 * nprod * l.Mp * l.Np * Kp,
+          (double)nplanes * (l.Mp + l.Np) * Kp + (double)ts * M * N * (0 == k0 && 0 == beta ? 1 : 2));
+        continue;
+      }
       if (0 == result) { /* int8 work of every pair up to the cutoff (pairs of all-zero planes are skipped), or every prime */
         token = (NULL == fixed ? lxs_profile_begin(hs) : NULL);
         result = lxs_oz_level_gemm(l.crt, (const signed char*)(base + l.planes_a), (const signed char*)(base + l.planes_b),
