@@ -91,7 +91,7 @@ int lxs_oz_level_gemm(int crt, const signed char* pa, const signed char* pb, con
 /* FP64 recombination of the partials: zb[L] = first item of level L (cutoff + 2 entries) */
 int lxs_oz_recombine(int dtype, const int* c32, const int* zb, int cutoff, int Mp, int Np, const int* ea,
   const int* eb, int M, int N, double alpha, double beta, void* c, int ldc, void* hip_stream);
-/* Scheme 1 in one kernel, without partials (ozaki_pairs.hip): cutoff s - 1 (triangle) or 2 (s - 1) (all pairs) and K
+/* Scheme 1 in one kernel, without partials (ozaki_pairs.h): cutoff s - 1 (triangle) or 2 (s - 1) (all pairs) and K
    short enough for exact int32 level sums (lxs_oz_pairs_fits); the same result as level GEMM and recombination */
 int lxs_oz_pairs_fits(int s, int cutoff, int Kp);
 /* work-groups that share a tile's k (1: none), with room for nitems partial planes of Mp x Np ints at part */

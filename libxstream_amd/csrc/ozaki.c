@@ -7,7 +7,7 @@
  * adaptive choice as in samples/ozaki/ozaki_gemm.c:520-587 (Scheme 1 while its pair count is below
  * the prime count plus the reconstruction's share). The device work is ozaki.hip: per-operand
  * preprocessing into int8 planes (digits or residues), then per K pass one kernel for all pairs and the recombination
- * (Scheme 1 over the triangle or all pairs, ozaki_pairs.hip), or one int8 GEMM launch followed by the FP64 recombination
+ * (Scheme 1 over the triangle or all pairs, ozaki_pairs.h), or one int8 GEMM launch followed by the FP64 recombination
  * (other trims, or K too long for int32 level sums) or the CRT reconstruction (Scheme 2).
  */
 #include "lxs_internal.h"

@@ -25,7 +25,7 @@
  *               bounded).
  *   oz_recombine   per element: S_L = exact int64 sum of the level's partials, cd = sum over
  *               L = cutoff .. 0 of 2^(-7(L+2)) S_L in FP64, C = fma(alpha, 2^(ea+eb) cd, beta C).
- *               (Scheme 1 over the triangle or all pairs goes to ozaki_pairs.hip instead of these two, unless K
+ *               (Scheme 1 over the triangle or all pairs goes to ozaki_pairs.h instead of these two, unless K
  *               is too long for int32 level sums.)
  *   dgemm_f64   128x128 or 64x64 tiles with v_mfma_f64_16x16x4f64 on FP64 operands (the comparator).
  */
@@ -36,6 +36,7 @@
 #include <stdlib.h>
 #include <pthread.h>
 #include "lxs_kernels.h"
+#include "ozaki_pairs.h"
 
 namespace {
 

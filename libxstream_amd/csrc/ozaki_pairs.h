@@ -5,6 +5,9 @@
  * oz_recombine: S_L exact in int32, cd = sum over L = cutoff .. 0 of 2^(-7(L+2)) S_L in FP64,
  * C = fma(alpha, 2^(ea + eb) cd, beta C).
  */
+#ifndef LXS_OZAKI_PAIRS_H
+#define LXS_OZAKI_PAIRS_H
+
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 #include "lxs_kernels.h"
@@ -306,3 +309,5 @@ extern "C" int lxs_oz_pairs(int dtype, const signed char* pa, const signed char*
   }
   return result;
 }
+
+#endif /* LXS_OZAKI_PAIRS_H */

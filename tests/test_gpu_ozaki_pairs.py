@@ -1,4 +1,4 @@
-"""Scheme I with all levels of an output tile in registers (ozaki_pairs.hip): every slice count over the triangle and over
+"""Scheme I with all levels of an output tile in registers (ozaki_pairs.h): every slice count over the triangle and over
 all pairs, tile edges, work-groups that share a tile's k, planes without a nonzero digit, and a K whose level sums
 would not fit int32 (the level GEMM's partials again). Bar: bit for bit the oracle."""
 import numpy as np
