@@ -63,7 +63,9 @@ typedef enum libsmm_acc_config_source_t {
   libsmm_acc_config_learned = 3  /* learned predictor */
 } libsmm_acc_config_source_t;
 
-/** configuration libsmm_acc_process would use for this shape; *source may be NULL */
+/** configuration libsmm_acc_process would use for this shape; *source may be NULL. For a shape whose source is the
+ *  shipped predictor and whose C block has up to 16 tiles of 16x16, process chooses by the stack's size as well, and
+ *  stacks shorter than the one a configuration was measured on get fewer entries per work-group */
 LIBXSTREAM_API int libsmm_acc_config_get(libsmm_acc_data_t datatype, int m, int n, int k, libsmm_acc_smm_config_t* config,
   int* source);
 /** the built-in heuristic's configuration for this shape (ignores the registry and the predictor) */

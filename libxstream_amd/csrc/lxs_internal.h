@@ -29,6 +29,7 @@ typedef struct lxs_config_t {
   int verbosity;
   int profile;   /* LIBXSTREAM_PROFILE: launch records (|value| + 1 histogram buckets; < 0 also prints each) */
   int profile_mem; /* LIBXSTREAM_PROFILE_MEM: copy and fill records (H2D, D2H, D2D, ZERO) */
+#define LXS_SMM_SPLIT_DEFAULT 2
   int split;     /* LIBXSTREAM_SMM_SPLIT: C-runs are cut past max(split*bs, split_min) entries (0: never) */
   int split_min; /* LIBXSTREAM_SMM_SPLIT_MIN: runs of up to this many entries are never cut (0: 64 in stacks of
                     at least LXS_SMM_SPLIT_FILL entries, none in shorter ones) */
@@ -59,6 +60,8 @@ void lxs_profile_finalize(void);
 
 /** learned predictor slot (mlp.c): EXIT_SUCCESS and a configuration when a confident model is installed */
 int lxs_learned_predict(int datatype, int m, int n, int k, libsmm_acc_smm_config_t* config);
+/** 1 when the installed model is the caller's (libsmm_acc_learned_set) and not the shipped one */
+int lxs_learned_is_user(void);
 void lxs_learned_finalize(void);
 /** load a model file and install it as the predictor, owned by the library until finalize */
 void lxs_learned_load_default(const char* path);

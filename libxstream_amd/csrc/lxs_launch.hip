@@ -91,7 +91,7 @@ static int mfma_variant(const mfma_entry_t* e) { return (0 != e->b4 ? 2 + e->b4 
 /* LDS bytes of an MFMA kernel: the partial blocks of the ep wavefronts (16 x 16 tiles, or one register per
    4x4-block instruction and lane) */
 static size_t mfma_lds(const mfma_entry_t* e, int dtype) {
-  return (1 < e->ep ? (size_t)e->ep * e->ti * e->tj * (2 == e->b4 ? 16 : (1 == e->b4 ? 64 : 256)) * (3 == dtype ? 8 : 4) : 0);
+  return (1 < e->ep || 0 != e->b4 ? (size_t)e->ep * e->ti * e->tj * (2 == e->b4 ? 16 : (1 == e->b4 ? 64 : 256)) * (3 == dtype ? 8 : 4) : 0);
 }
 /* a runtime-shape kernel covers (m, n): 16x16 tiles up to 16 ti x 16 tj, with at least two rows and columns
    where the kernel loads element pairs (an even number of tiles in both dimensions); 4x4 blocks with exactly

@@ -682,6 +682,15 @@ int lxs_learned_predict(int datatype, int m, int n, int k, libsmm_acc_smm_config
   return result;
 }
 
+/* a model that the caller installed (libsmm_acc_learned_set), not the shipped one or none */
+int lxs_learned_is_user(void) {
+  int result;
+  pthread_mutex_lock(&lxs_learned_lock);
+  result = (NULL != lxs_learned && lxs_learned_owned != lxs_learned);
+  pthread_mutex_unlock(&lxs_learned_lock);
+  return result;
+}
+
 void lxs_learned_load_default(const char* path) {
   libsmm_acc_mlp_t* model = NULL;
   if (EXIT_SUCCESS == libsmm_acc_mlp_load(&model, path)) {

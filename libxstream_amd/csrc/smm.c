@@ -724,6 +724,99 @@ int lxs_smm_tsplit(int bs, int split, int stack_size) {
   return (0 < lxs_cfg.split ? (floor < t ? t : floor) : 0);
 }
 
+/*
+ * Stack entries per work-group and cut factor of an entry-parallel kernel on a stack too short to fill the device
+ * with whole runs (fewer than LXS_SMM_SPLIT_FILL entries). Cutting a run into pieces shortens its chain of k-steps
+ * but adds an atomic update of C per piece, so it pays by x = 1000 k (padded / useful area of C) / (wavefronts x
+ * entries); over 19 shapes x 9 sizes from 300 to 7000 entries in runs of about 30, the geometric mean of the time
+ * against the best of ten choices, FP64 on 16x16 tiles: x < 2.2 whole 0.98-1.00 (pieces of 8: 0.68-0.86), 3.5-8 pieces
+ * of 8 0.93 (whole 0.83-0.75), 8-50 pieces of 4 0.95-0.99 (whole 0.60-0.45), above 1 to 2 entries. The lines lie lower on
+ * 4x4 blocks and higher in FP32, whose products take half the time and whose atomics do not (whole 0.93 at x = 6.7-10).
+ * Whole runs: a work-group takes the runs that begin among its entries, so fewer entries than a run has leave it one
+ * run (32: 0.53-0.68 of the best at 3000 to 10000 entries), and stacks of short runs want few (FP64 23x23x23, 10000 entries
+ * in runs of 1: 123 us with 24, 113 with 11). The kernels of large blocks have room for 512 work-groups only, and those
+ * without a run of their own take the places of others: 24 (FP64 64x64x64, 12000 entries: 24 158 us, 16 227).
+ */
+static void lxs_smm_pieces(int datatype, int m, int n, int k, int stack_size, const libsmm_acc_smm_config_t* config, int* bs,
+  int* split) {
+  const int tile = (2 == config->variant ? 16 : (3 == config->variant ? 8 : 4)), ep = config->nt / 64;
+  const double area = (double)(config->tm * tile) * (config->tn * tile) / ((double)m * n);
+  const double x = 1000.0 * k * area / ((double)ep * stack_size);
+  const int f64 = (dbcsr_type_real_8 == datatype);
+  double lim[3]; /* whole runs up to lim[0], pieces of 8 up to lim[1], of 4 up to lim[2], then of 1 to 2 */
+  if (4 == config->variant) lim[0] = lim[1] = (f64 ? 7.0 : 17.0), lim[2] = (f64 ? 20.0 : 17.0);
+  else if (3 == config->variant) lim[0] = 1.5, lim[1] = 5.0, lim[2] = 30.0;
+  else if (0 != f64) lim[0] = 3.0, lim[1] = 8.0, lim[2] = 50.0;
+  else lim[0] = 9.0, lim[1] = 25.0, lim[2] = 150.0;
+  if (x < lim[0]) {
+    *bs = (8000 <= stack_size ? (2 < ep ? 16 : 24) : (2000 <= stack_size ? stack_size / 500 : 4));
+    *split = 48 / *bs;
+  }
+  else if (x < lim[1]) *bs = 8, *split = 1;
+  else if (x < lim[2]) *bs = 4, *split = 1;
+  else *bs = 1, *split = 2;
+}
+
+/*
+ * Configuration for a shape without a tuned row and C blocks of up to 16 tiles of 16x16, by shape and stack size.
+ * The shipped predictor knows stacks of 30000 entries and no kernel of 64 k per stage. Trained on the kernels that took
+ * whole entries per wavefront, its choices (at 24 entries per work-group) reached 0.94-0.98 of the best kernel over 32
+ * shapes of m or n above 16 at 30000 and 200000 entries, this rule 0.99 (in both types); at 3000 entries 0.59 (FP32) and 0.73 (FP64).
+ * Blocks up to 16x16: 4x4 blocks splitting k while the fold of their blocks is cheap against the k-steps (FP64 below
+ * 12 blocks; FP32, whose fold costs four times as much, up to 4 blocks or 4 per 16-k step of a run of 30), with as
+ * many wavefronts per run as leave each about 8 steps (1 up to k = 6, 2 up to k = 18, else 4); over 17 such shapes
+ * from 2000 to 500000 entries 0.95-0.99 of the best, where predicted and tuned rows reached 0.67-0.87. Up to 1000 entries
+ * only the chain of one work-group counts, and the fold of more than 4 blocks is longer than the k-steps that it saves
+ * (11x11x33, 300 entries: FP64 6.7 us with 9 blocks, 5.5 with one tile; FP32 11.0 and 6.1). Everything else: 16x16 tiles,
+ * 4 wavefronts per run (2 above 8 tiles, all there are for short stacks).
+ */
+static int lxs_smm_rule(int datatype, int m, int n, int k, int stack_size, libsmm_acc_smm_config_t* config) {
+  const int ti = (m + 15) / 16, tj = (n + 15) / 16, f64 = (dbcsr_type_real_8 == datatype);
+  const int blocks = ((m + 3) / 4) * ((n + 3) / 4), shortened = (LXS_SMM_SPLIT_FILL > stack_size);
+  const double steps = 30.0 * k / 16.0; /* 16-k steps of a run of 30 entries */
+  const int latency = (1000 >= stack_size); /* nothing but the length of one work-group's chain counts */
+  if (16 < ti * tj) return EXIT_FAILURE;
+  memset(config, 0, sizeof(*config));
+  config->flush = 2;
+  if (16 >= m && 16 >= n && (4 >= blocks || (0 == latency && (0 != f64 ? 12 > blocks : 4.0 * blocks <= steps)))) {
+    config->variant = 4;
+    config->tm = (m + 3) / 4;
+    config->tn = (n + 3) / 4;
+    config->nt = 64 * (35 < steps || 0 != shortened ? 4 : (12 < steps ? 2 : 1));
+    config->kt = (0 != latency || (0 != shortened && 12 >= steps) ? 16 : 64);
+  }
+  else {
+    config->variant = 2;
+    config->tm = ti;
+    config->tn = tj;
+    config->nt = 64 * (8 < ti * tj ? 2 : ((0 != shortened && 16 < m + n && 4 >= ti * tj && 1 < ti * tj) ? 8 : 4));
+    config->kt = 16;
+  }
+  config->bs = 24;
+  config->split = 2;
+  if (EXIT_SUCCESS != libsmm_acc_config_valid((libsmm_acc_data_t)datatype, m, n, k, config)) return EXIT_FAILURE;
+  if (LXS_SMM_SPLIT_DEFAULT != lxs_cfg.split) config->split = 0; /* the caller's cut factor */
+  else if (0 != shortened) lxs_smm_pieces(datatype, m, n, k, stack_size, config, &config->bs, &config->split);
+  return EXIT_SUCCESS;
+}
+
+/* the configuration of one stack: a tuned row, the environment's or the caller's own model first, then the rule for
+   entry-parallel shapes, then the shipped predictor and the built-in heuristic */
+static void lxs_smm_select(int datatype, int m, int n, int k, int stack_size, libsmm_acc_smm_config_t* config) {
+  const lxs_smm_slot_t* slot;
+  libsmm_acc_smm_config_t env;
+  int untuned;
+  pthread_mutex_lock(&lxs_smm_lock);
+  slot = lxs_smm_lookup(datatype, m, n, k, 0);
+  untuned = (NULL == slot || libsmm_acc_config_learned == slot->source);
+  pthread_mutex_unlock(&lxs_smm_lock);
+  if (0 != untuned && 0 == lxs_learned_is_user() && EXIT_SUCCESS == lxs_smm_rule(datatype, m, n, k, stack_size, config)) {
+    env = *config;
+    if (0 == lxs_smm_env(&env)) return;
+  }
+  lxs_smm_resolve(datatype, m, n, k, config, NULL);
+}
+
 /* the launch arguments of one stack under a configuration (bs scaling, short-stack pair, cut length) */
 static void lxs_smm_fill(lxs_smm_args_t* out, const libsmm_acc_smm_config_t* config, const int* dev_param_stack,
   int stack_size, int datatype, const void* a, const void* b, void* c, int m, int n, int k, int param_format,
@@ -756,6 +849,16 @@ static void lxs_smm_fill(lxs_smm_args_t* out, const libsmm_acc_smm_config_t* con
     const long bs0 = args.bs, cbs = (bs0 > LXS_SMM_BS_MIN ? bs0 : LXS_SMM_BS_MIN);
     const long bs = ((long)stack_size * cbs + config->s - 2) / (config->s - 1);
     args.bs = (int)(bs < bs0 ? (1 > bs ? 1 : bs) : bs0);
+    if (2 <= config->variant && config->variant <= 4 && LXS_SMM_SPLIT_FILL > stack_size &&
+        LXS_SMM_SPLIT_DEFAULT == lxs_cfg.split) {
+      if (4 == config->variant && 256 > args.nt) { /* few wavefronts per run were chosen for many runs */
+        const int nt = args.nt, kt = args.kt;
+        args.nt = 256;
+        args.kt = 16;
+        if (0 == lxs_smm_available(datatype, 4, m, n, k, args.tm, args.tn, args.nt, args.kt)) args.nt = nt, args.kt = kt;
+      }
+      lxs_smm_pieces(datatype, m, n, k, stack_size, config, &args.bs, &split);
+    }
   }
   /* flush: atomic add, which is correct for any stack order (multiply.cl:657,687) and exact-once per
      element for a C-run that is not cut; flush 1 (plain read-modify-write) only when the caller has
@@ -790,7 +893,7 @@ int lxs_smm_enqueue(int datatype, const int* dev_param_stack, int stack_size, co
   libsmm_acc_smm_config_t config;
   lxs_smm_args_t args;
   if (0 >= stack_size) return 0;
-  lxs_smm_resolve(datatype, m, n, k, &config, NULL);
+  lxs_smm_select(datatype, m, n, k, stack_size, &config);
   lxs_smm_fill(&args, &config, dev_param_stack, stack_size, datatype, a, b, c, m, n, k, 0, lxs_cfg.grouped);
   return lxs_smm_launch(&args, hip_stream);
 }
@@ -831,7 +934,7 @@ static int lxs_smm_process(const int* dev_param_stack, int stack_size, libsmm_ac
   if (NULL == dev_param_stack || NULL == dev_a_data || NULL == dev_b_data || NULL == dev_c_data) {
     return lxs_error(EXIT_FAILURE, "libsmm_acc_process: NULL buffer");
   }
-  lxs_smm_resolve((int)datatype, m_max, n_max, k_max, &config, NULL);
+  lxs_smm_select((int)datatype, m_max, n_max, k_max, stack_size, &config);
   if (0 >= config.nt) return -1; /* no compiled kernel covers this shape: host fallback */
   result = lxs_smm_run(&config, dev_param_stack, stack_size, (int)datatype, dev_a_data, dev_b_data, dev_c_data, m_max,
     n_max, k_max, stack_stream, param_format, lxs_cfg.grouped);

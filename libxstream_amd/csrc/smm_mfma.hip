@@ -581,6 +581,18 @@ __device__ __forceinline__ void ep_body(T* __restrict__ cdata, const T* __restri
     }
   };
 
+  /* LDS only: loads in flight stay in flight; one wavefront needs no barrier */
+  const auto sync = [&]() {
+    if constexpr (1 < EP) {
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+      __builtin_amdgcn_s_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+    }
+    else {
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+    }
+  };
   for (;;) { /* one run (or piece of a cut run) [h, r) per iteration */
     const int c0 = c_uni(h);
     const int r = run_end(h, c0);
@@ -624,9 +636,7 @@ __device__ __forceinline__ void ep_body(T* __restrict__ cdata, const T* __restri
        the flush, tiles shared out */
     fold();
     folded = false;
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+    sync();
     if constexpr (2 == B4) { /* four instructions t at a time, one per quarter-wavefront: row i, column j */
       T* const cblk = cdata + (c0 - pz);
       const int x = lane & 15, rb = TI * (x >> 2), cb = TJ * (x & 3);
@@ -697,10 +707,8 @@ __device__ __forceinline__ void ep_body(T* __restrict__ cdata, const T* __restri
         }
       }
     }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-    __builtin_amdgcn_s_barrier(); /* every sum is read before the next run's partials overwrite LDS */
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
     if (!own_next) break;
+    sync(); /* every sum is read before the next run's partials overwrite LDS */
     h = r;
   }
 #undef LXS_LOAD_KSTEP
@@ -722,7 +730,7 @@ __global__ void __launch_bounds__(64 * EP, (6 == KB && 9 == TI * TJ ? 3 : 4)) sm
 }
 /* FP64 on 4x4 blocks that split k: C blocks up to 4 TI x 4 TJ, KB k-steps of 16 per stage */
 template <typename T, int TI, int TJ, int EP, int KB, int MC, int NC, int KC>
-__global__ void __launch_bounds__(64 * EP, 4) smm_mfma_ek(LXS_EP_ARGS) {
+__global__ void __launch_bounds__(64 * EP, (4 == KB && 8 <= TI * TJ ? 3 : 4)) smm_mfma_ek(LXS_EP_ARGS) {
   ep_body<T, TI, TJ, EP, KB, MC, NC, KC, 2>(LXS_EP_PASS);
 }
 
@@ -796,6 +804,19 @@ const mfma_entry_t mfma_table[] = {
   LXS_EKG(3, 1, 8, 1) LXS_EKG(3, 2, 8, 1) LXS_EKG(3, 3, 8, 1) LXS_EKG(3, 4, 8, 1) LXS_EKG(4, 1, 8, 1) LXS_EKG(4, 2, 8, 1)
   LXS_EKG(4, 3, 8, 1) LXS_EKG(4, 4, 8, 1) LXS_EKG(1, 1, 4, 2) LXS_EKG(1, 2, 4, 2) LXS_EKG(1, 3, 4, 2) LXS_EKG(1, 4, 4, 2)
   LXS_EKG(2, 1, 4, 2) LXS_EKG(2, 2, 4, 2) LXS_EKG(3, 1, 4, 2) LXS_EKG(4, 1, 4, 2)
+  /* the same for large and small numbers of runs by rule (lxs_smm_rule): 64 of k per stage, 1, 2 or 4 wavefronts per run */
+  LXS_EKG(1, 1, 1, 4) LXS_EKG(1, 2, 1, 4) LXS_EKG(1, 3, 1, 4) LXS_EKG(1, 4, 1, 4)
+  LXS_EKG(2, 1, 1, 4) LXS_EKG(2, 2, 1, 4) LXS_EKG(2, 3, 1, 4) LXS_EKG(2, 4, 1, 4)
+  LXS_EKG(3, 1, 1, 4) LXS_EKG(3, 2, 1, 4) LXS_EKG(3, 3, 1, 4) LXS_EKG(3, 4, 1, 4)
+  LXS_EKG(4, 1, 1, 4) LXS_EKG(4, 2, 1, 4) LXS_EKG(4, 3, 1, 4) LXS_EKG(4, 4, 1, 4)
+  LXS_EKG(1, 1, 2, 4) LXS_EKG(1, 2, 2, 4) LXS_EKG(1, 3, 2, 4) LXS_EKG(1, 4, 2, 4)
+  LXS_EKG(2, 1, 2, 4) LXS_EKG(2, 2, 2, 4) LXS_EKG(2, 3, 2, 4) LXS_EKG(2, 4, 2, 4)
+  LXS_EKG(3, 1, 2, 4) LXS_EKG(3, 2, 2, 4) LXS_EKG(3, 3, 2, 4) LXS_EKG(3, 4, 2, 4)
+  LXS_EKG(4, 1, 2, 4) LXS_EKG(4, 2, 2, 4) LXS_EKG(4, 3, 2, 4) LXS_EKG(4, 4, 2, 4)
+  LXS_EKG(1, 1, 4, 4) LXS_EKG(1, 2, 4, 4) LXS_EKG(1, 3, 4, 4) LXS_EKG(1, 4, 4, 4)
+  LXS_EKG(2, 1, 4, 4) LXS_EKG(2, 2, 4, 4) LXS_EKG(2, 3, 4, 4) LXS_EKG(2, 4, 4, 4)
+  LXS_EKG(3, 1, 4, 4) LXS_EKG(3, 2, 4, 4) LXS_EKG(3, 3, 4, 4) LXS_EKG(3, 4, 4, 4)
+  LXS_EKG(4, 1, 4, 4) LXS_EKG(4, 2, 4, 4) LXS_EKG(4, 3, 4, 4) LXS_EKG(4, 4, 4, 4)
 };
 
 } /* namespace */
