@@ -78,10 +78,20 @@ int lxs_trans_launch(const int* trs_stack, int offset, int stack_size, void* dat
   void* hip_stream);
 int lxs_zero_launch(void* ptr, size_t nbytes, void* hip_stream);
 
-/* Ozaki scheme I (ozaki.hip). Operand element (r, k) at p[r * rs + k * ks] (rs or ks is 1);
-   planes: s x Rp x Kp int8 (Rp multiple of 256, Kp multiple of 128); e: Rp ints; occ: 8 ints */
-int lxs_oz_preprocess(int dtype, const void* p, long rs, long ks, int R, int K, int s, int Rp, int Kp, int* e,
-  int* occ, signed char* planes, void* hip_stream);
+/* One operand of an Ozaki product (ozaki.hip): element (r, k) at p[r * rs + k * ks] (rs or ks is 1), r < R;
+   planes: digit or residue planes of Rp x Kp int8 (Rp multiple of 256, Kp multiple of 128); e: Rp ints; occ: 8 ints
+   (scheme 1), else NULL */
+typedef struct lxs_oz_operand_t {
+  const void* p;
+  long rs, ks;
+  int R, Rp;
+  int* e;
+  int* occ;
+  signed char* planes;
+} lxs_oz_operand_t;
+/* scheme 1: exponents and s digit planes of both operands */
+int lxs_oz_preprocess(int dtype, const lxs_oz_operand_t* a, const lxs_oz_operand_t* b, int K, int s, int Kp,
+  void* hip_stream);
 /* int8 GEMM over work items {level, u0, u1, pad} (host array), element (i, j) of item z at
    out + z Mp Np + j Mp + i. crt = 0 (scheme 1): s digit planes, item level L over the pairs (p, L - p),
    int32 partials, at most 2080 units (pair, k-block of 64) per item. crt = 1 (scheme 2): s residue
@@ -107,13 +117,13 @@ int lxs_oz_scale(int dtype, void* c, int ldc, int M, int N, double beta, void* h
 int lxs_oz_static_scratch(void** ptr);
 /* Ozaki scheme 2 (CRT): moduli in use order, pairwise coprime and at most 256, so that symmetric residues
    fit int8; the first np of them serve a call. Residue planes: np x Rp x Kp int8 of the integers
-   trunc(|v| 2^(mb - trim - E)) (E: the row's exponent, mb = 53 or 24) with the sign of v, times the
-   reconstruction weight w_p = ((M / m_p) mod m_p)^-1 mod m_p when weight != 0 (one operand carries it, so
-   the int8 GEMM's residues are the CRT coefficients). */
+   trunc(|v| 2^(mb - trim - E)) (E: the row's exponent, mb = 53 or 24) with the sign of v, those of a times the
+   reconstruction weight w_p = ((M / m_p) mod m_p)^-1 mod m_p (one operand carries it, so the int8 GEMM's residues are
+   the CRT coefficients). */
 #define LXS_OZ_NPRIMES_MAX 16
 #define LXS_OZ_MODULI 256, 255, 253, 251, 247, 241, 239, 233, 229, 227, 223, 211, 199, 197, 193, 191
-int lxs_oz_crt_preprocess(int dtype, const void* p, long rs, long ks, int R, int K, int np, int weight, int trim, int Rp,
-  int Kp, int* e, signed char* planes, void* hip_stream);
+int lxs_oz_crt_preprocess(int dtype, const lxs_oz_operand_t* a, const lxs_oz_operand_t* b, int K, int np, int trim, int Kp,
+  void* hip_stream);
 /* C = alpha 2^(ea + eb + sh0) x + beta C, x the integer (|x| < M / 2, M the product of the first np moduli) whose
    CRT coefficients c_p = x w_p mod m_p are the sums of the residue bytes of the prime's items zb[p] .. zb[p + 1] - 1,
    mod m_p (the A operand's residues carry w_p) */

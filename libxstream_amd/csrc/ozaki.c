@@ -458,22 +458,12 @@ static int oz_gemm_real(ozaki_context_t* ctx, hipStream_t hs, int ta, int tb, in
       const double nprod = (0 != l.crt ? np : ozaki_count_pairs(s, cutoff, 0));
       const int nplanes = (0 != l.crt ? np : s);
       void* token = (NULL == fixed ? lxs_profile_begin(hs) : NULL);
-      if (0 != l.crt) {
-        result = lxs_oz_crt_preprocess(dtype, da + ts * (size_t)k0 * aks, ars, aks, M, kk, np, 1, trim, l.Mp, Kp,
-          (int*)(base + l.ea), (signed char*)(base + l.planes_a), hs);
-        if (0 == result) {
-          result = lxs_oz_crt_preprocess(dtype, db + ts * (size_t)k0 * bks, bcs, bks, N, kk, np, 0, trim, l.Np, Kp,
-            (int*)(base + l.eb), (signed char*)(base + l.planes_b), hs);
-        }
-      }
-      else {
-        result = lxs_oz_preprocess(dtype, da + ts * (size_t)k0 * aks, ars, aks, M, kk, s, l.Mp, Kp, (int*)(base + l.ea), occ,
-          (signed char*)(base + l.planes_a), hs);
-        if (0 == result) {
-          result = lxs_oz_preprocess(dtype, db + ts * (size_t)k0 * bks, bcs, bks, N, kk, s, l.Np, Kp, (int*)(base + l.eb),
-            occ + 8, (signed char*)(base + l.planes_b), hs);
-        }
-      }
+      const lxs_oz_operand_t oa = {da + ts * (size_t)k0 * aks, ars, aks, M, l.Mp, (int*)(base + l.ea),
+        0 == l.crt ? occ : NULL, (signed char*)(base + l.planes_a)};
+      const lxs_oz_operand_t ob = {db + ts * (size_t)k0 * bks, bcs, bks, N, l.Np, (int*)(base + l.eb),
+        0 == l.crt ? occ + 8 : NULL, (signed char*)(base + l.planes_b)};
+      if (0 != l.crt) result = lxs_oz_crt_preprocess(dtype, &oa, &ob, kk, np, trim, Kp, hs);
+      else result = lxs_oz_preprocess(dtype, &oa, &ob, kk, s, Kp, hs);
       lxs_profile_end(token, hs, "ozaki_pre", 0.0, (double)ts * ((double)M + N) * kk + (double)nplanes * (l.Mp + l.Np) * Kp);
       if (0 == result && 0 != pairs) { /* every pair, level and the recombination in one kernel */
         token = (NULL == fixed ? lxs_profile_begin(hs) : NULL);

@@ -13,7 +13,7 @@
  * Zero, subnormal and non-finite inputs count as zero (ozaki_common.cl:784-805).
  *
  * Kernels (new design for MI355X):
- *   oz_init     exponents := none, occupancy := 0
+ *   oz_init     exponents := none, occupancy := 0 (this and the next two: both operands per launch)
  *   oz_exp      per-row (A) / per-column (B) exponent: max over the row of (biased exponent - bias + 1)
  *   oz_slice    digits of 64x64 tiles into s planes [s][Rp][Kp] (k contiguous, rows padded to 256,
  *               k to 128, padding zero), so GEMM operand tiles are plain 16-byte vectors; sets one
@@ -117,22 +117,47 @@ __device__ __forceinline__ void oz_load16(double* v, const T* __restrict__ p, lo
   }
 }
 
-__global__ void __launch_bounds__(256) oz_init(int* __restrict__ e, int n, int* __restrict__ occ) {
-  const int i = blockIdx.x * 256 + threadIdx.x;
-  if (i < n) e[i] = OZ_EXP_NONE;
-  if (NULL != occ && 0 == blockIdx.x && (int)threadIdx.x < 8) occ[threadIdx.x] = 0;
+/*
+ * The three preprocessing passes (init, exponents, planes) each take both operands in one launch: work-groups below
+ * ga belong to a, the others to b. A pass over one operand of 1000 x 1000 lasts about as long as its launch and fills
+ * a quarter of the device. Scheme 1, us a call with 3 and with 6 launches: 100x200x300 43 and 51, 1000x1100x900 131 and
+ * 142; scheme 2 39 and 54, 89 and 102 (4096^3: 1390 and 1410).
+ */
+struct oz_op_t {
+  lxs_oz_operand_t o;
+  int nx; /* tiles along the grid's first dimension */
+};
+
+__global__ void __launch_bounds__(256) oz_init(lxs_oz_operand_t a, lxs_oz_operand_t b) {
+  const int x = blockIdx.x * 256 + threadIdx.x, i = x - a.Rp; /* Rp: a multiple of 256 */
+  int* const e = (0 > i ? a.e + x : b.e + i);
+  *e = OZ_EXP_NONE;
+  if (0 == blockIdx.x && NULL != a.occ && threadIdx.x < 16) (threadIdx.x < 8 ? a.occ : b.occ)[threadIdx.x & 7] = 0;
+}
+
+/* operand and tile of a work-group */
+__device__ __forceinline__ lxs_oz_operand_t oz_pick(const oz_op_t& a, const oz_op_t& b, int ga, int& bx, int& by) {
+  const bool first = ((int)blockIdx.x < ga);
+  const int t = (int)blockIdx.x - (first ? 0 : ga), nx = (first ? a.nx : b.nx);
+  by = t / nx;
+  bx = t - by * nx;
+  return (first ? a.o : b.o);
 }
 
 template <typename T>
-__global__ void __launch_bounds__(256) oz_exp(const T* __restrict__ p, long rs, long ks, int R, int K,
-  int* __restrict__ e) {
+__global__ void __launch_bounds__(256) oz_exp(oz_op_t a, oz_op_t b, int ga, int K) {
   __shared__ int red[4][64];
+  int bx, by;
+  const lxs_oz_operand_t o = oz_pick(a, b, ga, bx, by);
+  const long rs = o.rs, ks = o.ks;
+  const int R = o.R;
+  int* const e = o.e;
   /* consecutive work-groups along the contiguous dimension */
-  const int r0 = (1 == ks ? blockIdx.y : blockIdx.x) * OZ_TILE, k0 = (1 == ks ? blockIdx.x : blockIdx.y) * OZ_TILE;
+  const int r0 = (1 == ks ? by : bx) * OZ_TILE, k0 = (1 == ks ? bx : by) * OZ_TILE;
   int r, kq;
   oz_owner(rs, r, kq);
   double v[16];
-  oz_load16<T>(v, p, rs, ks, r0 + r, k0 + kq, R, K);
+  oz_load16<T>(v, (const T*)o.p, rs, ks, r0 + r, k0 + kq, R, K);
   int ex = OZ_EXP_NONE;
 #pragma unroll
   for (int x = 0; x < 16; ++x) ex = max(ex, oz_expo(v[x]));
@@ -151,24 +176,23 @@ __global__ void __launch_bounds__(256) oz_exp(const T* __restrict__ p, long rs, 
   }
 }
 
-/* exponent pass: 64 x 64 tiles, the first grid dimension along the contiguous one */
-static dim3 oz_exp_grid(long ks, int Rp, int Kp) {
-  return (1 == ks) ? dim3((unsigned int)(Kp / OZ_TILE), (unsigned int)(Rp / OZ_TILE))
-                   : dim3((unsigned int)(Rp / OZ_TILE), (unsigned int)(Kp / OZ_TILE));
-}
-
 /* s int8 digits of 16 consecutive k of one row, written as one 16-byte vector per plane */
 template <typename T>
-__global__ void __launch_bounds__(256) oz_slice(const T* __restrict__ p, long rs, long ks, int R, int K,
-  const int* __restrict__ e, int s, int Rp, int Kp, int8_t* __restrict__ planes, int* __restrict__ occ) {
-  const int r0 = blockIdx.x * OZ_TILE, k0 = blockIdx.y * OZ_TILE;
+__global__ void __launch_bounds__(256) oz_slice(oz_op_t a, oz_op_t b, int ga, int K, int s, int Kp) {
+  int bx, by;
+  const lxs_oz_operand_t o = oz_pick(a, b, ga, bx, by);
+  const int r0 = bx * OZ_TILE, k0 = by * OZ_TILE, R = o.R, Rp = o.Rp;
+  const long rs = o.rs, ks = o.ks;
+  const int* const e = o.e;
+  int* const occ = o.occ;
+  int8_t* const planes = (int8_t*)o.planes;
   const int tid = threadIdx.x;
   int r, kq;
   oz_owner(rs, r, kq);
   const int row = r0 + r;
   const int ex = (row < R ? e[row] : OZ_EXP_NONE);
   double x[16];
-  oz_load16<T>(x, p, rs, ks, row, k0 + kq, R, K);
+  oz_load16<T>(x, (const T*)o.p, rs, ks, row, k0 + kq, R, K);
 #pragma unroll
   for (int i = 0; i < 16; ++i) x[i] = (OZ_EXP_NONE != ex ? ldexp(x[i], -ex) : 0.0); /* |x| < 1, exact */
   for (int pl = 0; pl < s; ++pl) {
@@ -592,8 +616,8 @@ __device__ __forceinline__ unsigned int oz_mod27(unsigned int x, int p) {
 /*
  * Residue planes of one 64 x 64 tile: every element v of row r with the row's exponent E (|v| < 2^E)
  * becomes the integer a = trunc(|v| 2^(mb - t - E)) (mb = 53 for FP64, 24 for FP32; t trimmed bits);
- * plane p holds the symmetric residue of sign(v) a w_p mod m_p, in [lo_p, lo_p + m_p), as int8 (w_p: 1, or
- * the reconstruction weight for weight = np > 0, see oz_res_tab_t). A thread owns 16 consecutive k of one
+ * plane p holds the symmetric residue of sign(v) a w_p mod m_p, in [lo_p, lo_p + m_p), as int8 (w_p: 1 for operand b,
+ * the reconstruction weight for operand a, see oz_res_tab_t). A thread owns 16 consecutive k of one
  * row and writes one 16-byte vector per plane.
  * Per plane and element: x = sum of the 7 bytes of a times 2^(8 i) w mod m (two byte dot products,
  * x < 7 * 255^2 < 2^19, x = a w mod m), y = x - lo or m 2^12 - x - lo by the sign (so y = sign a w - lo
@@ -602,16 +626,20 @@ __device__ __forceinline__ unsigned int oz_mod27(unsigned int x, int p) {
  * of 1 / m >= 2^-8), and the residue is lo + (y mod m).
  */
 template <typename T>
-__global__ void __launch_bounds__(256) oz_residues(const T* __restrict__ p, long rs, long ks, int R, int K,
-  const int* __restrict__ e, int np, int weight, int mb, int trim, int Rp, int Kp, int8_t* __restrict__ planes) {
-  const int r0 = blockIdx.x * OZ_TILE, k0 = blockIdx.y * OZ_TILE;
+__global__ void __launch_bounds__(256) oz_residues(oz_op_t a, oz_op_t b, int ga, int K, int np, int mb, int trim, int Kp) {
+  int bx, by;
+  const lxs_oz_operand_t o = oz_pick(a, b, ga, bx, by);
+  const int r0 = bx * OZ_TILE, k0 = by * OZ_TILE, R = o.R, Rp = o.Rp;
+  const long rs = o.rs, ks = o.ks;
+  const int* const e = o.e;
+  int8_t* const planes = (int8_t*)o.planes;
   /* four lanes per row (k chunks of 16), 16 rows per wavefront, for either operand layout: each lane's 16
      residue bytes of a plane continue its neighbour's, so a wavefront stores 1 KB contiguous per plane */
   const int r = (int)threadIdx.x >> 2, kq = ((int)threadIdx.x & 3) * 16;
   const int row = r0 + r;
   const int ex = (row < R ? e[row] : OZ_EXP_NONE);
   double t[16];
-  oz_load16<T>(t, p, rs, ks, row, k0 + kq, R, K);
+  oz_load16<T>(t, (const T*)o.p, rs, ks, row, k0 + kq, R, K);
   unsigned int alo[16], ahi[16]; /* a = ahi 2^32 + alo, a < 2^53 */
   unsigned int nm[16];           /* all ones for negative v, else 0 */
 #pragma unroll
@@ -626,7 +654,7 @@ __global__ void __launch_bounds__(256) oz_residues(const T* __restrict__ p, long
     ahi[i] = (unsigned int)(a >> 32);
     nm[i] = 0u - (unsigned int)(bits >> 63);
   }
-  const int w = (0 != weight ? np : 0);
+  const int w = ((int)blockIdx.x < ga ? np : 0); /* a carries the weight */
 #pragma unroll
   for (int pl = 0; pl < LXS_OZ_NPRIMES_MAX; ++pl) {
     if (pl < np) {
@@ -1110,24 +1138,37 @@ __global__ void __launch_bounds__(256) oz_ccombine(const T* __restrict__ t1, con
 } /* namespace */
 
 /* digit planes, exponents and occupancy of one operand: element (r, k) at p[r * rs + k * ks] */
-extern "C" int lxs_oz_preprocess(int dtype, const void* p, long rs, long ks, int R, int K, int s, int Rp, int Kp,
-  int* e, int* occ, signed char* planes, void* hip_stream) {
+/* both operands' tiles: the first grid dimension along the contiguous one (along: exponents) or along the rows */
+static unsigned int oz_tiles(const lxs_oz_operand_t* a, const lxs_oz_operand_t* b, int Kp, int along, oz_op_t* oa,
+  oz_op_t* ob) {
+  oa->o = *a;
+  ob->o = *b;
+  oa->nx = (0 != along && 1 == a->ks ? Kp : a->Rp) / OZ_TILE;
+  ob->nx = (0 != along && 1 == b->ks ? Kp : b->Rp) / OZ_TILE;
+  return (unsigned int)((long)(a->Rp / OZ_TILE) * (Kp / OZ_TILE));
+}
+static int oz_operands_ok(const lxs_oz_operand_t* a, const lxs_oz_operand_t* b, int K, int Kp) {
+  const lxs_oz_operand_t* o[2] = {a, b};
+  for (int i = 0; i < 2; ++i) {
+    if (0 >= o[i]->Rp || 0 != o[i]->Rp % LT || o[i]->Rp < o[i]->R || !((1 == o[i]->rs) || (1 == o[i]->ks))) return 0;
+  }
+  return 0 == Kp % LK && 0 < Kp && Kp >= K && 2147483647L >= ((long)a->Rp + b->Rp) / OZ_TILE * (Kp / OZ_TILE);
+}
+
+extern "C" int lxs_oz_preprocess(int dtype, const lxs_oz_operand_t* a, const lxs_oz_operand_t* b, int K, int s, int Kp,
+  void* hip_stream) {
   const hipStream_t st = (hipStream_t)hip_stream;
-  const dim3 egrid = oz_exp_grid(ks, Rp, Kp), grid((unsigned int)(Rp / OZ_TILE), (unsigned int)(Kp / OZ_TILE));
-  if (0 != Rp % LT || 0 != Kp % LK || Rp < R || Kp < K || 0 >= Kp || 1 > s || 8 < s) return LXS_ELIMIT;
-  if (!((1 == rs) || (1 == ks))) return LXS_ELIMIT;
-  oz_init<<<(Rp + 255) / 256, 256, 0, st>>>(e, Rp, occ);
-  if (3 == dtype) {
-    oz_exp<double><<<egrid, 256, 0, st>>>((const double*)p, rs, ks, R, K, e);
-    oz_slice<double><<<grid, 256, 0, st>>>((const double*)p, rs, ks, R, K, e, s, Rp, Kp, planes, occ);
-  }
-  else if (1 == dtype) {
-    oz_exp<float><<<egrid, 256, 0, st>>>((const float*)p, rs, ks, R, K, e);
-    oz_slice<float><<<grid, 256, 0, st>>>((const float*)p, rs, ks, R, K, e, s, Rp, Kp, planes, occ);
-  }
-  else {
-    return LXS_ENOVARIANT;
-  }
+  oz_op_t oa, ob;
+  if (3 != dtype && 1 != dtype) return LXS_ENOVARIANT;
+  if (0 == oz_operands_ok(a, b, K, Kp) || 1 > s || 8 < s) return LXS_ELIMIT;
+  const unsigned int ga = oz_tiles(a, b, Kp, 1, &oa, &ob);
+  const unsigned int grid = ga + (unsigned int)((long)(b->Rp / OZ_TILE) * (Kp / OZ_TILE));
+  oz_init<<<(a->Rp + b->Rp) / 256, 256, 0, st>>>(*a, *b);
+  if (3 == dtype) oz_exp<double><<<grid, 256, 0, st>>>(oa, ob, (int)ga, K);
+  else oz_exp<float><<<grid, 256, 0, st>>>(oa, ob, (int)ga, K);
+  (void)oz_tiles(a, b, Kp, 0, &oa, &ob);
+  if (3 == dtype) oz_slice<double><<<grid, 256, 0, st>>>(oa, ob, (int)ga, K, s, Kp);
+  else oz_slice<float><<<grid, 256, 0, st>>>(oa, ob, (int)ga, K, s, Kp);
   return (int)hipGetLastError();
 }
 
@@ -1226,27 +1267,21 @@ extern "C" int lxs_oz_level_gemm(int crt, const signed char* pa, const signed ch
   return (int)hipGetLastError();
 }
 
-extern "C" int lxs_oz_crt_preprocess(int dtype, const void* p, long rs, long ks, int R, int K, int np, int weight,
-  int trim, int Rp, int Kp, int* e, signed char* planes, void* hip_stream) {
+extern "C" int lxs_oz_crt_preprocess(int dtype, const lxs_oz_operand_t* a, const lxs_oz_operand_t* b, int K, int np,
+  int trim, int Kp, void* hip_stream) {
   const hipStream_t st = (hipStream_t)hip_stream;
-  const dim3 egrid = oz_exp_grid(ks, Rp, Kp), grid((unsigned int)(Rp / OZ_TILE), (unsigned int)(Kp / OZ_TILE));
   const int mb = (3 == dtype ? 53 : 24);
-  if (0 != Rp % LT || 0 != Kp % LK || Rp < R || Kp < K || 0 >= Kp || 1 > np || LXS_OZ_NPRIMES_MAX < np) return LXS_ELIMIT;
-  if (!((1 == rs) || (1 == ks)) || 0 > trim || mb <= trim) return LXS_ELIMIT;
-  oz_init<<<(Rp + 255) / 256, 256, 0, st>>>(e, Rp, NULL);
-  if (3 == dtype) {
-    oz_exp<double><<<egrid, 256, 0, st>>>((const double*)p, rs, ks, R, K, e);
-    oz_residues<double><<<grid, 256, 0, st>>>((const double*)p, rs, ks, R, K, e, np, weight, mb, trim, Rp, Kp,
-      (int8_t*)planes);
-  }
-  else if (1 == dtype) {
-    oz_exp<float><<<egrid, 256, 0, st>>>((const float*)p, rs, ks, R, K, e);
-    oz_residues<float><<<grid, 256, 0, st>>>((const float*)p, rs, ks, R, K, e, np, weight, mb, trim, Rp, Kp,
-      (int8_t*)planes);
-  }
-  else {
-    return LXS_ENOVARIANT;
-  }
+  oz_op_t oa, ob;
+  if (3 != dtype && 1 != dtype) return LXS_ENOVARIANT;
+  if (0 == oz_operands_ok(a, b, K, Kp) || 1 > np || LXS_OZ_NPRIMES_MAX < np || 0 > trim || mb <= trim) return LXS_ELIMIT;
+  const unsigned int ga = oz_tiles(a, b, Kp, 1, &oa, &ob);
+  const unsigned int grid = ga + (unsigned int)((long)(b->Rp / OZ_TILE) * (Kp / OZ_TILE));
+  oz_init<<<(a->Rp + b->Rp) / 256, 256, 0, st>>>(*a, *b);
+  if (3 == dtype) oz_exp<double><<<grid, 256, 0, st>>>(oa, ob, (int)ga, K);
+  else oz_exp<float><<<grid, 256, 0, st>>>(oa, ob, (int)ga, K);
+  (void)oz_tiles(a, b, Kp, 0, &oa, &ob);
+  if (3 == dtype) oz_residues<double><<<grid, 256, 0, st>>>(oa, ob, (int)ga, K, np, mb, trim, Kp);
+  else oz_residues<float><<<grid, 256, 0, st>>>(oa, ob, (int)ga, K, np, mb, trim, Kp);
   return (int)hipGetLastError();
 }
 
