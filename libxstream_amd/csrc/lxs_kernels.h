@@ -139,10 +139,10 @@ int lxs_oz_ccombine(int dtype, const void* t1, const void* t2, const void* t3, i
   const double* beta, void* c, int ldc, void* hip_stream);
 
 /* Ozaki scheme I over a parameter stack (ozaki_stack.hip): planes_a na * s * 4 KB, planes_b nb * s * 4 KB,
-   ea na * 64 ints, eb nb * 64 ints, info 1 int of device scratch */
+   ea na * 64 ints, eb nb * 64 ints, info 1 int of device scratch; ncus: CUs of the device */
 int lxs_ozs_process(int dtype, const int* stack, int S, int m, int n, int k, const void* a, int na, const void* b,
   int nb, void* c, int s, int cutoff, signed char* planes_a, int* ea, signed char* planes_b, int* eb, int* info,
-  void* hip_stream);
+  int ncus, void* hip_stream);
 
 /* learned predictor MLP (mlp.hip): activations [batch][features], weights [out][in] then bias [out] */
 int lxs_mlp_forward(const float* x, const float* w, int batch, int nin, int nout, int relu, float* y, void* hip_stream);

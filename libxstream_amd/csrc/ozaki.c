@@ -652,7 +652,8 @@ LIBXSTREAM_API int ozaki_stack(ozaki_context_t* ctx, libxstream_stream_t* stream
   token = lxs_profile_begin(hs);
   result = lxs_ozs_process(dtype, dev_stack, stack_size, m, n, k, dev_a, na, dev_b, nb, dev_c, s, oz_cutoff(ctx),
     (signed char*)base, (int*)(base + pla + plb), (signed char*)(base + pla),
-    (int*)(base + pla + plb + oz_up(sizeof(int) * 64 * (size_t)na, OZ_ALIGN)), (int*)(base + need - OZ_ALIGN), hs);
+    (int*)(base + pla + plb + oz_up(sizeof(int) * 64 * (size_t)na, OZ_ALIGN)), (int*)(base + need - OZ_ALIGN),
+    lxs_cfg.ncus, hs);
   lxs_profile_end(token, hs, "ozaki_stack", 2.0 * stack_size * m * n * k,
     (double)stack_size * (0 != ctx->use_double ? 8 : 4) * ((double)m * k + (double)k * n + 2.0 * m * n));
   return (0 == result ? EXIT_SUCCESS : lxs_error(EXIT_FAILURE, "ozaki_stack: kernel launch failed"));

@@ -14,7 +14,7 @@
  *               (FP64, or FP32 updated through FP64); per entry the 2s digit planes of its A and B
  *               blocks move into LDS by DMA (double-buffered across entries), every level sum
  *               S_L = sum over pairs p + q = L of A_p B_q^T (64 x 64 x 64) accumulates exactly in its own
- *               int32 tile (v_mfma_i32_32x32x32_i8, 4 wavefronts of 32 x 32), then
+ *               int32 tile (v_mfma_i32_16x16x64_i8, 8 wavefronts of 32 x 16), then
  *               cd = sum over L = cutoff .. 0 of 2^(-7(L+2)) S_L in FP64 and C += 2^(ea_i + eb_j) cd.
  *               A stack that is not sorted by C is processed by one work-group, run after run, in order.
  * Every element of C is therefore updated entry by entry in stack order, reproducibly.
@@ -103,25 +103,39 @@ __device__ __forceinline__ void ozs_dma4(const int* src, int8_t* lds_dst) {
   __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
     (__attribute__((address_space(3))) void*)lds_dst, 4, 0, 0);
 }
-constexpr int SEX = 512; /* LDS bytes per wavefront for an entry's exponent rows (A rows, then B columns) */
+constexpr int SEX = 2 * SB * 4; /* LDS bytes of an entry's exponent rows (A rows, then B columns) */
 
 /*
- * LDS: two entry buffers of 2 NS planes (A planes, then B planes), 4 KB each, and each wavefront's copy of the
- * entry's exponent rows (2 x 256 bytes); row r of a plane holds its
- * 4 chunks of 16 bytes with chunk c at position c ^ ((r >> 2) & 3). Wave w moves rows 16 w .. 16 w + 15 of
- * every plane (one DMA instruction per plane: lane l writes position l % 4 of row 16 w + l / 4).
+ * LDS: two entry buffers of 2 NS planes (A planes, then B planes), 4 KB each, and the entry's exponent rows; row r of a
+ * plane holds its 4 chunks of 16 bytes with chunk c at position c ^ ((r >> 2) & 3). Wavefronts 0..3 move the planes
+ * of A, 4..7 those of B, wavefront w rows 16 (w & 3) .. + 15 (one DMA instruction per plane: lane l writes position
+ * l % 4 of row 16 (w & 3) + l / 4); rows past m or n are not moved, what they leave in the tile is not stored.
+ *
+ * 8 wavefronts, two per SIMD, each 32 x 16 elements of the block (v_mfma_i32_16x16x64_i8: all 64 k in one instruction,
+ * the B planes as first operand): 15 level sums of 8 registers each for 8 slices over all pairs. Wavefronts 4..7 cross the
+ * barrier of an entry between its products and its recombination, 0..3 before its products: on every SIMD one
+ * wavefront's FP64 recombination (120 conversions and 120 FMA) runs beside the other's products. The entries of a
+ * work-group follow each other without a break from run to run, and the records of 64 of them are one lane each
+ * (chains of dependent scalar loads before an entry's DMA: 1791 -> 1976 us below).
+ * Bound: 8 slices over all pairs, the products (4096 cycles an entry and SIMD) and what of the DMA (64 KB an entry, 3.7 TB/s
+ * over the device) and the barrier they do not cover. With 4 wavefronts of 32 x 32, one per SIMD, products and
+ * recombination took turns. us a call, before -> now: FP64 64x64x64, 100000 entries, 8 slices 2583 -> 1791, 20000 entries, 7
+ * slices 584 -> 326; 23x23x23, 50000, 8 slices 1379 -> 517; 33x13x50, 5000, 6 slices 175 -> 76; FP32 64x30x64, 100000, 3 slices
+ * 603 -> 354. Work-groups as many as are resident: 256 (5 to 8 slices) 517 us and 512 625 us for 23x23x23 above, two per
+ * CU for 3 and 4 slices (FP32 45x45x13, 60000, 4 slices: 512 353 us, 256 488, 1024 401).
  */
 template <typename T, int NS, int CUT>
-__global__ void __launch_bounds__(256) ozs_stack(const int* __restrict__ stack, int S, const int* __restrict__ info,
-  const int8_t* __restrict__ pa, const int* __restrict__ ea, const int8_t* __restrict__ pb, const int* __restrict__ eb,
-  int cutoff_rt, int m, int n, int k, int na, int nb, T* __restrict__ c) {
+__global__ void __launch_bounds__(512, (4 >= NS ? 4 : 2)) ozs_stack(const int* __restrict__ stack, int S,
+  const int* __restrict__ info, const int8_t* __restrict__ pa, const int* __restrict__ ea, const int8_t* __restrict__ pb,
+  const int* __restrict__ eb, int cutoff_rt, int m, int n, int k, int na, int nb, T* __restrict__ c) {
   /* the level cutoff: compiled in (CUT >= 0), so the pair loop below has no conditional matrix-core work,
      or taken at run time (CUT < 0) */
   const int cutoff = (0 <= CUT ? CUT : cutoff_rt);
-  __shared__ __attribute__((aligned(1024))) int8_t lds0[2 * NS * SPL + 4 * SEX], lds1[2 * NS * SPL + 4 * SEX];
+  __shared__ __attribute__((aligned(1024))) int8_t lds0[2 * NS * SPL + SEX], lds1[2 * NS * SPL + SEX];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wi = wave & 1, wj = wave >> 1;
+  const int late = wave >> 2; /* 1: recombines an entry after the next barrier */
+  const int wi = wave & 1, wj = ((wave >> 1) & 1) + 2 * late;
   const int unsorted = info[0];
   const unsigned int mk = (unsigned int)(m * k), kn = (unsigned int)(k * n);
   /* this work-group's share of the stack (all of it for work-group 0 when the stack is not grouped by C) */
@@ -129,133 +143,146 @@ __global__ void __launch_bounds__(256) ozs_stack(const int* __restrict__ stack, 
   const int lo = (0 != unsorted ? 0 : (int)blockIdx.x * share);
   const int hi = (0 != unsorted ? S : (lo + share < S ? lo + share : S));
   if (0 != unsorted && 0 != blockIdx.x) return;
-  /* this lane's element of the 32 x 32 tile: column i (A rows), rows j (B columns) per register */
-  const int i = 32 * wi + (lane & 31);
-  const int drow = 16 * wave + (lane >> 2), dchunk = (lane & 3) ^ ((lane >> 4) & 3);
-  const int frow = lane & 31, fswz = (frow >> 2) & 3;
-  const int fpos0 = (lane >> 5) ^ fswz, fpos1 = (2 + (lane >> 5)) ^ fswz;
-  /* run boundaries found 64 entries at a time (one lane each, then a ballot) */
-  int e0 = lo; /* the first run that starts in [lo, hi) */
-  for (;;) {
-    const int x = e0 + lane;
-    const bool start = (x < hi) && (0 == x || stack[3 * x + 2] != stack[3 * (x - 1) + 2]);
-    const unsigned long long bal = __ballot(start);
-    if (0 != bal) {
-      e0 += __ffsll((long long)bal) - 1;
-      break;
+  /* run boundaries found 64 entries at a time (one lane each, then a ballot): from the first run that starts in
+     [lo, hi) to the end of the last one */
+  const auto first_start = [&](int x0, int x1) {
+    for (; x0 < x1; x0 += 64) {
+      const int x = x0 + lane;
+      const unsigned long long bal = __ballot(x < x1 && (0 == x || stack[3 * x + 2] != stack[3 * (x - 1) + 2]));
+      if (0 != bal) return x0 + __ffsll((long long)bal) - 1;
     }
-    e0 += 64;
-    if (e0 >= hi) {
-      e0 = hi;
-      break;
-    }
-  }
-  while (e0 < hi) { /* the run of entries e0 .. e1 - 1 (one C offset), walked to its end */
-    const int cofs = stack[3 * e0 + 2];
-    int e1 = e0 + 1;
-    for (;;) {
-      const int x = e1 + lane;
-      const unsigned long long bal = __ballot(x >= S || stack[3 * x + 2] != cofs);
-      if (0 != bal) {
-        e1 += __ffsll((long long)bal) - 1;
-        break;
-      }
-      e1 += 64;
-    }
-    const long cbase = (long)cofs - 1;
-    double creg[16];
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int j = 32 * wj + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-      creg[r] = (i < m && j < n) ? (double)c[cbase + i + (long)j * m] : 0.0;
-    }
-    /* block indices of entry e, -1 when its offsets are not block starts inside the pools */
-    auto blocks = [&](int e, int& ab, int& bb) {
-      const int ao = __builtin_amdgcn_readfirstlane(stack[3 * e] - 1), bo = __builtin_amdgcn_readfirstlane(stack[3 * e + 1] - 1);
-      const unsigned int aq = (unsigned int)ao / mk, bq = (unsigned int)bo / kn;
-      ab = (0 <= ao && (unsigned int)ao == aq * mk && aq < (unsigned int)na) ? (int)aq : -1;
-      bb = (0 <= bo && (unsigned int)bo == bq * kn && bq < (unsigned int)nb) ? (int)bq : -1;
-    };
-    /* no branch around the DMA (an entry without valid blocks loads block 0, unused), so the compiler
-       can count the outstanding loads on every path */
-    auto dma = [&](int8_t* buf, int ab, int bb) {
-      ab = (0 <= ab ? ab : 0);
-      bb = (0 <= bb ? bb : 0);
+    return x1;
+  };
+  const int e0 = __builtin_amdgcn_readfirstlane(first_start(lo, hi));
+  if (e0 >= hi) return;
+  const int e1 = __builtin_amdgcn_readfirstlane(first_start(hi, S));
+  /* the DMA of this wavefront: planes of one operand, 16 of their rows */
+  const int dr = 16 * (wave & 3), drow = dr + (lane >> 2), dchunk = (lane & 3) ^ ((lane >> 4) & 3);
+  const bool dma_any = (dr < (0 == late ? m : n));
+  const int8_t* const dsrc = (0 == late ? pa : pb) + drow * SB + 16 * dchunk;
+  const int* const dex = (0 == late ? ea : eb) + lane;
+  /* the tile: columns i (A rows) 32 wi + 16 x + lane % 16, rows j (B columns) 16 wj + 4 (lane / 16) + r per register */
+  const bool active = (32 * wi < m && 16 * wj < n);
+  const int frow = lane & 15, fpos = 16 * ((lane >> 4) ^ ((frow >> 2) & 3));
+  const int i0 = 32 * wi + frow, j0 = 16 * wj + 4 * (lane >> 4);
+  double creg[2][4];
+  i4_t acc[2 * NS - 1][2];
+  int exi[2];
+  i4_t exj;
+  /* entries base .. base + 63, one per lane: the blocks of A and B (-1 when an offset is not a block start inside the
+     pool) and the C offset; first, last: bit l set when entry base + l begins or ends a run */
+  int base, wa, wb, wc;
+  unsigned long long firsts, lasts;
+  const auto block_of = [](int ofs, unsigned int sz, int cnt) {
+    const unsigned int q = (unsigned int)ofs / sz;
+    return (0 <= ofs && (unsigned int)ofs == q * sz && q < (unsigned int)cnt) ? (int)q : -1;
+  };
+  const auto window = [&](int x0) {
+    const int x = min(x0 + lane, S - 1);
+    const int ra = stack[3 * x], rb = stack[3 * x + 1], rc = stack[3 * x + 2];
+    const int before = stack[3 * max(x - 1, 0) + 2], after = stack[3 * min(x + 1, S - 1) + 2];
+    wa = block_of(ra - 1, mk, na);
+    wb = block_of(rb - 1, kn, nb);
+    wc = rc;
+    firsts = __ballot(x == e0 || before != rc);
+    lasts = __ballot(x + 1 >= e1 || after != rc);
+    base = x0;
+  };
+  /* entry e into buffer e % 2; an entry without valid blocks loads block 0, unused */
+  const auto dma = [&](int8_t* buf, int e) {
+    const int blk = max(__builtin_amdgcn_readlane(0 == late ? wa : wb, e - base), 0);
+    if (dma_any) {
 #pragma unroll
       for (int pl = 0; pl < NS; ++pl) {
-        ozs_dma16(pa + ((long)ab * NS + pl) * SPL + drow * SB + 16 * dchunk, buf + pl * SPL + wave * 1024);
-        ozs_dma16(pb + ((long)bb * NS + pl) * SPL + drow * SB + 16 * dchunk, buf + (NS + pl) * SPL + wave * 1024);
+        ozs_dma16(dsrc + ((long)blk * NS + pl) * SPL, buf + (late * NS + pl) * SPL + (wave & 3) * 1024);
       }
-      /* the 64 row exponents of the A block and column exponents of the B block, one copy per wavefront */
-      ozs_dma4(ea + (long)ab * SB + lane, buf + 2 * NS * SPL + wave * SEX);
-      ozs_dma4(eb + (long)bb * SB + lane, buf + 2 * NS * SPL + wave * SEX + SB * 4);
-    };
-    int ab, bb;
-    blocks(e0, ab, bb);
-    dma(lds0, ab, bb);
-    for (int e = e0; e < e1; ++e) {
-      int8_t* const cur = (0 == ((e - e0) & 1) ? lds0 : lds1);
-      int8_t* const nxt = (0 == ((e - e0) & 1) ? lds1 : lds0);
-      const int ac = ab, bc = bb;
-      __builtin_amdgcn_s_waitcnt(0); /* own DMA of entry e, own reads of entry e - 1 */
-      __syncthreads();              /* every wave's DMA of e has landed, every wave is done with e - 1 */
-      /* entry e + 1 into the other buffer; the last entry of the run loads its own blocks again (unused).
-         The loop has no other global loads, so nothing waits for this DMA before the next entry */
-      blocks(e + 1 < e1 ? e + 1 : e, ab, bb);
-      dma(nxt, ab, bb);
-      if (0 <= ac && 0 <= bc) {
-        /* exponents from LDS: row i of A (SNONE past m), columns 32 wj + 8 q + 4 (lane / 32) + 0..3 of B */
-        const int* const lex = (const int*)(cur + 2 * NS * SPL + wave * SEX);
-        const int exi = lex[i];
-        i4_t exj4[4];
+    }
+    if (0 == (wave & 3)) ozs_dma4(dex + (long)blk * SB, buf + 2 * NS * SPL + late * SB * 4);
+  };
+  bool valid = false, last = false; /* of the entry whose level sums are in acc */
+  T* cblk = c;
+  const auto recombine = [&]() {
+    if (valid) {
 #pragma unroll
-        for (int q = 0; q < 4; ++q) exj4[q] = *(const i4_t*)(lex + SB + 32 * wj + 8 * q + 4 * (lane >> 5));
-        i4_t fa[NS][2], fb[NS][2];
+      for (int x = 0; x < 2; ++x) {
 #pragma unroll
-        for (int pl = 0; pl < NS; ++pl) {
-          const int8_t* const la = cur + pl * SPL + (32 * wi + frow) * SB;
-          const int8_t* const lb = cur + (NS + pl) * SPL + (32 * wj + frow) * SB;
-          fa[pl][0] = *(const i4_t*)(la + 16 * fpos0);
-          fa[pl][1] = *(const i4_t*)(la + 16 * fpos1);
-          fb[pl][0] = *(const i4_t*)(lb + 16 * fpos0);
-          fb[pl][1] = *(const i4_t*)(lb + 16 * fpos1);
-        }
-        i16_t acc[2 * NS - 1];
-#pragma unroll
-        for (int L = 0; L < 2 * NS - 1; ++L) acc[L] = i16_t{0};
-#pragma unroll
-        for (int p = 0; p < NS; ++p) {
-#pragma unroll
-          for (int q = 0; q < NS; ++q) {
-            if (p + q <= cutoff) {
-              acc[p + q] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fb[q][0], fa[p][0], acc[p + q], 0, 0, 0);
-              acc[p + q] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fb[q][1], fa[p][1], acc[p + q], 0, 0, 0);
-            }
-          }
-        }
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int j = 32 * wj + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
+        for (int r = 0; r < 4; ++r) {
           double cd = 0.0;
 #pragma unroll
           for (int L = 2 * NS - 2; 0 <= L; --L) {
-            if (L <= cutoff) cd = fma(ldexp(1.0, -7 * (L + 2)), (double)acc[L][r], cd);
+            if (L <= cutoff) cd = fma(ldexp(1.0, -7 * (L + 2)), (double)acc[L][x][r], cd);
           }
-          const int exj = (j < n ? exj4[r >> 2][r & 3] : SNONE);
-          const double v = (SNONE != exi && SNONE != exj) ? ldexp(cd, exi + exj) : 0.0;
-          creg[r] = (double)(T)(creg[r] + v);
+          const double v = (SNONE != exi[x] && SNONE != exj[r]) ? ldexp(cd, exi[x] + exj[r]) : 0.0;
+          creg[x][r] = (double)(T)(creg[x][r] + v);
         }
       }
     }
+    if (last && active) {
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int j = 32 * wj + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-      if (i < m && j < n) c[cbase + i + (long)j * m] = (T)creg[r];
+      for (int x = 0; x < 2; ++x) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          if (i0 + 16 * x < m && j0 + r < n) cblk[i0 + 16 * x + (long)(j0 + r) * m] = (T)creg[x][r];
+        }
+      }
     }
-    __builtin_amdgcn_s_waitcnt(0);
-    __syncthreads(); /* the buffers of this run are free before the next run's first DMA */
-    e0 = e1;
+  };
+  window(e0);
+  dma(lds0, e0);
+  for (int e = e0; e < e1; ++e) {
+    int8_t* const cur = (0 == ((e - e0) & 1) ? lds0 : lds1);
+    int8_t* const nxt = (0 == ((e - e0) & 1) ? lds1 : lds0);
+    __builtin_amdgcn_s_waitcnt(0); /* own DMA of entry e, own reads of entry e - 1 */
+    __syncthreads();              /* every wave's DMA of e has landed, every wave is done with e - 1 */
+    if (e + 1 - base >= 64) window(e);
+    dma(nxt, min(e + 1, e1 - 1)); /* the last entry loads itself again, unused */
+    if (0 != late && e != e0) recombine();
+    {
+      const int l = e - base;
+      const bool first = (0 != ((firsts >> l) & 1));
+      last = (0 != ((lasts >> l) & 1));
+      cblk = c + ((long)__builtin_amdgcn_readlane(wc, l) - 1);
+      valid = active && 0 <= __builtin_amdgcn_readlane(wa, l) && 0 <= __builtin_amdgcn_readlane(wb, l);
+      if (first && active) {
+#pragma unroll
+        for (int x = 0; x < 2; ++x) {
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            creg[x][r] = (i0 + 16 * x < m && j0 + r < n) ? (double)cblk[i0 + 16 * x + (long)(j0 + r) * m] : 0.0;
+          }
+        }
+        __builtin_amdgcn_s_waitcnt(0xF70); /* once per run, so that no recombination waits for the DMA of the next entry */
+      }
+    }
+    if (valid) {
+      /* exponents from LDS: rows of A, columns of B */
+      const int* const lex = (const int*)(cur + 2 * NS * SPL);
+      exi[0] = lex[i0];
+      exi[1] = lex[i0 + 16];
+      exj = *(const i4_t*)(lex + SB + j0);
+      i4_t fb[NS];
+#pragma unroll
+      for (int q = 0; q < NS; ++q) fb[q] = *(const i4_t*)(cur + (NS + q) * SPL + (16 * wj + frow) * SB + fpos);
+#pragma unroll
+      for (int L = 0; L < 2 * NS - 1; ++L) acc[L][0] = acc[L][1] = i4_t{0};
+#pragma unroll
+      for (int p = 0; p < NS; ++p) {
+        i4_t fa[2];
+#pragma unroll
+        for (int x = 0; x < 2; ++x) fa[x] = *(const i4_t*)(cur + p * SPL + (32 * wi + 16 * x + frow) * SB + fpos);
+#pragma unroll
+        for (int q = 0; q < NS; ++q) {
+          if (p + q <= cutoff) {
+#pragma unroll
+            for (int x = 0; x < 2; ++x) acc[p + q][x] = __builtin_amdgcn_mfma_i32_16x16x64_i8(fb[q], fa[x], acc[p + q][x], 0, 0, 0);
+          }
+        }
+      }
+    }
+    if (0 == late) recombine();
   }
+  if (0 != late) recombine();
+  __builtin_amdgcn_s_waitcnt(0); /* no DMA in flight at the end */
 }
 
 /* NS slices with the level cutoff compiled in for the triangle (NS - 1) and all pairs (2 NS - 2) */
@@ -263,13 +290,13 @@ template <typename T, int NS>
 void ozs_launch_ns(dim3 grid, hipStream_t st, const int* stack, int S, const int* info, const int8_t* pa,
   const int* ea, const int8_t* pb, const int* eb, int cutoff, int m, int n, int k, int na, int nb, T* c) {
   if (NS - 1 == cutoff) {
-    ozs_stack<T, NS, NS - 1><<<grid, 256, 0, st>>>(stack, S, info, pa, ea, pb, eb, cutoff, m, n, k, na, nb, c);
+    ozs_stack<T, NS, NS - 1><<<grid, 512, 0, st>>>(stack, S, info, pa, ea, pb, eb, cutoff, m, n, k, na, nb, c);
   }
   else if (2 * (NS - 1) == cutoff) {
-    ozs_stack<T, NS, 2 * (NS - 1)><<<grid, 256, 0, st>>>(stack, S, info, pa, ea, pb, eb, cutoff, m, n, k, na, nb, c);
+    ozs_stack<T, NS, 2 * (NS - 1)><<<grid, 512, 0, st>>>(stack, S, info, pa, ea, pb, eb, cutoff, m, n, k, na, nb, c);
   }
   else {
-    ozs_stack<T, NS, -1><<<grid, 256, 0, st>>>(stack, S, info, pa, ea, pb, eb, cutoff, m, n, k, na, nb, c);
+    ozs_stack<T, NS, -1><<<grid, 512, 0, st>>>(stack, S, info, pa, ea, pb, eb, cutoff, m, n, k, na, nb, c);
   }
 }
 
@@ -299,14 +326,16 @@ int ozs_launch_stack(int s, dim3 grid, hipStream_t st, const int* stack, int S, 
  */
 extern "C" int lxs_ozs_process(int dtype, const int* stack, int S, int m, int n, int k, const void* a, int na,
   const void* b, int nb, void* c, int s, int cutoff, signed char* planes_a, int* ea, signed char* planes_b, int* eb,
-  int* info, void* hip_stream) {
+  int* info, int ncus, void* hip_stream) {
   const hipStream_t st = (hipStream_t)hip_stream;
   if (1 > m || SB < m || 1 > n || SB < n || 1 > k || SB < k || 1 > s || 8 < s || 0 > cutoff || 2 * (s - 1) < cutoff) {
     return LXS_ELIMIT;
   }
   if (0 >= S) return 0;
   if (0 >= na || 0 >= nb) return LXS_ELIMIT;
-  const dim3 grid((unsigned int)(S < 1024 ? S : 1024));
+  /* as many work-groups as are resident (LDS: one per CU above 4 slices, else two), each with one share of the stack */
+  const int wgs = (4 < s ? 1 : 2) * (0 < ncus ? ncus : 256);
+  const dim3 grid((unsigned int)(S < wgs ? S : wgs));
   const unsigned int cgrid = (unsigned int)((S + 255) / 256 < 256 ? (S + 255) / 256 : 256);
   int result = 0;
   if (3 == dtype) { /* A rows: (r, kk) at r + kk m; B columns: (j, kk) at j + kk n */
