@@ -311,10 +311,11 @@ def batched(lx, stream, steps, warmup):
     t1 = time.perf_counter()
     prof = lx.profile_get("batch")
     lx.profile_enable(False)
-    # every schedule kind replayed the same way: the persistent kernel (default and tuned chunking), the
+    # every schedule kind replayed the same way: the default (chosen by the work), the persistent kernel, the
     # per-stack launches in order, and the per-stack launches on concurrent lanes
     schedules = {}
-    for name, params in (("persistent_default", lx.BatchParams(0, 0, 0)), ("per_stack_in_order", lx.BatchParams(0, 0, 1)),
+    for name, params in (("default", lx.BatchParams(0, 0, 0)), ("persistent", lx.BatchParams(0, 8, 0)),
+                         ("per_stack_in_order", lx.BatchParams(0, 0, 1)),
                          ("per_stack_lanes", lx.BatchParams(0, 0, 2))):
         bb = lx.Batch(lx.REAL_8, items, params)
         for _ in range(warmup):

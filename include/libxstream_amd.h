@@ -111,8 +111,8 @@ LIBXSTREAM_API int libsmm_acc_read_ref_params(const char* line, int with_device,
 
 /**
  * Batched stack multiply (no counterpart in the reference): stacks of different (m, n, k) and
- * lengths, each with the semantics of libsmm_acc_process, in one persistent kernel launch; the
- * launch can be captured once into a hipGraph and replayed. m and n must lie in 1..64 (any k);
+ * lengths, each with the semantics of libsmm_acc_process, in one launch per stack or one persistent
+ * kernel launch for all; the launches can be captured once into a hipGraph and replayed. m and n must lie in 1..64 (any k);
  * all stacks share the batch's datatype. C-runs are flushed with atomic adds, so stacks may share
  * C pools and need not be sorted.
  */
@@ -125,11 +125,13 @@ typedef struct libsmm_acc_batch_stack_t {
 } libsmm_acc_batch_stack_t;
 typedef struct libsmm_acc_batch_t libsmm_acc_batch_t;
 /** the batch's schedule: entries per chunk sized to move about chunk_elements operand elements (8..512
- *  entries), blocks_per_cu persistent work-groups per CU; 0 selects the default (32 entries of 23x23x23, 8) */
+ *  entries), blocks_per_cu persistent work-groups per CU; 0 selects the default (32 entries of 23x23x23, 8). With every
+ *  field 0 (or no parameters) the batch chooses by its work: one launch per stack, in order on the stream (replay: or
+ *  in lanes as for per_stack 2), or the persistent kernel for many short stacks */
 typedef struct libsmm_acc_batch_params_t {
   int chunk_elements, blocks_per_cu;
-  int per_stack; /* 1: one libsmm_acc_process launch per stack (its own configuration) instead of the
-                    persistent kernel; libsmm_acc_batch_replay captures all of them in one graph;
+  int per_stack; /* 1: one libsmm_acc_process launch per stack (its own configuration);
+                    libsmm_acc_batch_replay captures all of them in one graph;
                     2: the same launches spread over 4 side streams that fork from the caller's stream and
                     join it again (independent branches of one graph), so that short stacks overlap */
 } libsmm_acc_batch_params_t;
@@ -143,7 +145,7 @@ LIBXSTREAM_API int libsmm_acc_batch_create_ex(libsmm_acc_data_t datatype, const 
  *  to scratch (the caller's C is not touched); blocks until done (allocates; not under capture) */
 LIBXSTREAM_API int libsmm_acc_batch_tune(libsmm_acc_data_t datatype, const libsmm_acc_batch_stack_t* stacks,
   int nstacks, libsmm_acc_batch_params_t* best, double* best_ms);
-/** enqueue the batch as one kernel launch on stream */
+/** enqueue the batch on stream */
 LIBXSTREAM_API int libsmm_acc_batch_process(libsmm_acc_batch_t* batch, void* stream);
 /** replay the batch from a hipGraph (captured on the first call) on stream */
 LIBXSTREAM_API int libsmm_acc_batch_replay(libsmm_acc_batch_t* batch, void* stream);

@@ -1,9 +1,9 @@
 /*
- * Batched stack multiply: stacks of different (m, n, k) and lengths in one persistent kernel
- * launch, optionally replayed from a captured hipGraph. Each stack has the semantics of
+ * Batched stack multiply: stacks of different (m, n, k) and lengths, one launch per stack or one persistent kernel
+ * for all, optionally replayed from a captured hipGraph. Each stack has the semantics of
  * libsmm_acc_process (samples/smm/acc_libsmm.h:45-47); the batch has no reference counterpart.
  *
- * Plan (built once on the host): every stack is cut into chunks of run-aligned entries, sized so
+ * Plan of the persistent kernel (built once on the host): every stack is cut into chunks of run-aligned entries, sized so
  * that a chunk moves about as many operand elements as 32 entries of 23x23x23; blocks that need
  * more than 4 output tiles of 16x16 get one work-group task per chunk (its 4 wavefronts split the
  * tiles), smaller blocks are packed 4 chunks per task (one per wavefront). Expensive tasks come
@@ -23,9 +23,11 @@ struct libsmm_acc_batch_t {
   hipGraph_t graph;
   hipGraphExec_t exec;
   double flops, bytes;
-  int per_stack;                 /* launch mode, libsmm_acc_batch_params_t */
-  libsmm_acc_batch_stack_t* host; /* the stacks as given (per-stack mode) */
-  /* per_stack 2: the launches spread over LXS_BATCH_LANES side streams that fork from the caller's stream
+  /* launch modes (libsmm_acc_batch_params_t.per_stack) of libsmm_acc_batch_process and _replay: as given, or chosen by
+     lxs_batch_modes (chosen 1) */
+  int eager, graphed, chosen;
+  libsmm_acc_batch_stack_t* host; /* the stacks as given (per-stack modes) */
+  /* mode 2: the launches spread over LXS_BATCH_LANES side streams that fork from the caller's stream
      and join it again (one graph with independent branches under replay); lane[i]: stack i's stream */
   hipStream_t side[LXS_BATCH_LANES];
   hipEvent_t fork, join[LXS_BATCH_LANES];
@@ -61,6 +63,39 @@ static void lxs_batch_release(libsmm_acc_batch_t* b) {
   free(b->lane);
   free(b->host);
   free(b);
+}
+
+/*
+ * The default schedule, by estimates of its time (us) from the number of stacks c, their operand bytes W and the longest
+ * stack: one launch per stack in order 12 + c (4.2, 5.5 from 50 and 6.5 from 200 entries on) + W / 3.5 TB/s; in lanes
+ * (replay only:
+ * libsmm_acc_batch_process may run on several streams at once, the lanes' streams and events are one set) 75 +
+ * the larger of 5 + 3.2 c and W / 4.3 TB/s; the persistent kernel 40 + its longest chain (FP64 0.9, FP32 0.72 per entry of
+ * 40 k, at most 260) + W / 1.8 TB/s. Measured by replay, FP64, stacks of mixed shapes up to 64x64x64, in order / lanes / persistent:
+ * 8 stacks of 10 entries 38 / 135 / 59, 24 of 100 142 / 157 / 184, 24 of 3000 312 / 160 / 534, 100 of 10 393 / 396 / 66, 100
+ * of 100 600 / 394 / 261, 100 of 1000 833 / 405 / 795, 24 of 1 to 100 thousand 1230 / 1058 / 3620: each entry of the
+ * persistent kernel is one wavefront's, while the stack's own kernel splits the k of a whole run over several.
+ */
+static void lxs_batch_modes(libsmm_acc_batch_t* b, const libsmm_acc_batch_stack_t* stacks, int nstacks) {
+  const double ts = (dbcsr_type_real_8 == b->dtype ? 8 : 4);
+  double bytes = 0, order = 12, lanes, persistent, chain = 0;
+  int i, count = 0;
+  for (i = 0; i < nstacks; ++i) {
+    const libsmm_acc_batch_stack_t* const s = stacks + i;
+    const double steps = (8 == ts ? 0.9 : 0.72) * s->stack_size * s->k / 40.0;
+    if (0 == s->stack_size) continue;
+    if (0 == lxs_smm_enqueue_ok(b->dtype, s->stack_size, s->m, s->n, s->k)) return; /* persistent */
+    ++count;
+    bytes += ts * s->stack_size * ((double)s->m * s->k + (double)s->k * s->n);
+    order += (200 <= s->stack_size ? 6.5 : (50 <= s->stack_size ? 5.5 : 4.2));
+    if (chain < steps) chain = steps;
+  }
+  order += bytes / 3.5e6;
+  lanes = 75 + (5 + 3.2 * count > bytes / 4.3e6 ? 5 + 3.2 * count : bytes / 4.3e6);
+  persistent = 40 + (chain < 260 ? chain : 260) + bytes / 1.8e6;
+  b->eager = (order < persistent ? 1 : 0);
+  b->graphed = (lanes < order && lanes < persistent ? 2 : b->eager);
+  b->chosen = 1;
 }
 
 LIBXSTREAM_API int libsmm_acc_batch_create_ex(libsmm_acc_data_t datatype, const libsmm_acc_batch_stack_t* stacks,
@@ -160,18 +195,19 @@ LIBXSTREAM_API int libsmm_acc_batch_create_ex(libsmm_acc_data_t datatype, const 
     b->dtype = (int)datatype;
     b->nstacks = nstacks;
     b->ntasks = ntasks;
-    b->per_stack = (NULL != params && 0 < params->per_stack ? (2 <= params->per_stack ? 2 : 1) : 0);
+    if (NULL != params && 0 < params->per_stack) b->eager = b->graphed = (2 <= params->per_stack ? 2 : 1);
+    else if (NULL == params || (0 >= params->chunk_elements && 0 >= params->blocks_per_cu)) lxs_batch_modes(b, stacks, nstacks);
     b->host = (libsmm_acc_batch_stack_t*)malloc(sizeof(*stacks) * (size_t)nstacks);
     if (NULL == b->host) result = lxs_error(EXIT_FAILURE, "libsmm_acc_batch_create: out of memory");
     else memcpy(b->host, stacks, sizeof(*stacks) * (size_t)nstacks);
-    for (i = 0; i < nstacks && 0 != b->per_stack && EXIT_SUCCESS == result; ++i) {
+    for (i = 0; i < nstacks && 0 == b->chosen && 0 != b->eager && EXIT_SUCCESS == result; ++i) {
       /* resolve (and cache) every shape's configuration now, so that no lookup or prediction runs
          while libsmm_acc_batch_replay captures the launches */
       libsmm_acc_smm_config_t cfg;
       result = libsmm_acc_config_get(datatype, stacks[i].m, stacks[i].n, stacks[i].k, &cfg, NULL);
     }
   }
-  if (EXIT_SUCCESS == result && 2 == b->per_stack) { /* lanes: stacks by flops, each to the least loaded */
+  if (EXIT_SUCCESS == result && (2 == b->eager || 2 == b->graphed)) { /* lanes: stacks by flops, each to the least loaded */
     double load[LXS_BATCH_LANES] = {0};
     int* const order = (int*)malloc(sizeof(int) * (size_t)nstacks);
     b->lane = (int*)malloc(sizeof(int) * (size_t)nstacks);
@@ -231,16 +267,17 @@ LIBXSTREAM_API int libsmm_acc_batch_create_ex(libsmm_acc_data_t datatype, const 
   return result;
 }
 
-static int lxs_batch_enqueue(libsmm_acc_batch_t* b, hipStream_t hs) {
+static int lxs_batch_enqueue(libsmm_acc_batch_t* b, int mode, hipStream_t hs) {
+  const int shared = (0 != b->chosen || 2 == mode); /* stacks may share C pools */
   int i, code = 0;
-  if (0 == b->per_stack) {
+  if (0 == mode) {
     code = lxs_batch_launch(b->dtype, b->desc, b->tasks, b->ntasks, b->nblocks, (void*)hs);
   }
-  else if (1 == b->per_stack) {
+  else if (1 == mode) {
     for (i = 0; i < b->nstacks && 0 == code; ++i) {
       const libsmm_acc_batch_stack_t* const s = b->host + i;
       code = lxs_smm_enqueue(b->dtype, s->dev_param_stack, s->stack_size, s->dev_a_data, s->dev_b_data, s->dev_c_data,
-        s->m, s->n, s->k, (void*)hs);
+        s->m, s->n, s->k, shared, (void*)hs);
     }
   }
   else { /* fork to the side streams, one launch per stack on its lane, join (the C flush is atomic, so
@@ -251,7 +288,7 @@ static int lxs_batch_enqueue(libsmm_acc_batch_t* b, hipStream_t hs) {
     for (i = 0; i < b->nstacks && 0 == code; ++i) {
       const libsmm_acc_batch_stack_t* const s = b->host + i;
       code = lxs_smm_enqueue(b->dtype, s->dev_param_stack, s->stack_size, s->dev_a_data, s->dev_b_data, s->dev_c_data,
-        s->m, s->n, s->k, (void*)b->side[b->lane[i]]);
+        s->m, s->n, s->k, shared, (void*)b->side[b->lane[i]]);
     }
     for (l = 0; l < LXS_BATCH_LANES && 0 == code; ++l) {
       code = (int)hipEventRecord(b->join[l], b->side[l]);
@@ -269,7 +306,7 @@ LIBXSTREAM_API int libsmm_acc_batch_process(libsmm_acc_batch_t* batch, void* str
   result = lxs_ensure_device();
   if (EXIT_SUCCESS != result) return result;
   token = lxs_profile_begin(hs);
-  result = lxs_batch_enqueue(batch, hs);
+  result = lxs_batch_enqueue(batch, batch->eager, hs);
   lxs_profile_end(token, hs, "batch", batch->flops, batch->bytes);
   return result;
 }
@@ -288,7 +325,7 @@ LIBXSTREAM_API int libsmm_acc_batch_replay(libsmm_acc_batch_t* batch, void* stre
       result = lxs_hip(hipStreamBeginCapture(batch->capture, hipStreamCaptureModeThreadLocal), "hipStreamBeginCapture");
     }
     if (EXIT_SUCCESS == result) {
-      const int launched = lxs_batch_enqueue(batch, batch->capture);
+      const int launched = lxs_batch_enqueue(batch, batch->graphed, batch->capture);
       const int ended = lxs_hip(hipStreamEndCapture(batch->capture, &batch->graph), "hipStreamEndCapture");
       result = (EXIT_SUCCESS != launched ? launched : ended);
     }
@@ -316,7 +353,7 @@ LIBXSTREAM_API int libsmm_acc_batch_destroy(libsmm_acc_batch_t* batch) {
   if (NULL != batch) {
     if (NULL != batch->exec) result = lxs_hip(hipGraphExecDestroy(batch->exec), "hipGraphExecDestroy");
     if (NULL != batch->graph) (void)hipGraphDestroy(batch->graph);
-    if (2 == batch->per_stack) (void)hipDeviceSynchronize(); /* side streams may still run the last process */
+    if (2 == batch->eager) (void)hipDeviceSynchronize(); /* side streams may still run the last process */
     lxs_batch_release(batch);
   }
   return result;
@@ -386,9 +423,9 @@ LIBXSTREAM_API int libsmm_acc_batch_tune(libsmm_acc_data_t datatype, const libsm
     }
     else p.per_stack = 1 + (i - last); /* one launch per stack with its own configuration, in order or in lanes */
     result = libsmm_acc_batch_create_ex(datatype, trial, nstacks, &p, &b);
-    if (EXIT_SUCCESS == result) result = lxs_batch_enqueue(b, hs); /* warm-up */
+    if (EXIT_SUCCESS == result) result = lxs_batch_enqueue(b, b->eager, hs); /* warm-up */
     if (EXIT_SUCCESS == result) result = lxs_hip(hipEventRecord(e0, hs), "hipEventRecord");
-    for (r = 0; r < 3 && EXIT_SUCCESS == result; ++r) result = lxs_batch_enqueue(b, hs);
+    for (r = 0; r < 3 && EXIT_SUCCESS == result; ++r) result = lxs_batch_enqueue(b, b->eager, hs);
     if (EXIT_SUCCESS == result) result = lxs_hip(hipEventRecord(e1, hs), "hipEventRecord");
     if (EXIT_SUCCESS == result) result = lxs_hip(hipEventSynchronize(e1), "hipEventSynchronize");
     if (EXIT_SUCCESS == result) result = lxs_hip(hipEventElapsedTime(&ms, e0, e1), "hipEventElapsedTime");

@@ -74,8 +74,10 @@ void lxs_smm_finalize(void);
    entries keep runs of up to 64 entries whole (unless LIBXSTREAM_SMM_SPLIT_MIN says otherwise) */
 #define LXS_SMM_SPLIT_FILL 16384
 int lxs_smm_tsplit(int bs, int split, int stack_size);
-/* one stack with its resolved configuration on a HIP stream, no profile records (hipError_t or LXS_E*) */
+/* one stack with its resolved configuration on a HIP stream, no profile records (hipError_t or LXS_E*); shared:
+   always an atomic flush of C */
 int lxs_smm_enqueue(int datatype, const int* dev_param_stack, int stack_size, const void* a, const void* b, void* c,
-  int m, int n, int k, void* hip_stream);
+  int m, int n, int k, int shared, void* hip_stream);
+int lxs_smm_enqueue_ok(int datatype, int stack_size, int m, int n, int k);
 
 #endif /*LXS_INTERNAL_H*/

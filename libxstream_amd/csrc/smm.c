@@ -887,15 +887,24 @@ static int lxs_smm_run(const libsmm_acc_smm_config_t* config, const int* dev_par
 }
 
 /* one stack with its resolved configuration on a HIP stream, without profile records (the batch's
-   per-stack mode, also under graph capture); the result is a hipError_t or an LXS_E* code */
+   per-stack mode, also under graph capture); shared: other launches may update the same C blocks meanwhile, so
+   the flush is atomic whatever was promised for one stack; the result is a hipError_t or an LXS_E* code */
 int lxs_smm_enqueue(int datatype, const int* dev_param_stack, int stack_size, const void* a, const void* b, void* c,
-  int m, int n, int k, void* hip_stream) {
+  int m, int n, int k, int shared, void* hip_stream) {
   libsmm_acc_smm_config_t config;
   lxs_smm_args_t args;
   if (0 >= stack_size) return 0;
   lxs_smm_select(datatype, m, n, k, stack_size, &config);
-  lxs_smm_fill(&args, &config, dev_param_stack, stack_size, datatype, a, b, c, m, n, k, 0, lxs_cfg.grouped);
+  lxs_smm_fill(&args, &config, dev_param_stack, stack_size, datatype, a, b, c, m, n, k, 0,
+    0 == shared ? lxs_cfg.grouped : 0);
   return lxs_smm_launch(&args, hip_stream);
+}
+
+/* whether lxs_smm_enqueue has a kernel for the stack (resolves, and caches where that applies, its configuration) */
+int lxs_smm_enqueue_ok(int datatype, int stack_size, int m, int n, int k) {
+  libsmm_acc_smm_config_t config;
+  lxs_smm_select(datatype, m, n, k, stack_size, &config);
+  return EXIT_SUCCESS == libsmm_acc_config_valid((libsmm_acc_data_t)datatype, m, n, k, &config);
 }
 
 LIBXSTREAM_API int libsmm_acc_process_config(const libsmm_acc_smm_config_t* config, const int* dev_param_stack,
