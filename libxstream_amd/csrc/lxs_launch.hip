@@ -94,7 +94,7 @@ static size_t mfma_lds(const mfma_entry_t* e, int dtype) {
   return (1 < e->ep || 0 != e->b4 ? (size_t)e->ep * e->ti * e->tj * (2 == e->b4 ? 16 : (1 == e->b4 ? 64 : 256)) * (3 == dtype ? 8 : 4) : 0);
 }
 /* a runtime-shape kernel covers (m, n): 16x16 tiles up to 16 ti x 16 tj, with at least two rows and columns
-   where the kernel loads element pairs (an even number of tiles in both dimensions); 4x4 blocks with exactly
+   for an even number of tiles in both dimensions; 4x4 blocks with exactly
    the ti = ceil(m / 8), tj = ceil(n / 8) the shape needs (each lane loads ti consecutive rows, tj columns), or
    ti = ceil(m / 4), tj = ceil(n / 4) when the blocks split k */
 static int mfma_fits(const mfma_entry_t* e, int m, int n) {
@@ -103,6 +103,8 @@ static int mfma_fits(const mfma_entry_t* e, int m, int n) {
     return m <= r * e->ti && m > r * (e->ti - 1) && n <= r * e->tj && n > r * (e->tj - 1);
   }
   if (0 == e->ti % 2 && 0 == e->tj % 2 && (2 > m || 2 > n)) return 0;
+  /* 4 wavefronts above 8 tiles: for exactly that grid, smaller blocks have their own */
+  if (4 == e->ep && 8 < e->ti * e->tj && (m <= 16 * (e->ti - 1) || n <= 16 * (e->tj - 1))) return 0;
   return m <= 16 * e->ti && n <= 16 * e->tj;
 }
 
@@ -119,6 +121,11 @@ static const mfma_entry_t* mfma_find(int dtype, int variant, int m, int n, int k
     }
     if (e->m == m && e->n == n && e->k == k) return e;
     if (0 == e->m && NULL == generic && mfma_fits(e, m, n)) generic = e;
+  }
+  if (NULL != generic && 0 == generic->b4 && 1 < generic->ep) {
+    /* fewer rows or columns than the tiles of a group load at once: the grid without the idle tiles */
+    const int v = (3 == dtype ? 2 : 4), gi = (generic->ti < v ? generic->ti : v), gj = (generic->tj < v ? generic->tj : v);
+    if (m < gi || n < gj) return mfma_find(dtype, variant, m, n, k, (m + 15) / 16, (n + 15) / 16, nt, kt);
   }
   return generic;
 }

@@ -101,15 +101,54 @@ __device__ __forceinline__ typename pair_of<T>::type gload2(const T* p) {
   return *(const __attribute__((address_space(1))) typename pair_of<T>::type*)p;
 }
 
-/* Paired tiles: output tiles 2p and 2p+1 of one dimension interleave the 32 rows (or columns) from 32p on,
-   so that one two-element load per lane feeds both tiles. Lane l of the pair loads the elements at
-   s = min(32p + 2l, extent - 2) and s + 1 (clamped so both stay inside the extent) for tiles 2p and 2p+1.
-   Output row l of tile 2p+q is then element s + q; it is written by exactly one lane: an unclamped pair,
-   or for an odd extent the lane whose pair would start at extent - 1 (tile 2p+1 holds that last element). */
-__device__ __forceinline__ int pair_start(int p, int l, int extent) { return min(32 * p + 2 * l, extent - 2); }
-__device__ __forceinline__ bool pair_owner(int p, int q, int l, int extent) {
-  const int base = 32 * p + 2 * l;
-  return base <= extent - 2 || (1 == q && base == extent - 1);
+/* Grouped tiles: up to V = 16 bytes / element size tiles of one dimension form a group whose rows (or columns)
+   are interleaved, so that one load of up to 16 bytes per lane feeds all of them. Lane l of the group of G tiles from base on
+   loads the G elements at s = min(base + G l, extent - G) (clamped so all stay inside the extent, which has at least G)
+   for the group's tiles 0 .. G - 1. Output row l of its tile x is then element s + x; it is written by the one lane with
+   s + x >= base + G l. */
+template <typename T>
+constexpr int group_max = 16 / (int)sizeof(T);
+template <typename T>
+__host__ __device__ constexpr int group_of(int c, int ntiles) { /* tiles of group c */
+  return (ntiles - c * group_max<T> < group_max<T> ? ntiles - c * group_max<T> : group_max<T>);
+}
+template <typename T>
+__device__ __forceinline__ int group_base(int c, int g, int l) { return 16 * group_max<T> * c + g * l; }
+template <typename T>
+__device__ __forceinline__ int group_start(int c, int g, int l, int extent) { return min(group_base<T>(c, g, l), extent - g); }
+
+/* G consecutive elements at the element type's alignment */
+typedef float f4u_t __attribute__((ext_vector_type(4), aligned(4)));
+struct f3u_t { float x, y, z; }; /* a vector of three would be loaded as four */
+template <int G, typename T>
+__device__ __forceinline__ void gload_group(T* v, const T* p) {
+  if constexpr (1 == G) {
+    v[0] = gload(p);
+  }
+  else if constexpr (2 == G) {
+    const typename pair_of<T>::type w = gload2(p);
+    v[0] = w[0];
+    v[1] = w[1];
+  }
+  else if constexpr (3 == G) {
+    const auto* const q = (const __attribute__((address_space(1))) f3u_t*)p;
+    v[0] = q->x;
+    v[1] = q->y;
+    v[2] = q->z;
+  }
+  else {
+    const f4u_t w = *(const __attribute__((address_space(1))) f4u_t*)p;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[i] = w[i];
+  }
+}
+
+/* this lane's elements of NTILE tiles, group by group */
+template <int NTILE, int C, typename T>
+__device__ __forceinline__ void gload_tiles(T* v, const T* p, const int* off) {
+  constexpr int V = group_max<T>;
+  gload_group<group_of<T>(C, NTILE)>(v + C * V, p + off[C]);
+  if constexpr ((C + 1) * V < NTILE) gload_tiles<NTILE, C + 1>(v, p, off);
 }
 
 /* Long C-runs are cut into pieces at the segment boundaries of the stack (multiples of the

@@ -136,8 +136,8 @@ static int lxs_smm_fit_kt(int datatype, int m, int n, int k, libsmm_acc_smm_conf
  * that split k (variant 4; 4 wavefronts per run, 32 stack entries per work-group, a kernel compiled for the
  * shape first): on ten such shapes it ran 0.81-1.0 of the best variant-4 configuration, itself 1.0-2.2x
  * faster than the best on 16x16 tiles. Other C blocks of up to 16 tiles of 16x16 (m, n <= 64) go to the
- * entry-parallel matrix-core kernel (variant 2) for exactly that tile grid, with the most wavefronts per
- * run compiled for it (8 up to 4 tiles, 4 up to 8, 2 up to 16; a kernel compiled for the shape first) and
+ * entry-parallel matrix-core kernel (variant 2) for exactly that tile grid, with 8 wavefronts per
+ * run up to 4 tiles, 4 up to 8, 2 up to 16 (a kernel compiled for the shape first) and
  * 32 (FP64) or 16 (FP32) stack entries per work-group: over the 419 such shapes of the autotuner's
  * 500-triplet sweeps this reaches 0.94 (FP64) and 0.92 (FP32) of each shape's best on average.
  * Larger blocks: the matrix-core kernel with one wavefront per run when at least 30% of the covered
@@ -735,7 +735,8 @@ int lxs_smm_tsplit(int bs, int split, int stack_size) {
  * Whole runs: a work-group takes the runs that begin among its entries, so fewer entries than a run has leave it one
  * run (32: 0.53-0.68 of the best at 3000 to 10000 entries), and stacks of short runs want few (FP64 23x23x23, 10000 entries
  * in runs of 1: 123 us with 24, 113 with 11). The kernels of large blocks have room for 512 work-groups only, and those
- * without a run of their own take the places of others: 24 (FP64 64x64x64, 12000 entries: 24 158 us, 16 227).
+ * without a run of their own take the places of others: 24 (FP64 64x64x64, 12000 entries: 24 158 us, 16 227; FP32
+ * 40x40x40, 10000 entries: 24 37 us, 16 48).
  */
 static void lxs_smm_pieces(int datatype, int m, int n, int k, int stack_size, const libsmm_acc_smm_config_t* config, int* bs,
   int* split) {
@@ -749,7 +750,7 @@ static void lxs_smm_pieces(int datatype, int m, int n, int k, int stack_size, co
   else if (0 != f64) lim[0] = 3.0, lim[1] = 8.0, lim[2] = 50.0;
   else lim[0] = 9.0, lim[1] = 25.0, lim[2] = 150.0;
   if (x < lim[0]) {
-    *bs = (8000 <= stack_size ? (2 < ep ? 16 : 24) : (2000 <= stack_size ? stack_size / 500 : 4));
+    *bs = (8000 <= stack_size ? (2 != config->variant || 8 >= config->tm * config->tn ? 16 : 24) : (2000 <= stack_size ? stack_size / 500 : 4));
     *split = 48 / *bs;
   }
   else if (x < lim[1]) *bs = 8, *split = 1;
@@ -768,7 +769,7 @@ static void lxs_smm_pieces(int datatype, int m, int n, int k, int stack_size, co
  * from 2000 to 500000 entries 0.95-0.99 of the best, where predicted and tuned rows reached 0.67-0.87. Up to 1000 entries
  * only the chain of one work-group counts, and the fold of more than 4 blocks is longer than the k-steps that it saves
  * (11x11x33, 300 entries: FP64 6.7 us with 9 blocks, 5.5 with one tile; FP32 11.0 and 6.1). Everything else: 16x16 tiles,
- * 4 wavefronts per run (2 above 8 tiles, all there are for short stacks).
+ * 4 wavefronts per run (FP64 above 8 tiles: 2; short stacks of 2 to 4 tiles: 8).
  */
 static int lxs_smm_rule(int datatype, int m, int n, int k, int stack_size, libsmm_acc_smm_config_t* config) {
   const int ti = (m + 15) / 16, tj = (n + 15) / 16, f64 = (dbcsr_type_real_8 == datatype);
@@ -789,7 +790,7 @@ static int lxs_smm_rule(int datatype, int m, int n, int k, int stack_size, libsm
     config->variant = 2;
     config->tm = ti;
     config->tn = tj;
-    config->nt = 64 * (8 < ti * tj ? 2 : ((0 != shortened && 16 < m + n && 4 >= ti * tj && 1 < ti * tj) ? 8 : 4));
+    config->nt = 64 * (0 != f64 && 8 < ti * tj ? 2 : ((0 != shortened && 16 < m + n && 4 >= ti * tj && 1 < ti * tj) ? 8 : 4));
     config->kt = 16;
   }
   config->bs = 24;

@@ -278,6 +278,13 @@ __global__ void __launch_bounds__(64 * NWI) smm_mfma(T* __restrict__ cdata, cons
  * (every wavefront computes it, so all take the same path through the barriers).
  * Barriers wait for LDS only (a fence restricted to the local address space).
  *
+ * 16x16 tiles: the rows of up to 16 bytes of tiles (2 in FP64, 4 in FP32) interleave, so one load per lane feeds them all
+ * (lxs::group_start). With one load per tile, as odd tile counts had it, each 128-byte line was touched 5 times and the
+ * L1 cache waited 0.72 of its time for lines on their way (FP32 45x45x13, S=100000: 183 -> 119 us, 33x33x4 S=200000 182
+ * -> 112, 60x50x40 S=20000 150 -> 126, 14x30x8 S=205558 54 -> 46; FP64 45x45x13 185 -> 174, 55x17x7 S=60000 69 -> 62,
+ * 15x48x12 S=19927 22 -> 20). The products are taken as B^T A^T: lanes 0 .. 15 hold neighbouring rows of C, so that the
+ * updates of an instruction lie in 4 columns instead of 16 (FP32 23x23x23, S=100000: 90 -> 74).
+ *
  * B4 (FP64, smm_mfma_eb): the same run protocol on 4x4 blocks instead of 16x16 tiles. v_mfma_f64_4x4x4_4b
  * multiplies four independent 4x4x4 blocks at the FP64 matrix-core rate of the 16x16x4 form (a quarter of
  * its cycles), so a C block is padded to multiples of 8 instead of 16: 23 x 23 takes 24 x 24 (54 MFMA per
@@ -410,16 +417,14 @@ __device__ __forceinline__ void ep_body(T* __restrict__ cdata, const T* __restri
     return stack_size;
   };
 
-  /* PAIR (even tile counts): paired tiles (lxs::pair_start), one two-element load per lane feeds two tiles,
-     which halves the fragment load instructions and the cache lines they touch */
-  constexpr bool PAIR = (0 == B4) && (0 == TI % 2) && (0 == TJ % 2);
-  constexpr int PI = (PAIR ? TI / 2 : 1), PJ = (PAIR ? TJ / 2 : 1);
+  /* 16x16 tiles: grouped (lxs::group_start), one load of up to 16 bytes per lane and group */
+  constexpr int V = lxs::group_max<T>, GI = (TI + V - 1) / V, GJ = (TJ + V - 1) / V;
   typedef typename lxs::pair_of<T>::type v2_t;
-  int aoff[TI], boff[TJ];
+  int aoff[GI], boff[GJ];
 #pragma unroll
-  for (int ti = 0; ti < TI; ++ti) aoff[ti] = (PAIR ? lxs::pair_start(ti >> 1, li, M) : min(16 * ti + li, M - 1));
+  for (int c = 0; c < GI; ++c) aoff[c] = lxs::group_start<T>(c, lxs::group_of<T>(c, TI), li, M);
 #pragma unroll
-  for (int tj = 0; tj < TJ; ++tj) boff[tj] = (PAIR ? lxs::pair_start(tj >> 1, li, N) : min(16 * tj + li, N - 1));
+  for (int c = 0; c < GJ; ++c) boff[c] = lxs::group_start<T>(c, lxs::group_of<T>(c, TJ), li, N);
   const T* const zeros = lxs::zeros<T>();
   /* B4: this lane's first A row r4 and first B column c4 (TI rows, TJ columns from there); element pairs start
      at min(row, M - 2) so they stay inside the block, and a pair whose first row is the last row of the block
@@ -442,7 +447,6 @@ __device__ __forceinline__ void ep_body(T* __restrict__ cdata, const T* __restri
   typedef typename lxs::mfma4<T>::acc_t acc4_t;
   acc4_t prod4[TI][TJ]; /* B4 */
   T fa[KB][TI], fb[KB][TJ];
-  v2_t pa[KB][PI], pb[KB][PJ];
   const acc_t zero = {T(0), T(0), T(0), T(0)};
 #pragma unroll
   for (int ti = 0; ti < TI; ++ti) {
@@ -522,17 +526,9 @@ __device__ __forceinline__ void ep_body(T* __restrict__ cdata, const T* __restri
       for (int p = 0; p < TJ2; ++p) qb[kb][p] = lxs::gload2(bp + min(c4 + 2 * p, N - 2));
       if constexpr (0 != TJ % 2) fb[kb][0] = gload(bp + min(c4 + TJ - 1, N - 1));
     }
-    else if constexpr (PAIR) {
-#pragma unroll
-      for (int p = 0; p < PI; ++p) pa[kb][p] = lxs::gload2(ap + aoff[2 * p]);
-#pragma unroll
-      for (int p = 0; p < PJ; ++p) pb[kb][p] = lxs::gload2(bp + boff[2 * p]);
-    }
     else {
-#pragma unroll
-      for (int ti = 0; ti < TI; ++ti) fa[kb][ti] = gload(ap + aoff[ti]);
-#pragma unroll
-      for (int tj = 0; tj < TJ; ++tj) fb[kb][tj] = gload(bp + boff[tj]);
+      lxs::gload_tiles<TI, 0>(fa[kb], ap, aoff);
+      lxs::gload_tiles<TJ, 0>(fb[kb], bp, boff);
     }
   };
   /* the k-step in slot kb; MASK: operands are zeroed where this lane's k lies past the range (not valid) */
@@ -555,15 +551,9 @@ __device__ __forceinline__ void ep_body(T* __restrict__ cdata, const T* __restri
     }
     else {
 #pragma unroll
-      for (int ti = 0; ti < TI; ++ti) {
-        if constexpr (PAIR) av[ti] = pa[kb][ti >> 1][ti & 1];
-        else av[ti] = fa[kb][ti];
-      }
+      for (int ti = 0; ti < TI; ++ti) av[ti] = fa[kb][ti];
 #pragma unroll
-      for (int tj = 0; tj < TJ; ++tj) {
-        if constexpr (PAIR) bv[tj] = pb[kb][tj >> 1][tj & 1];
-        else bv[tj] = fb[kb][tj];
-      }
+      for (int tj = 0; tj < TJ; ++tj) bv[tj] = fb[kb][tj];
     }
     if constexpr (MASK) {
 #pragma unroll
@@ -576,7 +566,7 @@ __device__ __forceinline__ void ep_body(T* __restrict__ cdata, const T* __restri
 #pragma unroll
       for (int tj = 0; tj < TJ; ++tj) {
         if constexpr (0 != B4) prod4[ti][tj] = lxs::mfma4<T>::mma(av[ti], bv[tj], prod4[ti][tj]);
-        else prod[ti][tj] = mfma<T>::mma(av[ti], bv[tj], prod[ti][tj]);
+        else prod[ti][tj] = mfma<T>::mma(bv[tj], av[ti], prod[ti][tj]); /* lane % 16: row of C, so a flush is coalesced */
       }
     }
   };
@@ -685,16 +675,17 @@ __device__ __forceinline__ void ep_body(T* __restrict__ cdata, const T* __restri
       for (int t = q; t < NTILE; t += EP) {
         const int ti = t / TJ, tj = t - ti * TJ;
         /* element of the block behind output row/column l of a tile, and whether this lane writes it */
-        const int j = (PAIR ? lxs::pair_start(tj >> 1, li, N) + (tj & 1) : 16 * tj + li);
-        const bool jown = (PAIR ? lxs::pair_owner(tj >> 1, tj & 1, li, N) : j < N);
+        const int ci = ti / V, cj = tj / V, gi = min(V, TI - ci * V), gj = min(V, TJ - cj * V);
+        const int i = lxs::group_start<T>(ci, gi, li, M) + (ti - ci * V);
+        const bool iown = (i >= lxs::group_base<T>(ci, gi, li));
 #pragma unroll
         for (int x = 0; x < 4; ++x) {
           T v = red[(t * 4 + x) * 64 + lane];
 #pragma unroll
           for (int p = 1; p < EP; ++p) v += red[((p * NTILE + t) * 4 + x) * 64 + lane];
-          const int ii = mfma<T>::row(lane, x);
-          const int i = (PAIR ? lxs::pair_start(ti >> 1, ii, M) + (ti & 1) : 16 * ti + ii);
-          const bool iown = (PAIR ? lxs::pair_owner(ti >> 1, ti & 1, ii, M) : i < M);
+          const int jj = mfma<T>::row(lane, x);
+          const int j = lxs::group_start<T>(cj, gj, jj, N) + (tj - cj * V);
+          const bool jown = (j >= lxs::group_base<T>(cj, gj, jj));
           if (iown && jown) {
             T* const ptr = cblk + j * M + i;
             if (flush_atomic) {
@@ -720,7 +711,7 @@ __device__ __forceinline__ void ep_body(T* __restrict__ cdata, const T* __restri
 #define LXS_EP_PASS cdata, adata, bdata, stack, stack_size, bs, m_rt, n_rt, k_rt, kt_unused, atomic, ps, pz, tsplit
 
 template <typename T, int TI, int TJ, int EP, int KB, int MC, int NC, int KC>
-__global__ void __launch_bounds__(64 * EP, (TI * TJ <= 4 ? (2 == EP && 6 == KB ? 3 : 4) : 1)) smm_mfma_ep(LXS_EP_ARGS) {
+__global__ void __launch_bounds__(64 * EP, (TI * TJ <= 4 ? (2 == EP && 6 == KB ? 3 : 4) : (4 == sizeof(T) && TI * TJ <= 9 ? 4 : 1))) smm_mfma_ep(LXS_EP_ARGS) {
   ep_body<T, TI, TJ, EP, KB, MC, NC, KC, 0>(LXS_EP_PASS);
 }
 /* FP64 on 4x4 blocks: C blocks up to 8 TI x 8 TJ */
@@ -777,6 +768,12 @@ const mfma_entry_t mfma_table[] = {
   LXS_MEG(2, 4, 4, 4) LXS_MEG(3, 1, 4, 4) LXS_MEG(3, 2, 4, 4) LXS_MEG(4, 1, 4, 4) LXS_MEG(4, 2, 4, 4)
   LXS_MEG(5, 1, 4, 4) LXS_MEG(1, 1, 8, 4) LXS_MEG(1, 2, 8, 4) LXS_MEG(1, 3, 8, 4) LXS_MEG(1, 4, 8, 4)
   LXS_MEG(2, 1, 8, 4) LXS_MEG(2, 2, 8, 4) LXS_MEG(3, 1, 8, 4) LXS_MEG(4, 1, 8, 4)
+#if !LXS_CAT(LXS_IS_, LXS_TAG)
+  /* FP32: 4 wavefronts per run up to 16 tiles (us with 2 and 4: 45x45x13, 10000 entries 24 and 18, 100000 119 and 108;
+     64x64x64, 30000 entries 291 and 217, 100000 604 and 554) */
+  LXS_MEG(2, 5, 4, 4) LXS_MEG(3, 3, 4, 4) LXS_MEG(3, 4, 4, 4) LXS_MEG(3, 5, 4, 4) LXS_MEG(4, 3, 4, 4)
+  LXS_MEG(4, 4, 4, 4) LXS_MEG(5, 2, 4, 4) LXS_MEG(5, 3, 4, 4)
+#endif
 #if LXS_CAT(LXS_IS_, LXS_TAG)
   /* entry-parallel on 4x4 blocks (FP64): the stack workloads whose blocks pad less to multiples of 8 than to 16 */
   LXS_EB(23, 23, 23, 3, 3, 4, 3) LXS_EB(23, 23, 23, 3, 3, 8, 3) LXS_EB(23, 23, 23, 3, 3, 4, 6)
