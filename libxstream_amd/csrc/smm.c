@@ -733,10 +733,12 @@ int lxs_smm_tsplit(int bs, int split, int stack_size) {
  * of 8 0.93 (whole 0.83-0.75), 8-50 pieces of 4 0.95-0.99 (whole 0.60-0.45), above 1 to 2 entries. The lines lie lower on
  * 4x4 blocks and higher in FP32, whose products take half the time and whose atomics do not (whole 0.93 at x = 6.7-10).
  * Whole runs: a work-group takes the runs that begin among its entries, so fewer entries than a run has leave it one
- * run (32: 0.53-0.68 of the best at 3000 to 10000 entries), and stacks of short runs want few (FP64 23x23x23, 10000 entries
- * in runs of 1: 123 us with 24, 113 with 11). The kernels of large blocks have room for 512 work-groups only, and those
- * without a run of their own take the places of others: 24 (FP64 64x64x64, 12000 entries: 24 158 us, 16 227; FP32
- * 40x40x40, 10000 entries: 24 37 us, 16 48).
+ * run (32: 0.53-0.68 of the best at 3000 to 10000 entries). Blocks above 16x16 keep a CU busy with one work-group, and two of
+ * them with a run on one CU, next to others without any, cost twice the time: at most 250 work-groups while a run is
+ * longer than their share, then 24 entries (us by entries per work-group: FP32 64x64x64 S=3000 12 46, 10 78; 32x32x32 S=3000 12
+ * 11.2, 6 16.8; 23x23x23 S=10000 24 14.3, 16 17.1; FP64 23x23x23 S=4000 16 10.3, 8 16.3; 64x64x64 S=12000 24 158, 16 227).
+ * Smaller blocks: up to 500 work-groups and 16 entries, which cost runs of 30 nothing and help stacks of short runs (FP32
+ * 8x8x8 S=10000 in runs of 1: 16 53 us, 24 74).
  */
 static void lxs_smm_pieces(int datatype, int m, int n, int k, int stack_size, const libsmm_acc_smm_config_t* config, int* bs,
   int* split) {
@@ -750,7 +752,8 @@ static void lxs_smm_pieces(int datatype, int m, int n, int k, int stack_size, co
   else if (0 != f64) lim[0] = 3.0, lim[1] = 8.0, lim[2] = 50.0;
   else lim[0] = 9.0, lim[1] = 25.0, lim[2] = 150.0;
   if (x < lim[0]) {
-    *bs = (8000 <= stack_size ? (2 != config->variant || 8 >= config->tm * config->tn ? 16 : 24) : (2000 <= stack_size ? stack_size / 500 : 4));
+    if (16 < m || 16 < n) *bs = (6000 <= stack_size ? 24 : (1000 <= stack_size ? stack_size / 250 : 4));
+    else *bs = (8000 <= stack_size ? 16 : (2000 <= stack_size ? stack_size / 500 : 4));
     *split = 48 / *bs;
   }
   else if (x < lim[1]) *bs = 8, *split = 1;
