@@ -22,6 +22,8 @@ struct mfma_entry_t {
 };
 
 const size_t lds_limit = 65536;
+/* k of one launch of the entry-parallel kernels: they multiply k and the flat indices of a run by 24-bit factors */
+const int ep_k_max = 1 << 24;
 
 /* In-place transpose of listed blocks: column-major m x n -> row-major m x n. Wavefront w of a work-group
  * transposes block blockIdx.x * W + w on its own (W = blockDim.x / 64 blocks in flight per work-group),
@@ -333,6 +335,19 @@ extern "C" int lxs_smm_launch(const lxs_smm_args_t* a, void* hip_stream) {
   const void *pa, *pb;
   const int* stack;
   void* args[14];
+  if (2 <= a->variant && a->variant <= 4 && ep_k_max < k) { /* parts of k, each one launch that adds to C */
+    const size_t ts = (3 == a->dtype ? 8 : 4);
+    int k0, result = 0;
+    for (k0 = 0; k0 < k && 0 == result;) {
+      lxs_smm_args_t part = *a;
+      part.a = (const char*)a->a + ts * (size_t)m * k0;
+      part.b = (const char*)a->b + ts * (size_t)n * k0;
+      part.k = (ep_k_max < k - k0 ? ep_k_max : k - k0);
+      k0 += part.k;
+      result = lxs_smm_launch(&part, hip_stream);
+    }
+    return result;
+  }
   if (1 <= a->variant && a->variant <= 4) {
     const mfma_entry_t* const e = mfma_find(a->dtype, a->variant, a->m, a->n, a->k, a->tm, a->tn, a->nt, a->kt);
     if (NULL == e) return LXS_ENOVARIANT;
