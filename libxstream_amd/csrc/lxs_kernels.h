@@ -95,20 +95,28 @@ int lxs_oz_preprocess(int dtype, const lxs_oz_operand_t* a, const lxs_oz_operand
 /* int8 GEMM over work items {level, u0, u1, pad} (host array), element (i, j) of item z at
    out + z Mp Np + j Mp + i. crt = 0 (scheme 1): s digit planes, item level L over the pairs (p, L - p),
    int32 partials, at most 2080 units (pair, k-block of 64) per item. crt = 1 (scheme 2): s residue
-   planes, item level = prime, sums mod m_prime as bytes, at most 2047 units (k-blocks) per item. */
+   planes, item level = prime, sums mod m_prime as bytes, at most 2047 units (k-blocks) per item.
+   gate: -1, or the cutoff of a call that lxs_oz_pairs serves unless few planes hold digits (lxs_oz_pairs_gate).
+   Items of a level without a pair of planes that both hold digits are not written. */
 int lxs_oz_level_gemm(int crt, const signed char* pa, const signed char* pb, const int* occa, const int* occb,
-  const int* items, int nitems, int s, int Mp, int Np, int Kp, void* out, void* hip_stream);
-/* FP64 recombination of the partials: zb[L] = first item of level L (cutoff + 2 entries) */
+  const int* items, int nitems, int s, int Mp, int Np, int Kp, void* out, int gate, void* hip_stream);
+/* FP64 recombination of the partials: zb[L] = first item of level L (cutoff + 2 entries); occa, occb: the planes that
+   hold digits (levels without a pair of them count as zero), or NULL: every level has its partials; gate: 0, or the Kp
+   of a call that lxs_oz_pairs serves unless few planes hold digits */
 int lxs_oz_recombine(int dtype, const int* c32, const int* zb, int cutoff, int Mp, int Np, const int* ea,
-  const int* eb, int M, int N, double alpha, double beta, void* c, int ldc, void* hip_stream);
+  const int* eb, int M, int N, double alpha, double beta, void* c, int ldc, const int* occa, const int* occb, int s,
+  int gate, void* hip_stream);
 /* Scheme 1 in one kernel, without partials (ozaki_pairs.h): cutoff s - 1 (triangle) or 2 (s - 1) (all pairs) and K
    short enough for exact int32 level sums (lxs_oz_pairs_fits); the same result as level GEMM and recombination */
 int lxs_oz_pairs_fits(int s, int cutoff, int Kp);
 /* work-groups that share a tile's k (1: none), with room for nitems partial planes of Mp x Np ints at part */
 int lxs_oz_pairs_split(int s, int cutoff, int M, int N, int Kp, int nitems);
+/* 1 for work so large that level GEMM and recombination are launched as well (gate): the kernels look at the planes that
+   hold digits, and oz_pairs or the other two leave at once */
+int lxs_oz_pairs_gate(int s, int cutoff, int M, int N, int Kp, int ks);
 int lxs_oz_pairs(int dtype, const signed char* pa, const signed char* pb, const int* occa, const int* occb, int s,
   int cutoff, int Mp, int Np, int Kp, const int* ea, const int* eb, int M, int N, double alpha, double beta, void* c,
-  int ldc, int ks, int* part, void* hip_stream);
+  int ldc, int ks, int* part, int gate, void* hip_stream);
 int lxs_oz_scale(int dtype, void* c, int ldc, int M, int N, double beta, void* hip_stream);
 /* bytes of the per-device static scratch of ozaki_gemm_noalloc (ozaki.hip) */
 #define LXS_OZ_STATIC_BYTES ((size_t)64 << 20)

@@ -454,7 +454,9 @@ static int oz_gemm_real(ozaki_context_t* ctx, hipStream_t hs, int ta, int tb, in
       /* the last pass may need fewer primes */
       const int np = (0 != l.crt ? oz_crt_primes(l.np, mb - trim, kk) : 0);
       const int pairs = (0 == l.crt && 0 != lxs_oz_pairs_fits(s, cutoff, Kp));
-      const int nitems = (0 == pairs ? oz_plan(ctx, l.crt, np, Kp / OZ_UNIT_K, tiles, impl->items, zb) : 0);
+      const int ks = (0 != pairs ? lxs_oz_pairs_split(s, cutoff, M, N, Kp, l.nitems) : 1);
+      const int gate = (0 != pairs ? lxs_oz_pairs_gate(s, cutoff, M, N, Kp, ks) : 0);
+      const int nitems = (0 == pairs || 0 != gate ? oz_plan(ctx, l.crt, np, Kp / OZ_UNIT_K, tiles, impl->items, zb) : 0);
       const double nprod = (0 != l.crt ? np : ozaki_count_pairs(s, cutoff, 0));
       const int nplanes = (0 != l.crt ? np : s);
       void* token = (NULL == fixed ? lxs_profile_begin(hs) : NULL);
@@ -469,7 +471,15 @@ static int oz_gemm_real(ozaki_context_t* ctx, hipStream_t hs, int ta, int tb, in
         token = (NULL == fixed ? lxs_profile_begin(hs) : NULL);
         result = lxs_oz_pairs(dtype, (const signed char*)(base + l.planes_a), (const signed char*)(base + l.planes_b), occ,
           occ + 8, s, cutoff, l.Mp, l.Np, Kp, (const int*)(base + l.ea), (const int*)(base + l.eb), M, N, alpha,
-          (0 == k0 ? beta : 1.0), dc, ldc, lxs_oz_pairs_split(s, cutoff, M, N, Kp, l.nitems), (int*)(base + l.out), hs);
+          (0 == k0 ? beta : 1.0), dc, ldc, ks, (int*)(base + l.out), gate, hs);
+        if (0 == result && 0 != gate) { /* these leave at once if that one did the work, and the other way round */
+          result = lxs_oz_level_gemm(0, (const signed char*)(base + l.planes_a), (const signed char*)(base + l.planes_b),
+            occ, occ + 8, impl->items, nitems, s, l.Mp, l.Np, Kp, base + l.out, cutoff, hs);
+        }
+        if (0 == result && 0 != gate) {
+          result = lxs_oz_recombine(dtype, (const int*)(base + l.out), zb, cutoff, l.Mp, l.Np, (const int*)(base + l.ea),
+            (const int*)(base + l.eb), M, N, alpha, (0 == k0 ? beta : 1.0), dc, ldc, occ, occ + 8, s, Kp, hs);
+        }
         lxs_profile_end(token, hs, "ozaki_i8", 2.0 * nprod * l.Mp * l.Np * Kp,
           (double)nplanes * (l.Mp + l.Np) * Kp + (double)ts * M * N * (0 == k0 && 0 == beta ? 1 : 2));
         continue;
@@ -477,7 +487,7 @@ static int oz_gemm_real(ozaki_context_t* ctx, hipStream_t hs, int ta, int tb, in
       if (0 == result) { /* int8 work of every pair up to the cutoff (pairs of all-zero planes are skipped), or every prime */
         token = (NULL == fixed ? lxs_profile_begin(hs) : NULL);
         result = lxs_oz_level_gemm(l.crt, (const signed char*)(base + l.planes_a), (const signed char*)(base + l.planes_b),
-          occ, occ + 8, impl->items, nitems, nplanes, l.Mp, l.Np, Kp, base + l.out, hs);
+          occ, occ + 8, impl->items, nitems, nplanes, l.Mp, l.Np, Kp, base + l.out, -1, hs);
         lxs_profile_end(token, hs, "ozaki_i8", 2.0 * nprod * l.Mp * l.Np * Kp,
           (double)nplanes * (l.Mp + l.Np) * Kp + (0 != l.crt ? 1.0 : 4.0) * nitems * l.Mp * l.Np);
       }
@@ -492,7 +502,7 @@ static int oz_gemm_real(ozaki_context_t* ctx, hipStream_t hs, int ta, int tb, in
         }
         else {
           result = lxs_oz_recombine(dtype, (const int*)(base + l.out), zb, cutoff, l.Mp, l.Np, (const int*)(base + l.ea),
-            (const int*)(base + l.eb), M, N, alpha, (0 == k0 ? beta : 1.0), dc, ldc, hs);
+            (const int*)(base + l.eb), M, N, alpha, (0 == k0 ? beta : 1.0), dc, ldc, occ, occ + 8, s, 0, hs);
           lxs_profile_end(token, hs, "ozaki_fp64", 0.0, 4.0 * nitems * M * N + bc);
         }
       }

@@ -24,9 +24,10 @@
  *               zero are skipped. Every item writes int32 partial sums (exact: an item's units are
  *               bounded).
  *   oz_recombine   per element: S_L = exact int64 sum of the level's partials, cd = sum over
- *               L = cutoff .. 0 of 2^(-7(L+2)) S_L in FP64, C = fma(alpha, 2^(ea+eb) cd, beta C).
+ *               L = cutoff .. 0 of 2^(-7(L+2)) S_L in FP64, C = fma(alpha, 2^(ea+eb) cd, beta C). Levels
+ *               without a pair whose planes both hold digits are neither written nor read.
  *               (Scheme 1 over the triangle or all pairs goes to ozaki_pairs.h instead of these two, unless K
- *               is too long for int32 level sums.)
+ *               is too long for int32 level sums, or the product is large and few planes hold digits.)
  *   dgemm_f64   128x128 or 64x64 tiles with v_mfma_f64_16x16x4f64 on FP64 operands (the comparator).
  */
 #include <hip/hip_runtime.h>
@@ -284,7 +285,7 @@ constexpr int oz_wait_vm_lgkm0(int vm) { return (vm & 15) | ((vm >> 4) << 14) | 
 template <int CRT, int NST>
 __global__ void __launch_bounds__(256) oz_level_gemm(const int8_t* __restrict__ pa, const int8_t* __restrict__ pb,
   const int* __restrict__ occa, const int* __restrict__ occb, oz_items_t items, int s, int Mp, int Np, int Kp,
-  const int8_t* __restrict__ zero, void* __restrict__ out) {
+  const int8_t* __restrict__ zero, void* __restrict__ out, int gate) {
   /* one array per stage ([A|B][256 rows x 64 bytes]): distinct objects, so the compiler can tell the DMA
      targets of the stages in flight from the stage being read */
   __shared__ __attribute__((aligned(1024))) int8_t ls0[2 * QTILE], ls1[2 * QTILE], ls2[2 * QTILE], ls3[2 * QTILE];
@@ -300,13 +301,12 @@ __global__ void __launch_bounds__(256) oz_level_gemm(const int8_t* __restrict__ 
   const int pend = (0 != CRT ? L + 1 : (L < s - 1 ? L : s - 1) + 1);
   unsigned int oa = ~0u, ob = ~0u;
   if (0 == CRT) {
-    oa = ob = 0;
-    for (int p = 0; p < s; ++p) {
-      oa |= (0 != occa[p] ? 1u : 0u) << p;
-      ob |= (0 != occb[p] ? 1u : 0u) << p;
-    }
-    oa = __builtin_amdgcn_readfirstlane(oa);
-    ob = __builtin_amdgcn_readfirstlane(ob);
+    oa = oz_occupied(occa, s);
+    ob = oz_occupied(occb, s);
+    if (0 <= gate && !oz_few_pairs(oa, ob, s, gate, Kp)) return; /* oz_pairs' */
+    unsigned int levels;
+    (void)oz_some_pairs(oa, ob, s, L, levels);
+    if (0 == ((levels >> L) & 1u)) return; /* oz_recombine skips the level */
   }
   /* pair p of the item has work: both planes hold a nonzero digit (always, for residues) */
   auto active = [&](int p) -> bool { return 0 != CRT || 0 != ((oa >> p) & (ob >> (L - p)) & 1u); };
@@ -509,13 +509,20 @@ struct oz_levels_t {
 template <typename T>
 __global__ void __launch_bounds__(256) oz_recombine(const int* __restrict__ c32, oz_levels_t lv, int cutoff, int Mp,
   int Np, const int* __restrict__ ea, const int* __restrict__ eb, int M, int N, double alpha, double beta,
-  T* __restrict__ c, int ldc) {
+  T* __restrict__ c, int ldc, const int* __restrict__ occa, const int* __restrict__ occb, int s, int gate) { /* gate: 0, or Kp */
+  unsigned int levels = ~0u; /* bit L: the level has partials */
+  if (NULL != occa) {
+    const unsigned int oa = oz_occupied(occa, s), ob = oz_occupied(occb, s);
+    if (0 != gate && !oz_few_pairs(oa, ob, s, cutoff, gate)) return;
+    (void)oz_some_pairs(oa, ob, s, cutoff, levels);
+  }
   for (long x = blockIdx.x * 256L + threadIdx.x; x < (long)M * N; x += (long)gridDim.x * 256) {
     const int i = (int)(x % M), j = (int)(x / M);
     const long o = (long)j * Mp + i;
     double cd = 0;
     for (int L = cutoff; L >= 0; --L) {
       long long sum = 0;
+      if (0 == ((levels >> L) & 1u)) continue;
       for (int z = lv.zb[L]; z < lv.zb[L + 1]; ++z) sum += c32[(long)z * Mp * Np + o];
       cd += ldexp(1.0, -7 * (L + 2)) * (double)sum;
     }
@@ -1217,7 +1224,7 @@ extern "C" int lxs_oz_static_scratch(void** ptr) {
 /* items: host array of nitems x {level, u0, u1, pad}; item z writes at out + z * Mp * Np (int32 partials,
    or residue bytes with crt); planes row-padded to a multiple of 256 and k-padded to a multiple of 128 */
 extern "C" int lxs_oz_level_gemm(int crt, const signed char* pa, const signed char* pb, const int* occa,
-  const int* occb, const int* items, int nitems, int s, int Mp, int Np, int Kp, void* out, void* hip_stream) {
+  const int* occb, const int* items, int nitems, int s, int Mp, int Np, int Kp, void* out, int gate, void* hip_stream) {
   const int8_t* const zero = oz_zero_ptr();
   const int nkb = Kp / QK;
   if (0 != Mp % LT || 0 != Np % LT || 0 != Kp % LK || 0 >= Kp || (1 << 22) < Kp || 0 >= nitems || NULL == zero) {
@@ -1259,10 +1266,10 @@ extern "C" int lxs_oz_level_gemm(int crt, const signed char* pa, const signed ch
     const hipStream_t st = (hipStream_t)hip_stream;
     void* const o = (0 == crt ? (void*)((int*)out + (long)z0 * Mp * Np) : (void*)((uint8_t*)out + (long)z0 * Mp * Np));
     const int8_t *a8 = (const int8_t*)pa, *b8 = (const int8_t*)pb;
-    if (0 == crt && 4 == nst) oz_level_gemm<0, 4><<<grid, 256, 0, st>>>(a8, b8, occa, occb, arg, s, Mp, Np, Kp, zero, o);
-    else if (0 == crt) oz_level_gemm<0, 5><<<grid, 256, 0, st>>>(a8, b8, occa, occb, arg, s, Mp, Np, Kp, zero, o);
-    else if (4 == nst) oz_level_gemm<1, 4><<<grid, 256, 0, st>>>(a8, b8, occa, occb, arg, s, Mp, Np, Kp, zero, o);
-    else oz_level_gemm<1, 5><<<grid, 256, 0, st>>>(a8, b8, occa, occb, arg, s, Mp, Np, Kp, zero, o);
+    if (0 == crt && 4 == nst) oz_level_gemm<0, 4><<<grid, 256, 0, st>>>(a8, b8, occa, occb, arg, s, Mp, Np, Kp, zero, o, gate);
+    else if (0 == crt) oz_level_gemm<0, 5><<<grid, 256, 0, st>>>(a8, b8, occa, occb, arg, s, Mp, Np, Kp, zero, o, gate);
+    else if (4 == nst) oz_level_gemm<1, 4><<<grid, 256, 0, st>>>(a8, b8, occa, occb, arg, s, Mp, Np, Kp, zero, o, gate);
+    else oz_level_gemm<1, 5><<<grid, 256, 0, st>>>(a8, b8, occa, occb, arg, s, Mp, Np, Kp, zero, o, gate);
   }
   return (int)hipGetLastError();
 }
@@ -1311,7 +1318,8 @@ extern "C" int lxs_oz_crt_recombine(int dtype, const unsigned char* r8, const in
 
 /* zb: first item per level, cutoff + 2 entries */
 extern "C" int lxs_oz_recombine(int dtype, const int* c32, const int* zb, int cutoff, int Mp, int Np, const int* ea,
-  const int* eb, int M, int N, double alpha, double beta, void* c, int ldc, void* hip_stream) {
+  const int* eb, int M, int N, double alpha, double beta, void* c, int ldc, const int* occa, const int* occb, int s,
+  int gate, void* hip_stream) {
   oz_levels_t lv;
   const long blocks = ((long)M * N + 255) / 256;
   const unsigned int grid = (unsigned int)(blocks < 4096 ? blocks : 4096);
@@ -1320,11 +1328,11 @@ extern "C" int lxs_oz_recombine(int dtype, const int* c32, const int* zb, int cu
   for (int L = 0; L < 17; ++L) lv.zb[L] = (L <= cutoff + 1 ? zb[L] : zb[cutoff + 1]);
   if (3 == dtype) {
     oz_recombine<double><<<grid, 256, 0, (hipStream_t)hip_stream>>>(c32, lv, cutoff, Mp, Np, ea, eb, M, N, alpha, beta,
-      (double*)c, ldc);
+      (double*)c, ldc, occa, occb, s, gate);
   }
   else if (1 == dtype) {
     oz_recombine<float><<<grid, 256, 0, (hipStream_t)hip_stream>>>(c32, lv, cutoff, Mp, Np, ea, eb, M, N, alpha, beta,
-      (float*)c, ldc);
+      (float*)c, ldc, occa, occb, s, gate);
   }
   else {
     return LXS_ENOVARIANT;

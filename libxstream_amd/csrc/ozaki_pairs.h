@@ -26,6 +26,40 @@ __device__ __forceinline__ void ozp_dma16(const int8_t* src, int8_t* lds_dst) {
     (__attribute__((address_space(3))) void*)lds_dst, 16, 0, 0);
 }
 
+/* one bit per plane that holds a nonzero digit (one load for all of them) */
+__device__ __forceinline__ unsigned int oz_occupied(const int* occ, int s) {
+  const int lane = threadIdx.x & 63;
+  return (unsigned int)__ballot(lane < s && 0 != occ[lane < s ? lane : 0]);
+}
+/* the pairs p + q <= cutoff with digits in both planes; levels: one bit per level p + q that has any */
+__device__ __forceinline__ int oz_some_pairs(unsigned int oa, unsigned int ob, int s, int cutoff, unsigned int& levels) {
+  int some = 0;
+  levels = 0;
+  for (int p = 0; p < s && p <= cutoff; ++p) {
+    const unsigned int q = (0 != ((oa >> p) & 1u) ? ob & ((2u << (cutoff - p)) - 1u) : 0u);
+    some += __popc(q);
+    levels |= q << p;
+  }
+  return some;
+}
+/* all pairs up to the cutoff s - 1 or 2 (s - 1) */
+__host__ __device__ constexpr int oz_all_pairs(int s, int cutoff) { return (2 * (s - 1) == cutoff ? s * s : s * (s + 1) / 2); }
+/*
+ * 1 when oz_level_gemm and oz_recombine, which move and multiply only the planes with digits, are faster than oz_pairs,
+ * which moves every plane of a tile: the products of the pairs with digits, and int32 partials per level that cost about
+ * as much as 3000 k of a pair, against the products of all pairs. ms a call by the bits of whole numbers in FP64 (one
+ * plane per 7), oz_pairs / the other two: 8192^3, 8 slices, triangle: 7 bits 11.5 / 1.6, 21 13.2 / 5.6, 35 16.0 / 12.3, 42
+ * 15.7 / 14.9; 4096^3 all pairs 7 1.64 / 0.42, 28 2.2 / 1.47, 42 2.8 / 2.66; 8192x8192x1024 all pairs 28 2.34 / 2.23, 35
+ * 2.58 / 2.97, 6 slices 28 1.79 / 2.15. The partials cost more where all pairs share a tile's loads.
+ */
+__device__ __forceinline__ bool oz_few_pairs(unsigned int oa, unsigned int ob, int s, int cutoff, int Kp) {
+  unsigned int levels;
+  const int some = oz_some_pairs(oa, ob, s, cutoff, levels);
+  /* whole numbers: the three kernels of a call have to agree */
+  return 100L * ((long)some * Kp + 3000L * __popc(levels)) <=
+    (2 * (s - 1) == cutoff ? 75L : 92L) * oz_all_pairs(s, cutoff) * Kp;
+}
+
 /*
  * A work-group of 4 wavefronts (2 x 2) computes 64 WI x 64 elements of C, a wavefront 32 WI x 32 (v_mfma_i32_32x32x32_i8,
  * the B planes as first operand as in oz_level_gemm): CUT + 1 level sums of 16 WI registers each. Per block of 64 k the
@@ -47,7 +81,7 @@ template <int NS, int CUT, int WI>
 __global__ void __launch_bounds__(256) oz_pairs(const int8_t* __restrict__ pa, const int8_t* __restrict__ pb,
   const int* __restrict__ occa, const int* __restrict__ occb, int Mp, int Np, int Kp, int tiles_m, int tiles_n,
   const int* __restrict__ ea, const int* __restrict__ eb, int M, int N, double alpha, double beta, int dtype,
-  void* __restrict__ c, long ldc, int* __restrict__ part) {
+  void* __restrict__ c, long ldc, int* __restrict__ part, int gate) {
   constexpr int RA = 64 * WI, BUF = NS * (RA + PT) * 64, NDMA = NS * (WI + 1);
   __shared__ __attribute__((aligned(1024))) int8_t lds0[BUF], lds1[BUF];
   const int tid = threadIdx.x, lane = tid & 63;
@@ -66,14 +100,15 @@ __global__ void __launch_bounds__(256) oz_pairs(const int8_t* __restrict__ pa, c
   /* this work-group's blocks of k (all of them, or part blockIdx.y of gridDim.y, a multiple of two) */
   const int kb0 = 2 * (int)((long)(nkb / 2) * blockIdx.y / gridDim.y);
   const int kb1 = 2 * (int)((long)(nkb / 2) * (blockIdx.y + 1) / gridDim.y);
-  unsigned int oa = 0, ob = 0;
-#pragma unroll
-  for (int p = 0; p < NS; ++p) {
-    oa |= (0 != occa[p] ? 1u : 0u) << p;
-    ob |= (0 != occb[p] ? 1u : 0u) << p;
+  constexpr unsigned int EVERY = (1u << NS) - 1u;
+  unsigned int oa = oz_occupied(occa, NS), ob = oz_occupied(occb, NS); /* the planes to move and multiply */
+  if (0 != gate && oz_few_pairs(oa, ob, NS, CUT, Kp)) return; /* oz_level_gemm's */
+  {
+    /* above 0.65 of the pairs the products without branches are faster, zero planes and all (4096^3, 8 slices, ms:
+       triangle, 24 of 36 pairs 2.29 with branches, 2.16 without; all pairs, 36 of 64 2.77 and 3.06) */
+    unsigned int levels;
+    if (20 * oz_some_pairs(oa, ob, NS, CUT, levels) > 13 * oz_all_pairs(NS, CUT)) oa = ob = EVERY;
   }
-  oa = __builtin_amdgcn_readfirstlane(oa);
-  ob = __builtin_amdgcn_readfirstlane(ob);
   i16_t acc[CUT + 1][WI];
 #pragma unroll
   for (int L = 0; L <= CUT; ++L) {
@@ -85,14 +120,16 @@ __global__ void __launch_bounds__(256) oz_pairs(const int8_t* __restrict__ pa, c
   const int8_t* const ga = pa + ((long)(i0 / PROWS) * nkb * PROWS + i0 % PROWS) * 64;
   const int8_t* const gb = pb + ((long)(j0 / PROWS) * nkb * PROWS + j0 % PROWS) * 64;
   const long sa = (long)Mp * Kp, sb = (long)Np * Kp; /* bytes of a plane */
-  const auto dma = [&](int8_t* buf, int kb) {
+  const auto dma = [&](int8_t* buf, int kb, unsigned int ma, unsigned int mb) { /* ma, mb: the planes of A and B to move */
     const int8_t* const ka = ga + (long)kb * (PROWS * 64);
     const int8_t* const kbp = gb + (long)kb * (PROWS * 64);
 #pragma unroll
     for (int p = 0; p < NS; ++p) {
+      if (0 != ((ma >> p) & 1u)) {
 #pragma unroll
-      for (int x = 0; x < WI; ++x) ozp_dma16(ka + p * sa + x * 4096 + doff, buf + p * RA * 64 + x * 4096 + wave * 1024);
-      ozp_dma16(kbp + p * sb + doff, buf + NS * RA * 64 + p * 4096 + wave * 1024);
+        for (int x = 0; x < WI; ++x) ozp_dma16(ka + p * sa + x * 4096 + doff, buf + p * RA * 64 + x * 4096 + wave * 1024);
+      }
+      if (0 != ((mb >> p) & 1u)) ozp_dma16(kbp + p * sb + doff, buf + NS * RA * 64 + p * 4096 + wave * 1024);
     }
   };
   const int frow = lane & 31, fswz = (frow >> 2) & 3;
@@ -136,11 +173,11 @@ __global__ void __launch_bounds__(256) oz_pairs(const int8_t* __restrict__ pa, c
     __builtin_amdgcn_s_barrier(); /* no fence: DMA and reads are counted above */ \
     __asm__ __volatile__("" ::: "memory"); \
   } while (0)
-  dma(lds0, kb0);
+  dma(lds0, kb0, oa, ob);
   OZP_MIDSYNC();
-  dma(lds1, kb0 + 1);
+  dma(lds1, kb0 + 1, oa, ob);
   frags(lds0, 0, 0);
-  if ((1u << NS) - 1u == (oa & ob)) { /* every plane holds a digit: no branches */
+  if (EVERY == (oa & ob)) { /* no branches */
     /* a block: its second half's fragments while the first half is multiplied; then the DMA of the block after next
        and the next block's first fragments while the second half is multiplied */
 #define OZP_BLOCK(CUR, NXT, KB) \
@@ -153,7 +190,7 @@ __global__ void __launch_bounds__(256) oz_pairs(const int8_t* __restrict__ pa, c
     } \
     if constexpr (NM > NS * (WI + 1)) __builtin_amdgcn_sched_group_barrier(0x008, NM - NS * (WI + 1), 0); \
     OZP_MIDSYNC(); \
-    dma(CUR, min((KB) + 2, kb1 - 1)); \
+    dma(CUR, min((KB) + 2, kb1 - 1), EVERY, EVERY); \
     frags(NXT, 0, 0); \
     mfmas(1); \
     _Pragma("unroll") for (int i_ = 0; i_ < NS * (WI + 1); ++i_) { \
@@ -189,13 +226,13 @@ __global__ void __launch_bounds__(256) oz_pairs(const int8_t* __restrict__ pa, c
       frags(lds0, 1, 1);
       some(0);
       OZP_MIDSYNC();
-      dma(lds0, min(kb + 2, kb1 - 1));
+      dma(lds0, min(kb + 2, kb1 - 1), oa, ob);
       frags(lds1, 0, 0);
       some(1);
       frags(lds1, 1, 1);
       some(0);
       OZP_MIDSYNC();
-      dma(lds1, min(kb + 3, kb1 - 1));
+      dma(lds1, min(kb + 3, kb1 - 1), oa, ob);
       frags(lds0, 0, 0);
       some(1);
     }
@@ -245,13 +282,13 @@ __global__ void __launch_bounds__(256) oz_pairs(const int8_t* __restrict__ pa, c
 
 template <int NS, int CUT>
 int oz_pairs_launch(const int8_t* pa, const int8_t* pb, const int* occa, const int* occb, int Mp, int Np, int Kp, const int* ea,
-  const int* eb, int M, int N, double alpha, double beta, int dtype, void* c, int ldc, int ks, int* part, hipStream_t st) {
+  const int* eb, int M, int N, double alpha, double beta, int dtype, void* c, int ldc, int ks, int* part, int gate, hipStream_t st) {
   /* 128 rows of A per tile where the level sums fit 256 registers and two buffers the LDS */
   constexpr int WI = (32 * (CUT + 1) <= 256 && NS <= 6 ? 2 : 1);
   const int tm = (M + 64 * WI - 1) / (64 * WI), tn = (N + PT - 1) / PT;
   if ((double)tm * tn > 2147483647.0) return LXS_ELIMIT;
   oz_pairs<NS, CUT, WI><<<dim3((unsigned int)(tm * tn), (unsigned int)ks), 256, 0, st>>>(pa, pb, occa, occb, Mp, Np, Kp, tm,
-    tn, ea, eb, M, N, alpha, beta, dtype, c, (long)ldc, part);
+    tn, ea, eb, M, N, alpha, beta, dtype, c, (long)ldc, part, gate);
   return (int)hipGetLastError();
 }
 
@@ -270,14 +307,22 @@ extern "C" int lxs_oz_pairs_split(int s, int cutoff, int M, int N, int Kp, int n
   return (2 <= ks ? (int)ks : 1);
 }
 
+/* from this much work on (pairs x M x N x K; 0.6 ms of products) a call launches oz_pairs and oz_level_gemm, of which one
+   leaves the work to the other by the planes that hold digits */
+constexpr double OZP_GATE_WORK = 5e11;
+
+extern "C" int lxs_oz_pairs_gate(int s, int cutoff, int M, int N, int Kp, int ks) {
+  return (1 == ks && 2 < s && OZP_GATE_WORK <= (double)oz_all_pairs(s, cutoff) * M * N * Kp) ? 1 : 0;
+}
+
 extern "C" int lxs_oz_pairs(int dtype, const signed char* pa, const signed char* pb, const int* occa, const int* occb, int s,
   int cutoff, int Mp, int Np, int Kp, const int* ea, const int* eb, int M, int N, double alpha, double beta, void* c, int ldc,
-  int ks, int* part, void* hip_stream) {
+  int ks, int* part, int gate, void* hip_stream) {
   const hipStream_t st = (hipStream_t)hip_stream;
   const int8_t *a8 = (const int8_t*)pa, *b8 = (const int8_t*)pb;
   int result;
   if (0 == lxs_oz_pairs_fits(s, cutoff, Kp) || 0 != Mp % 256 || 0 != Np % 256 || 0 != Kp % 128 || Mp < M || Np < N ||
-      1 > ks || Kp / 128 < ks || (1 < ks && NULL == part)) {
+      1 > ks || Kp / 128 < ks || (1 < ks && (NULL == part || 0 != gate))) {
     return LXS_ELIMIT;
   }
   if (3 != dtype && 1 != dtype) return LXS_ENOVARIANT;
@@ -286,9 +331,9 @@ extern "C" int lxs_oz_pairs(int dtype, const signed char* pa, const signed char*
 #define OZP_CASE(NS) \
   case NS: \
     result = (NS - 1 == cutoff) ? oz_pairs_launch<NS, NS - 1>(a8, b8, occa, occb, Mp, Np, Kp, ea, eb, M, N, alpha, beta, \
-                                    dtype, c, ldc, ks, part, st) \
+                                    dtype, c, ldc, ks, part, gate, st) \
                                 : oz_pairs_launch<NS, 2 * (NS - 1)>(a8, b8, occa, occb, Mp, Np, Kp, ea, eb, M, N, alpha, \
-                                    beta, dtype, c, ldc, ks, part, st); \
+                                    beta, dtype, c, ldc, ks, part, gate, st); \
     break;
   switch (s) {
     OZP_CASE(1)
@@ -305,7 +350,8 @@ extern "C" int lxs_oz_pairs(int dtype, const signed char* pa, const signed char*
   if (0 == result && 1 < ks) { /* level L: the ks partials from L ks on */
     int zb[17], L;
     for (L = 0; L <= cutoff + 1; ++L) zb[L] = L * ks;
-    result = lxs_oz_recombine(dtype, part, zb, cutoff, Mp, Np, ea, eb, M, N, alpha, beta, c, ldc, hip_stream);
+    result = lxs_oz_recombine(dtype, part, zb, cutoff, Mp, Np, ea, eb, M, N, alpha, beta, c, ldc, NULL, NULL, s, 0,
+      hip_stream);
   }
   return result;
 }
