@@ -45,7 +45,9 @@
 typedef struct libsmm_acc_smm_config_t {
   int variant, tm, tn, nt, bs, kt, flush;
   int s;         /* stack size bs was chosen for (CSV column S); shorter stacks launch with bs scaled down
-                    (samples/smm/smm_kernel.c:463-473); 0: bs as given */
+                    (samples/smm/smm_kernel.c:463-473); 0: bs as given. For rows of the file that ships with the
+                    library, libsmm_acc_process chooses bs, split, and for variant 4 also nt and kt, of stacks below
+                    16384 entries by itself; a configuration that the caller gives is launched as it is */
   int split;     /* C-runs longer than split x bs entries are cut into pieces added atomically (CSV column
                     SPLIT); 0: LIBXSTREAM_SMM_SPLIT (default 2). In stacks of at least 16384 entries runs of
                     up to 64 entries are never cut (bitwise-reproducible C); LIBXSTREAM_SMM_SPLIT_MIN=n

@@ -26,6 +26,7 @@
 typedef struct lxs_smm_slot_t {
   int type, m, n, k, used, source;
   int devmatch; /* 1: a CSV row of the device that best matches the active one */
+  int shipped;  /* 1: a row of the file that ships with the library, which short stacks may be cut by (lxs_smm_pieces) */
   libsmm_acc_smm_config_t config;
 } lxs_smm_slot_t;
 
@@ -280,7 +281,7 @@ static int lxs_smm_env(libsmm_acc_smm_config_t* config) {
 }
 
 static int lxs_smm_register(int datatype, int m, int n, int k, const libsmm_acc_smm_config_t* config, int source,
-  int keep_best, int devmatch);
+  int keep_best, int devmatch, int shipped);
 
 static void lxs_smm_resolve(int datatype, int m, int n, int k, libsmm_acc_smm_config_t* config, int* source) {
   const lxs_smm_slot_t* slot;
@@ -296,7 +297,7 @@ static void lxs_smm_resolve(int datatype, int m, int n, int k, libsmm_acc_smm_co
     if (EXIT_SUCCESS == lxs_learned_predict(datatype, m, n, k, config)) { /* cached for the next lookup */
       src = libsmm_acc_config_learned;
       config->s = LXS_SMM_S; /* the model learned from sweeps at this stack size */
-      (void)lxs_smm_register(datatype, m, n, k, config, libsmm_acc_config_learned, 0, 0);
+      (void)lxs_smm_register(datatype, m, n, k, config, libsmm_acc_config_learned, 0, 0, 0);
     }
     else {
       lxs_smm_default(datatype, m, n, k, config);
@@ -338,7 +339,7 @@ LIBXSTREAM_API int libsmm_acc_config_get(libsmm_acc_data_t datatype, int m, int 
    over rows of other devices whatever their speed, and among rows of equal standing a duplicate replaces
    the entry only when it is faster (smm_acc.c:117-119, :204-235) */
 static int lxs_smm_register(int datatype, int m, int n, int k, const libsmm_acc_smm_config_t* config, int source,
-  int keep_best, int devmatch) {
+  int keep_best, int devmatch, int shipped) {
   lxs_smm_slot_t* slot;
   int result = EXIT_SUCCESS;
   pthread_mutex_lock(&lxs_smm_lock);
@@ -349,6 +350,7 @@ static int lxs_smm_register(int datatype, int m, int n, int k, const libsmm_acc_
       slot->config = *config;
       slot->source = source;
       slot->devmatch = devmatch;
+      slot->shipped = shipped;
     }
   }
   else {
@@ -363,7 +365,7 @@ LIBXSTREAM_API int libsmm_acc_config_set(libsmm_acc_data_t datatype, int m, int 
   if (EXIT_SUCCESS != libsmm_acc_config_valid(datatype, m, n, k, config)) {
     return lxs_error(EXIT_FAILURE, "libsmm_acc_config_set: configuration not valid for this shape");
   }
-  return lxs_smm_register((int)datatype, m, n, k, config, libsmm_acc_config_tuned, 0, 0);
+  return lxs_smm_register((int)datatype, m, n, k, config, libsmm_acc_config_tuned, 0, 0, 0);
 }
 
 LIBXSTREAM_API int libsmm_acc_kernel_variants(libsmm_acc_data_t datatype, int* quintuples, int cap) {
@@ -472,11 +474,7 @@ static void lxs_row_device(const char* line, int column, char* device, size_t si
   snprintf(device, size, "%.*s", (int)strcspn(line, lxs_delims), line);
 }
 
-LIBXSTREAM_API int libsmm_acc_params_load(const char* filename) {
-  return libsmm_acc_params_load_device(filename, NULL);
-}
-
-LIBXSTREAM_API int libsmm_acc_params_load_device(const char* filename, const char* device) {
+static int lxs_smm_params_load(const char* filename, const char* device, int shipped) {
   char line[1024], names[32][16], best[256] = "", active[16][32];
   int ncolumns = 0, nrows = 0, native, with_device, with_perf, nactive, devcol;
   long body;
@@ -572,7 +570,7 @@ LIBXSTREAM_API int libsmm_acc_params_load_device(const char* filename, const cha
     }
     if (0 != ok) {
       if (EXIT_SUCCESS != lxs_smm_register(key[0], key[1], key[2], key[3], &config, libsmm_acc_config_tuned, 1,
-                             devmatch)) {
+                             devmatch, shipped)) {
         break;
       }
       ++nrows;
@@ -583,6 +581,12 @@ LIBXSTREAM_API int libsmm_acc_params_load_device(const char* filename, const cha
   }
   fclose(file);
   return nrows;
+}
+
+LIBXSTREAM_API int libsmm_acc_params_load(const char* filename) { return lxs_smm_params_load(filename, NULL, 0); }
+
+LIBXSTREAM_API int libsmm_acc_params_load_device(const char* filename, const char* device) {
+  return lxs_smm_params_load(filename, device, 0);
 }
 
 LIBXSTREAM_API int libsmm_acc_params_save(const char* filename, const char* device) {
@@ -622,7 +626,7 @@ int lxs_smm_init(void) {
   char path[4096];
   if (NULL == env) {
     if (EXIT_SUCCESS == lxs_smm_default_params(path, sizeof(path), "tune_multiply_MI355X.csv")) {
-      (void)libsmm_acc_params_load(path);
+      (void)lxs_smm_params_load(path, NULL, 1);
     }
   }
   else if ('0' != *env && '\0' != *env) {
@@ -805,20 +809,39 @@ static int lxs_smm_rule(int datatype, int m, int n, int k, int stack_size, libsm
 }
 
 /* the configuration of one stack: a tuned row, the environment's or the caller's own model first, then the rule for
-   entry-parallel shapes, then the shipped predictor and the built-in heuristic */
+   entry-parallel shapes, then the shipped predictor and the built-in heuristic. Stacks too short to fill the device are
+   cut by lxs_smm_pieces where the configuration is this library's own choice: the rule or a row of the shipped file
+   without a short-stack pair. What the caller chose (a file, libsmm_acc_config_set, OPENCL_LIBSMM_SMM_*,
+   LIBXSTREAM_SMM_SPLIT) is launched as it is, bs scaled by its S. */
 static void lxs_smm_select(int datatype, int m, int n, int k, int stack_size, libsmm_acc_smm_config_t* config) {
   const lxs_smm_slot_t* slot;
   libsmm_acc_smm_config_t env;
-  int untuned;
+  int untuned, shipped, source = libsmm_acc_config_default;
   pthread_mutex_lock(&lxs_smm_lock);
   slot = lxs_smm_lookup(datatype, m, n, k, 0);
   untuned = (NULL == slot || libsmm_acc_config_learned == slot->source);
+  shipped = (NULL != slot && 0 != slot->shipped);
   pthread_mutex_unlock(&lxs_smm_lock);
   if (0 != untuned && 0 == lxs_learned_is_user() && EXIT_SUCCESS == lxs_smm_rule(datatype, m, n, k, stack_size, config)) {
     env = *config;
     if (0 == lxs_smm_env(&env)) return;
   }
-  lxs_smm_resolve(datatype, m, n, k, config, NULL);
+  lxs_smm_resolve(datatype, m, n, k, config, &source);
+  if (0 != shipped && libsmm_acc_config_tuned == source && 0 == config->bs_short && 2 <= config->variant &&
+      config->variant <= 4 && LXS_SMM_SPLIT_FILL > stack_size && stack_size < config->s &&
+      LXS_SMM_SPLIT_DEFAULT == lxs_cfg.split) {
+    int bs = config->bs, split = config->split;
+    lxs_smm_pieces(datatype, m, n, k, stack_size, config, &bs, &split);
+    if (4 == config->variant && 256 > config->nt) { /* few wavefronts per run were chosen for many runs */
+      const int nt = config->nt, kt = config->kt;
+      config->nt = 256;
+      config->kt = 16;
+      if (EXIT_SUCCESS != libsmm_acc_config_valid((libsmm_acc_data_t)datatype, m, n, k, config)) config->nt = nt, config->kt = kt;
+    }
+    config->bs = bs;
+    config->split = split;
+    config->s = 0; /* not scaled again */
+  }
 }
 
 /* the launch arguments of one stack under a configuration (bs scaling, short-stack pair, cut length) */
@@ -853,16 +876,6 @@ static void lxs_smm_fill(lxs_smm_args_t* out, const libsmm_acc_smm_config_t* con
     const long bs0 = args.bs, cbs = (bs0 > LXS_SMM_BS_MIN ? bs0 : LXS_SMM_BS_MIN);
     const long bs = ((long)stack_size * cbs + config->s - 2) / (config->s - 1);
     args.bs = (int)(bs < bs0 ? (1 > bs ? 1 : bs) : bs0);
-    if (2 <= config->variant && config->variant <= 4 && LXS_SMM_SPLIT_FILL > stack_size &&
-        LXS_SMM_SPLIT_DEFAULT == lxs_cfg.split) {
-      if (4 == config->variant && 256 > args.nt) { /* few wavefronts per run were chosen for many runs */
-        const int nt = args.nt, kt = args.kt;
-        args.nt = 256;
-        args.kt = 16;
-        if (0 == lxs_smm_available(datatype, 4, m, n, k, args.tm, args.tn, args.nt, args.kt)) args.nt = nt, args.kt = kt;
-      }
-      lxs_smm_pieces(datatype, m, n, k, stack_size, config, &args.bs, &split);
-    }
   }
   /* flush: atomic add, which is correct for any stack order (multiply.cl:657,687) and exact-once per
      element for a C-run that is not cut; flush 1 (plain read-modify-write) only when the caller has

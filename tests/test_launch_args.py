@@ -108,3 +108,47 @@ def test_long_k_result(tid):
         stream.close()
         lx.finalize()
     assert out[0] == expected
+
+
+# variant tm tn nt bs kt flush s split bs_short split_short
+TUNED = {"23x23x23": (lx.REAL_8, 23, 23, 23, "2 2 2 512 32 16 2 30000 3 0 0"), "5x5x5": (lx.REAL_4, 5, 5, 5, "4 2 2 64 24 64 2 30000 2 0 0")}
+
+
+def scaled(bs, stack_size, s):
+    """bs for a stack shorter than the s it was chosen for (smm_kernel.c:463-473)"""
+    return min(bs, max(1, -(-stack_size * max(bs, 32) // (s - 1)))) if s > 1 and stack_size < s else bs
+
+
+@pytest.mark.parametrize("name", sorted(TUNED))
+@pytest.mark.parametrize("entries", [300, 3000, 12000, 16383])
+def test_explicit_configurations_are_launched(launches, tmp_path, name, entries):
+    """what the caller sets (process_config, config_set, a file, the environment) is launched in short stacks: bs scaled
+    by s, its own cut factor, threads and k per stage"""
+    tid, m, n, k, text = TUNED[name]
+    _, _, _, nt, bs, kt, _, s, split, _, _ = map(int, text.split())
+    shape = "%d %d %d %d" % (tid, m, n, k)
+    path = tmp_path / "mine.csv"
+    v, tm, tn, _, _, _, fl, _, _, bss, sps = text.split()
+    path.write_text("DEVICE;TYPEID;M;N;K;S;GFLOPS;VARIANT;TM;TN;NT;BS;KT;FLUSH;SPLIT;BSS;SPLITS\n"
+                    "MI355X;%d;%d;%d;%d;%d;1.0;%s;%s;%s;%d;%d;%d;%s;%d;%s;%s\n" % (tid, m, n, k, s, v, tm, tn, nt, bs, kt, fl,
+                                                                                split, bss, sps))
+    process = "process %s %d" % (shape, entries)
+    made = [launches(["config %s %d %s" % (shape, entries, text)])[0][0],
+            launches(["set %s %s" % (shape, text), process])[1][0],
+            launches([process], OPENCL_LIBSMM_SMM_PARAMS=str(path))[0][0]]
+    expected = scaled(bs, entries, s)
+    for one in made:
+        assert len(one) == 1 and (one[0]["nt"], one[0]["kt"], one[0]["bs"]) == (nt, kt, expected), made
+        assert one[0]["tsplit"] == split * expected and one[0]["groups"] == -(-entries // expected)
+    env = launches([process], OPENCL_LIBSMM_SMM_BS="20")[0][0][0]
+    assert env["bs"] == scaled(20, entries, s)
+
+
+@pytest.mark.parametrize("entries", [300, 12000])
+def test_short_stack_pair_is_launched(launches, entries):
+    """bs_short and split_short of a configuration, for stacks of at most s entries"""
+    text = "2 2 2 512 32 16 2 16000 3 9 2"
+    for command in (["config 3 23 23 23 %d %s" % (entries, text)],
+                    ["set 3 23 23 23 " + text, "process 3 23 23 23 %d" % entries]):
+        (made,), _, rc = launches(command)[-1]
+        assert 0 == rc and made["bs"] == scaled(9, entries, 16000) and made["tsplit"] == 2 * made["bs"]
