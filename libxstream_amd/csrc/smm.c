@@ -831,13 +831,13 @@ static void lxs_smm_select(int datatype, int m, int n, int k, int stack_size, li
       config->variant <= 4 && LXS_SMM_SPLIT_FILL > stack_size && stack_size < config->s &&
       LXS_SMM_SPLIT_DEFAULT == lxs_cfg.split) {
     int bs = config->bs, split = config->split;
-    lxs_smm_pieces(datatype, m, n, k, stack_size, config, &bs, &split);
     if (4 == config->variant && 256 > config->nt) { /* few wavefronts per run were chosen for many runs */
       const int nt = config->nt, kt = config->kt;
       config->nt = 256;
       config->kt = 16;
       if (EXIT_SUCCESS != libsmm_acc_config_valid((libsmm_acc_data_t)datatype, m, n, k, config)) config->nt = nt, config->kt = kt;
     }
+    lxs_smm_pieces(datatype, m, n, k, stack_size, config, &bs, &split);
     config->bs = bs;
     config->split = split;
     config->s = 0; /* not scaled again */

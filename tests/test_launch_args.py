@@ -152,3 +152,15 @@ def test_short_stack_pair_is_launched(launches, entries):
                     ["set 3 23 23 23 " + text, "process 3 23 23 23 %d" % entries]):
         (made,), _, rc = launches(command)[-1]
         assert 0 == rc and made["bs"] == scaled(9, entries, 16000) and made["tsplit"] == 2 * made["bs"]
+
+
+@pytest.mark.parametrize("tid", [lx.REAL_8, lx.REAL_4])
+@pytest.mark.parametrize("entries", [300, 500, 750, 1500, 1800, 5000])
+def test_cut_follows_the_launched_wavefronts(launches, tid, entries):
+    """5x5x5: the shipped row (one wavefront per run at 30000 entries, four in short stacks) and the rule for shapes
+    without a row launch the same threads, so they cut the stack alike"""
+    commands = ["process %d 5 5 5 %d" % (tid, entries)]
+    row = launches(commands)[0][0][0]
+    rule = launches(commands, OPENCL_LIBSMM_SMM_PARAMS="0")[0][0][0]
+    assert row["nt"] == rule["nt"] == 256
+    assert (row["bs"], row["tsplit"]) == (rule["bs"], rule["tsplit"])
