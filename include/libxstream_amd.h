@@ -59,15 +59,15 @@ typedef struct libsmm_acc_smm_config_t {
 
 /** where a configuration came from */
 typedef enum libsmm_acc_config_source_t {
-  libsmm_acc_config_default = 0, /* built-in heuristic */
+  libsmm_acc_config_default = 0, /* built in: the rule by shape and stack size, or the heuristic */
   libsmm_acc_config_tuned = 1,   /* registry: CSV file, libsmm_acc_config_set or autotuner */
   libsmm_acc_config_env = 2,     /* OPENCL_LIBSMM_SMM_* environment overrides */
   libsmm_acc_config_learned = 3  /* learned predictor */
 } libsmm_acc_config_source_t;
 
-/** configuration libsmm_acc_process would use for this shape; *source may be NULL. For a shape whose source is the
- *  shipped predictor and whose C block has up to 16 tiles of 16x16, process chooses by the stack's size as well, and
- *  stacks shorter than the one a configuration was measured on get fewer entries per work-group */
+/** configuration libsmm_acc_process would use for this shape; *source may be NULL. A shape without a registered row whose
+ *  C block has up to 16 tiles of 16x16 gets a built-in choice by shape and stack size while the shipped predictor serves
+ *  with its default threshold: reported is the one for a stack of 30000 entries */
 LIBXSTREAM_API int libsmm_acc_config_get(libsmm_acc_data_t datatype, int m, int n, int k, libsmm_acc_smm_config_t* config,
   int* source);
 /** the built-in heuristic's configuration for this shape (ignores the registry and the predictor) */

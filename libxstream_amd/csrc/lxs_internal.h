@@ -60,8 +60,8 @@ void lxs_profile_finalize(void);
 
 /** learned predictor slot (mlp.c): EXIT_SUCCESS and a configuration when a confident model is installed */
 int lxs_learned_predict(int datatype, int m, int n, int k, libsmm_acc_smm_config_t* config);
-/** 1 when the installed model is the caller's (libsmm_acc_learned_set) and not the shipped one */
-int lxs_learned_is_user(void);
+/** 1 when the shipped model serves with its default confidence threshold */
+int lxs_learned_is_shipped(void);
 void lxs_learned_finalize(void);
 /** load a model file and install it as the predictor, owned by the library until finalize */
 void lxs_learned_load_default(const char* path);

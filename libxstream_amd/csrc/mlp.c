@@ -682,11 +682,12 @@ int lxs_learned_predict(int datatype, int m, int n, int k, libsmm_acc_smm_config
   return result;
 }
 
-/* a model that the caller installed (libsmm_acc_learned_set), not the shipped one or none */
-int lxs_learned_is_user(void) {
+/* the shipped model serves, without a threshold on its confidence (not the caller's model, LIBXSTREAM_LEARNED=0,
+   LIBXSTREAM_LEARNED_CONF or no model at all) */
+int lxs_learned_is_shipped(void) {
   int result;
   pthread_mutex_lock(&lxs_learned_lock);
-  result = (NULL != lxs_learned && lxs_learned_owned != lxs_learned);
+  result = (NULL != lxs_learned && lxs_learned_owned == lxs_learned && MLP_DEFAULT_CONF >= lxs_learned_conf);
   pthread_mutex_unlock(&lxs_learned_lock);
   return result;
 }

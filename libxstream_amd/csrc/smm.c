@@ -283,6 +283,8 @@ static int lxs_smm_env(libsmm_acc_smm_config_t* config) {
 static int lxs_smm_register(int datatype, int m, int n, int k, const libsmm_acc_smm_config_t* config, int source,
   int keep_best, int devmatch, int shipped);
 
+static void lxs_smm_select(int datatype, int m, int n, int k, int stack_size, libsmm_acc_smm_config_t* config, int* source);
+
 static void lxs_smm_resolve(int datatype, int m, int n, int k, libsmm_acc_smm_config_t* config, int* source) {
   const lxs_smm_slot_t* slot;
   int src = libsmm_acc_config_default;
@@ -328,10 +330,13 @@ LIBXSTREAM_API int libsmm_acc_config_heuristic(libsmm_acc_data_t datatype, int m
 
 LIBXSTREAM_API int libsmm_acc_config_get(libsmm_acc_data_t datatype, int m, int n, int k, libsmm_acc_smm_config_t* config,
   int* source) {
+  int src;
   if (NULL == config || 0 == lxs_typesize(datatype) || 0 >= m || 0 >= n || 0 >= k) {
     return lxs_error(EXIT_FAILURE, "libsmm_acc_config_get: invalid argument");
   }
-  lxs_smm_resolve((int)datatype, m, n, k, config, source);
+  lxs_smm_select((int)datatype, m, n, k, LXS_SMM_S, config, &src);
+  if (libsmm_acc_config_default == src && 0 == config->s) config->s = LXS_SMM_S; /* the rule's, for a stack of this size */
+  if (NULL != source) *source = src;
   return (0 < config->nt ? EXIT_SUCCESS : EXIT_FAILURE);
 }
 
@@ -808,26 +813,28 @@ static int lxs_smm_rule(int datatype, int m, int n, int k, int stack_size, libsm
   return EXIT_SUCCESS;
 }
 
-/* the configuration of one stack: a tuned row, the environment's or the caller's own model first, then the rule for
-   entry-parallel shapes, then the shipped predictor and the built-in heuristic. Stacks too short to fill the device are
+/* the configuration of one stack: a tuned row or the environment's first; then, in the place of the shipped predictor, the
+   rule for entry-parallel shapes; then the predictor (the shipped one for larger blocks, the caller's, or the shipped
+   one above the confidence that the caller asks for) and the built-in heuristic. Stacks too short to fill the device are
    cut by lxs_smm_pieces where the configuration is this library's own choice: the rule or a row of the shipped file
    without a short-stack pair. What the caller chose (a file, libsmm_acc_config_set, OPENCL_LIBSMM_SMM_*,
    LIBXSTREAM_SMM_SPLIT) is launched as it is, bs scaled by its S. */
-static void lxs_smm_select(int datatype, int m, int n, int k, int stack_size, libsmm_acc_smm_config_t* config) {
+static void lxs_smm_select(int datatype, int m, int n, int k, int stack_size, libsmm_acc_smm_config_t* config, int* source) {
   const lxs_smm_slot_t* slot;
   libsmm_acc_smm_config_t env;
-  int untuned, shipped, source = libsmm_acc_config_default;
+  int untuned, shipped;
   pthread_mutex_lock(&lxs_smm_lock);
   slot = lxs_smm_lookup(datatype, m, n, k, 0);
   untuned = (NULL == slot || libsmm_acc_config_learned == slot->source);
   shipped = (NULL != slot && 0 != slot->shipped);
   pthread_mutex_unlock(&lxs_smm_lock);
-  if (0 != untuned && 0 == lxs_learned_is_user() && EXIT_SUCCESS == lxs_smm_rule(datatype, m, n, k, stack_size, config)) {
+  *source = libsmm_acc_config_default;
+  if (0 != untuned && 0 != lxs_learned_is_shipped() && EXIT_SUCCESS == lxs_smm_rule(datatype, m, n, k, stack_size, config)) {
     env = *config;
     if (0 == lxs_smm_env(&env)) return;
   }
-  lxs_smm_resolve(datatype, m, n, k, config, &source);
-  if (0 != shipped && libsmm_acc_config_tuned == source && 0 == config->bs_short && 2 <= config->variant &&
+  lxs_smm_resolve(datatype, m, n, k, config, source);
+  if (0 != shipped && libsmm_acc_config_tuned == *source && 0 == config->bs_short && 2 <= config->variant &&
       config->variant <= 4 && LXS_SMM_SPLIT_FILL > stack_size && stack_size < config->s &&
       LXS_SMM_SPLIT_DEFAULT == lxs_cfg.split) {
     int bs = config->bs, split = config->split;
@@ -910,8 +917,9 @@ int lxs_smm_enqueue(int datatype, const int* dev_param_stack, int stack_size, co
   int m, int n, int k, int shared, void* hip_stream) {
   libsmm_acc_smm_config_t config;
   lxs_smm_args_t args;
+  int source;
   if (0 >= stack_size) return 0;
-  lxs_smm_select(datatype, m, n, k, stack_size, &config);
+  lxs_smm_select(datatype, m, n, k, stack_size, &config, &source);
   lxs_smm_fill(&args, &config, dev_param_stack, stack_size, datatype, a, b, c, m, n, k, 0,
     0 == shared ? lxs_cfg.grouped : 0);
   return lxs_smm_launch(&args, hip_stream);
@@ -920,7 +928,8 @@ int lxs_smm_enqueue(int datatype, const int* dev_param_stack, int stack_size, co
 /* whether lxs_smm_enqueue has a kernel for the stack (resolves, and caches where that applies, its configuration) */
 int lxs_smm_enqueue_ok(int datatype, int stack_size, int m, int n, int k) {
   libsmm_acc_smm_config_t config;
-  lxs_smm_select(datatype, m, n, k, stack_size, &config);
+  int source;
+  lxs_smm_select(datatype, m, n, k, stack_size, &config, &source);
   return EXIT_SUCCESS == libsmm_acc_config_valid((libsmm_acc_data_t)datatype, m, n, k, &config);
 }
 
@@ -960,7 +969,7 @@ static int lxs_smm_process(const int* dev_param_stack, int stack_size, libsmm_ac
   if (NULL == dev_param_stack || NULL == dev_a_data || NULL == dev_b_data || NULL == dev_c_data) {
     return lxs_error(EXIT_FAILURE, "libsmm_acc_process: NULL buffer");
   }
-  lxs_smm_select((int)datatype, m_max, n_max, k_max, stack_size, &config);
+  lxs_smm_select((int)datatype, m_max, n_max, k_max, stack_size, &config, &result);
   if (0 >= config.nt) return -1; /* no compiled kernel covers this shape: host fallback */
   result = lxs_smm_run(&config, dev_param_stack, stack_size, (int)datatype, dev_a_data, dev_b_data, dev_c_data, m_max,
     n_max, k_max, stack_stream, param_format, lxs_cfg.grouped);

@@ -164,3 +164,24 @@ def test_cut_follows_the_launched_wavefronts(launches, tid, entries):
     rule = launches(commands, OPENCL_LIBSMM_SMM_PARAMS="0")[0][0][0]
     assert row["nt"] == rule["nt"] == 256
     assert (row["bs"], row["tsplit"]) == (rule["bs"], rule["tsplit"])
+
+
+# without a row in the shipped file, up to 16 tiles of 16x16
+@pytest.mark.parametrize("shape", [(7, 9, 11), (16, 16, 5), (40, 20, 33), (60, 64, 9), (3, 4, 700)], ids=str)
+@pytest.mark.parametrize("tid", [lx.REAL_8, lx.REAL_4])
+def test_configuration_reported_and_predictor_switches(launches, tid, shape):
+    """config_get tells what process launches; the predictor switched off, cleared or held to a threshold that it misses
+    leads to the heuristic, as it does for larger blocks"""
+    name = "%d %d %d %d" % (tid, *shape)
+    commands = ["get " + name, "process %s 30000" % name, "process %s 500000" % name]
+    heuristic = lx.default_config(tid, *shape)
+    for env, clear in (({}, 0), (dict(LIBXSTREAM_LEARNED="0"), 0), (dict(LIBXSTREAM_LEARNED_CONF="1.5"), 0), ({}, 1)):
+        got, *made = launches(["clear"] * clear + commands, **env)[clear:]
+        source, variant, tm, tn, nt, bs, kt, flush, s, split, _, _ = got[1]
+        assert 0 == source and 30000 == s and 0 == got[2]
+        if env or clear:
+            assert (variant, tm, tn, nt, bs, kt) == (heuristic.variant, heuristic.tm, heuristic.tn, heuristic.nt,
+                                                     heuristic.bs, heuristic.kt)
+        for (one,), _, rc in made:
+            assert 0 == rc and (one["nt"], one["bs"]) == (nt, bs) and one["kt"] == (kt or one["kt"])
+            assert one["tsplit"] == max((split or 2) * bs, 64)
