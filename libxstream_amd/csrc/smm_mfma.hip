@@ -425,7 +425,6 @@ __device__ __forceinline__ void ep_body(T* __restrict__ cdata, const T* __restri
   for (int c = 0; c < GI; ++c) aoff[c] = lxs::group_start<T>(c, lxs::group_of<T>(c, TI), li, M);
 #pragma unroll
   for (int c = 0; c < GJ; ++c) boff[c] = lxs::group_start<T>(c, lxs::group_of<T>(c, TJ), li, N);
-  const T* const zeros = lxs::zeros<T>();
   /* B4: this lane's first A row r4 and first B column c4 (TI rows, TJ columns from there); element pairs start
      at min(row, M - 2) so they stay inside the block, and a pair whose first row is the last row of the block
      (a4x, b4x) holds that row in its second element (the first is the row before; read at use, so that no
@@ -702,7 +701,6 @@ __device__ __forceinline__ void ep_body(T* __restrict__ cdata, const T* __restri
     sync(); /* every sum is read before the next run's partials overwrite LDS */
     h = r;
   }
-#undef LXS_LOAD_KSTEP
 }
 
 #define LXS_EP_ARGS \
