@@ -151,6 +151,36 @@ __device__ __forceinline__ void gload_tiles(T* v, const T* p, const int* off) {
   if constexpr ((C + 1) * V < NTILE) gload_tiles<NTILE, C + 1>(v, p, off);
 }
 
+/* Sums over lanes without the LDS (DPP and the lane swaps of gfx950). Every lane l gets the sum over its row of 16
+   of the lanes with the same l % 4 (sum_row), or over all rows as well (sum_blocks); lanes 0 .. 3 of a row add
+   (x0 + x4) + (x8 + x12), then rows (0 + 1) + (2 + 3), the order that shuffles by 4, 8, 16, 32 give. */
+template <int N> /* the value of lane (l - N) mod 16 of the row */
+__device__ __forceinline__ float row_ror(float v) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x120 + N, 0xf, 0xf, true));
+}
+template <int N>
+__device__ __forceinline__ double row_ror(double v) {
+  typedef int i2_t __attribute__((ext_vector_type(2)));
+  i2_t w = __builtin_bit_cast(i2_t, v);
+  w.x = __builtin_amdgcn_update_dpp(0, w.x, 0x120 + N, 0xf, 0xf, true);
+  w.y = __builtin_amdgcn_update_dpp(0, w.y, 0x120 + N, 0xf, 0xf, true);
+  return __builtin_bit_cast(double, w);
+}
+template <typename T>
+__device__ __forceinline__ T sum_row(T v) {
+  v += row_ror<12>(v);
+  return v + row_ror<8>(v);
+}
+__device__ __forceinline__ float sum_blocks(float v) {
+  const unsigned int x = __builtin_bit_cast(unsigned int, sum_row(v));
+  const auto rows = __builtin_amdgcn_permlane16_swap(x, x, false, false);
+  const unsigned int r0 = rows[0], r1 = rows[1];
+  const unsigned int y = __builtin_bit_cast(unsigned int, __builtin_bit_cast(float, r0) + __builtin_bit_cast(float, r1));
+  const auto halves = __builtin_amdgcn_permlane32_swap(y, y, false, false);
+  const unsigned int h0 = halves[0], h1 = halves[1];
+  return __builtin_bit_cast(float, h0) + __builtin_bit_cast(float, h1);
+}
+
 /* Long C-runs are cut into pieces at the segment boundaries of the stack (multiples of the
    segment size bs, where one work-group's entries begin). Boundary entry i starts a new piece
    when the entry tsplit places earlier has the same C block ci: in a stack sorted by C, the run

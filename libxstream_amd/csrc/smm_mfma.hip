@@ -464,23 +464,20 @@ __device__ __forceinline__ void ep_body(T* __restrict__ cdata, const T* __restri
         if constexpr (2 == B4) {
           if constexpr (lxs::mfma4<T>::FP32) {
             /* sixteen k-blocks: lanes of one column j = l % 4 hold row i in register i, added over l ^ 4 .. l ^ 32 in
-               a fixed order; lanes 0..3 keep element 4 i + j */
+               a fixed order; lanes 4 i + j keep element (i, j) */
+            T v = lxs::sum_blocks(prod4[ti][tj][0]);
 #pragma unroll
-            for (int x = 0; x < 4; ++x) {
-              T v = prod4[ti][tj][x];
-              v += __shfl_xor(v, 4);
-              v += __shfl_xor(v, 8);
-              v += __shfl_xor(v, 16);
-              v += __shfl_xor(v, 32);
-              if (lane < 4) {
-                T* const slot = red + (q * NTILE + ti * TJ + tj) * 16 + 4 * x + lane;
-                *slot = (folded ? *slot : T(0)) + v;
-              }
+            for (int x = 1; x < 4; ++x) {
+              const T w = lxs::sum_blocks(prod4[ti][tj][x]);
+              v = (x == lane >> 2 ? w : v);
+            }
+            if (lane < 16) {
+              T* const slot = red + (q * NTILE + ti * TJ + tj) * 16 + lane;
+              *slot = (folded ? *slot : T(0)) + v;
             }
           }
           else { /* the four k-quarters of the block, added in a fixed order, then lanes 16 i + j */
-            const T v01 = prod4[ti][tj] + __shfl_xor(prod4[ti][tj], 4);
-            const T v = v01 + __shfl_xor(v01, 8);
+            const T v = lxs::sum_row(prod4[ti][tj]);
             if (0 == g4) {
               T* const slot = red + (q * NTILE + ti * TJ + tj) * 16 + ((lane >> 4) << 2) + (lane & 3);
               *slot = (folded ? *slot : T(0)) + v;
