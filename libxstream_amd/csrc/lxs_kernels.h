@@ -31,6 +31,7 @@ typedef struct lxs_smm_args_t {
   int pfmt;          /* 0: 3-int records, 1-based offsets; else 6-int DBM task records (m, n, k, a, b, c),
                         0-based offsets (samples/smm/kernels/multiply.cl:96-99) */
   int tsplit;        /* C-runs longer than this are cut at segment boundaries (<= 0: never) */
+  int piece;         /* variants 2 to 4: multiple of bs at which they are cut (0: bs) */
 } lxs_smm_args_t;
 
 /** number of LDS bytes the stack kernel needs for this configuration (0 if invalid) */

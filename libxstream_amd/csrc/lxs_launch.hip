@@ -327,14 +327,14 @@ extern "C" int lxs_smm_specialised(int dtype, int variant, int m, int n, int k, 
 }
 
 extern "C" int lxs_smm_launch(const lxs_smm_args_t* a, void* hip_stream) {
-  int kt, bs, atomic, ps, pz, tsplit = a->tsplit, stack_size = a->stack_size, m = a->m, n = a->n, k = a->k;
+  int kt, bs, piece, atomic, ps, pz, tsplit = a->tsplit, stack_size = a->stack_size, m = a->m, n = a->n, k = a->k;
   size_t lds;
   unsigned int nblocks;
   const void* fn;
   void* c;
   const void *pa, *pb;
   const int* stack;
-  void* args[14];
+  void* args[15];
   if (2 <= a->variant && a->variant <= 4 && ep_k_max < k) { /* parts of k, each one launch that adds to C */
     const size_t ts = (3 == a->dtype ? 8 : 4);
     int k0, result = 0;
@@ -366,6 +366,8 @@ extern "C" int lxs_smm_launch(const lxs_smm_args_t* a, void* hip_stream) {
   }
   if (0 >= stack_size) return 0;
   bs = (0 < a->bs ? a->bs : 32);
+  piece = (0 < a->piece ? a->piece : bs);
+  if (0 != piece % bs) return LXS_ELIMIT;
   nblocks = (unsigned int)((stack_size + bs - 1) / bs);
   atomic = a->atomic;
   c = a->c;
@@ -389,6 +391,7 @@ extern "C" int lxs_smm_launch(const lxs_smm_args_t* a, void* hip_stream) {
   args[11] = &ps;
   args[12] = &pz;
   args[13] = &tsplit;
+  args[14] = &piece; /* the entry-parallel kernels' */
   return (int)hipLaunchKernel(fn, dim3(nblocks), dim3((unsigned int)a->nt), args, lds, (hipStream_t)hip_stream);
 }
 

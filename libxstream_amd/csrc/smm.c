@@ -283,7 +283,8 @@ static int lxs_smm_env(libsmm_acc_smm_config_t* config) {
 static int lxs_smm_register(int datatype, int m, int n, int k, const libsmm_acc_smm_config_t* config, int source,
   int keep_best, int devmatch, int shipped);
 
-static void lxs_smm_select(int datatype, int m, int n, int k, int stack_size, libsmm_acc_smm_config_t* config, int* source);
+static void lxs_smm_select(int datatype, int m, int n, int k, int stack_size, libsmm_acc_smm_config_t* config, int* piece,
+  int* source);
 
 static void lxs_smm_resolve(int datatype, int m, int n, int k, libsmm_acc_smm_config_t* config, int* source) {
   const lxs_smm_slot_t* slot;
@@ -330,11 +331,11 @@ LIBXSTREAM_API int libsmm_acc_config_heuristic(libsmm_acc_data_t datatype, int m
 
 LIBXSTREAM_API int libsmm_acc_config_get(libsmm_acc_data_t datatype, int m, int n, int k, libsmm_acc_smm_config_t* config,
   int* source) {
-  int src;
+  int src, piece;
   if (NULL == config || 0 == lxs_typesize(datatype) || 0 >= m || 0 >= n || 0 >= k) {
     return lxs_error(EXIT_FAILURE, "libsmm_acc_config_get: invalid argument");
   }
-  lxs_smm_select((int)datatype, m, n, k, LXS_SMM_S, config, &src);
+  lxs_smm_select((int)datatype, m, n, k, LXS_SMM_S, config, &piece, &src);
   if (libsmm_acc_config_default == src && 0 == config->s) config->s = LXS_SMM_S; /* the rule's, for a stack of this size */
   if (NULL != source) *source = src;
   return (0 < config->nt ? EXIT_SUCCESS : EXIT_FAILURE);
@@ -719,7 +720,8 @@ LIBXSTREAM_API c_dbcsr_acc_bool_t libsmm_acc_process_suitable(c_dbcsr_acc_bool_t
 
 /* A C-run is summed by the work-group where it starts, unless it is longer than tsplit = split x bs
    entries (the configuration's split, else LIBXSTREAM_SMM_SPLIT, default 2; LIBXSTREAM_SMM_SPLIT=0 never
-   cuts): then it is cut at work-group boundaries and its pieces are added with atomics, so one long run
+   cuts): then it is cut at work-group boundaries (lxs_smm_args_t.piece: at some of them) and its pieces are added with
+   atomics, so one long run
    (many k-blocks into one C block) does not leave a single work-group working alone. Floor: in a stack of
    at least LXS_SMM_SPLIT_FILL entries (enough C-runs to occupy the device), runs of up to 64 entries are
    never cut: each is summed in one work-group in a fixed order and written once, so its C block gets the
@@ -733,41 +735,50 @@ int lxs_smm_tsplit(int bs, int split, int stack_size) {
   return (0 < lxs_cfg.split ? (floor < t ? t : floor) : 0);
 }
 
+static int lxs_smm_clamp(int v, int lo, int hi) { return (v < lo ? lo : (hi < v ? hi : v)); }
+
 /*
- * Stack entries per work-group and cut factor of an entry-parallel kernel on a stack too short to fill the device
- * with whole runs (fewer than LXS_SMM_SPLIT_FILL entries). Cutting a run into pieces shortens its chain of k-steps
- * but adds an atomic update of C per piece, so it pays by x = 1000 k (padded / useful area of C) / (wavefronts x
- * entries); over 19 shapes x 9 sizes from 300 to 7000 entries in runs of about 30, the geometric mean of the time
- * against the best of ten choices, FP64 on 16x16 tiles: x < 2.2 whole 0.98-1.00 (pieces of 8: 0.68-0.86), 3.5-8 pieces
- * of 8 0.93 (whole 0.83-0.75), 8-50 pieces of 4 0.95-0.99 (whole 0.60-0.45), above 1 to 2 entries. The lines lie lower on
- * 4x4 blocks and higher in FP32, whose products take half the time and whose atomics do not (whole 0.93 at x = 6.7-10).
- * Whole runs: a work-group takes the runs that begin among its entries, so fewer entries than a run has leave it one
- * run (32: 0.53-0.68 of the best at 3000 to 10000 entries). Blocks above 16x16 keep a CU busy with one work-group, and two of
- * them with a run on one CU, next to others without any, cost twice the time: at most 250 work-groups while a run is
- * longer than their share, then 24 entries (us by entries per work-group: FP32 64x64x64 S=3000 12 46, 10 78; 32x32x32 S=3000 12
- * 11.2, 6 16.8; 23x23x23 S=10000 24 14.3, 16 17.1; FP64 23x23x23 S=4000 16 10.3, 8 16.3; 64x64x64 S=12000 24 158, 16 227).
- * Smaller blocks: up to 500 work-groups and 16 entries, which cost runs of 30 nothing and help stacks of short runs (FP32
- * 8x8x8 S=10000 in runs of 1: 16 53 us, 24 74).
+ * Stack entries per work-group (bs), the length up to which runs stay whole (split x bs) and the pieces of longer ones, of
+ * an entry-parallel kernel on a stack too short to fill the device (fewer than LXS_SMM_SPLIT_FILL entries). A piece has
+ * a shorter chain of k-steps than its run but its own atomic update of C, so pieces are short where the chain is long
+ * against the stack: x = 1000 k (padded / useful area of C) / (wavefronts x entries). Few entries per work-group keep stacks
+ * of short runs, which say nothing of themselves here, on many work-groups; a longer run leaves all but the first of
+ * the work-groups of a piece without work.
+ * The lines are the best of 12 choices of bs x 11 of pieces in each of 11 ranges of x, over 11 shapes, both types, 300 to
+ * 15000 entries and runs of 1, 4, 10, 30, 100 and 1000 (902 stacks), a loss against one bs = entries / 1000 for every shape
+ * counted five times. Against that (and the kernels it was for), geometric mean over 14 shapes, both types and 7 sizes, by
+ * runs of 1, 2, 4, 10, 30, 100 and 1000: 1.37, 1.35, 1.32, 1.44, 1.47, 1.54 and 2.50; with 250 to 500 work-groups of pieces
+ * that suit runs of about 30, whatever the stack: 1.05, 1.13, 1.19, 1.30, 1.41, 1.27 and 1.94, and 0.31 for single entries of
+ * FP32 5x5x5 (S=10000: 15.9 -> 51.7 us; now 21.3, the most that this rule loses in a larger stack next to FP64 32x32x32
+ * in runs of 100, S=7000: 23.5 -> 34.2).
  */
 static void lxs_smm_pieces(int datatype, int m, int n, int k, int stack_size, const libsmm_acc_smm_config_t* config, int* bs,
-  int* split) {
+  int* split, int* piece) {
   const int tile = (2 == config->variant ? 16 : (3 == config->variant ? 8 : 4)), ep = config->nt / 64;
   const double area = (double)(config->tm * tile) * (config->tn * tile) / ((double)m * n);
   const double x = 1000.0 * k * area / ((double)ep * stack_size);
   const int f64 = (dbcsr_type_real_8 == datatype);
-  double lim[3]; /* whole runs up to lim[0], pieces of 8 up to lim[1], of 4 up to lim[2], then of 1 to 2 */
-  if (4 == config->variant) lim[0] = lim[1] = (f64 ? 7.0 : 17.0), lim[2] = (f64 ? 20.0 : 17.0);
-  else if (3 == config->variant) lim[0] = 1.5, lim[1] = 5.0, lim[2] = 30.0;
-  else if (0 != f64) lim[0] = 3.0, lim[1] = 8.0, lim[2] = 50.0;
-  else lim[0] = 9.0, lim[1] = 25.0, lim[2] = 150.0;
-  if (x < lim[0]) {
-    if (16 < m || 16 < n) *bs = (6000 <= stack_size ? 24 : (1000 <= stack_size ? stack_size / 250 : 4));
-    else *bs = (8000 <= stack_size ? 16 : (2000 <= stack_size ? stack_size / 500 : 4));
-    *split = 48 / *bs;
+  int whole; /* runs up to this length */
+  if (16 < m || 16 < n) {
+    if (3 == config->variant) *piece = (x < 1 ? 32 : (x < 6 ? 8 : (x < 40 ? 4 : 2)));
+    else if (0 != f64) *piece = (x < 2 ? 16 : (x < 10 ? 8 : (x < 50 ? 4 : 2)));
+    else *piece = (x < 3 ? 24 : (x < 12 ? 8 : (x < 70 ? 4 : 2)));
+    *bs = (8 <= *piece ? lxs_smm_clamp(stack_size / 500, 2, 8) : 1);
+    whole = (24 == *piece || (16 == *piece && x < 0.7) ? 40 : (8 == *piece ? 12 : *piece));
   }
-  else if (x < lim[1]) *bs = 8, *split = 1;
-  else if (x < lim[2]) *bs = 4, *split = 1;
-  else *bs = 1, *split = 2;
+  else if (4 != config->variant) {
+    *piece = (x < 3 ? (0 != f64 ? 8 : 16) : (x < 8 ? 8 : (x < 30 && 0 == f64 ? 4 : 2)));
+    *bs = (x < 3 ? lxs_smm_clamp(stack_size / 500, 4, 8) : (8 <= x && x < 30 ? 2 : 1));
+    whole = (16 == *piece ? 32 : (8 == *piece ? 12 : *piece));
+  }
+  else {
+    *piece = (x < (0 != f64 ? 1.5 : 3.0) ? 24 : (x < 8 ? 16 : 2));
+    *bs = (24 == *piece ? (0 != f64 ? lxs_smm_clamp(stack_size / 650, 4, 8) : lxs_smm_clamp(stack_size / 1000, 2, 8))
+                        : (16 == *piece ? lxs_smm_clamp(stack_size / 500, 2, 8) : 1));
+    whole = (24 == *piece ? 40 : (16 == *piece ? 32 : 2));
+  }
+  *piece = (*piece + *bs / 2) / *bs * *bs; /* pieces begin where work-groups do */
+  *split = (whole + *bs / 2) / *bs;
 }
 
 /*
@@ -783,7 +794,7 @@ static void lxs_smm_pieces(int datatype, int m, int n, int k, int stack_size, co
  * (11x11x33, 300 entries: FP64 6.7 us with 9 blocks, 5.5 with one tile; FP32 11.0 and 6.1). Everything else: 16x16 tiles,
  * 4 wavefronts per run (FP64 above 8 tiles: 2; short stacks of 2 to 4 tiles: 8).
  */
-static int lxs_smm_rule(int datatype, int m, int n, int k, int stack_size, libsmm_acc_smm_config_t* config) {
+static int lxs_smm_rule(int datatype, int m, int n, int k, int stack_size, libsmm_acc_smm_config_t* config, int* piece) {
   const int ti = (m + 15) / 16, tj = (n + 15) / 16, f64 = (dbcsr_type_real_8 == datatype);
   const int blocks = ((m + 3) / 4) * ((n + 3) / 4), shortened = (LXS_SMM_SPLIT_FILL > stack_size);
   const double steps = 30.0 * k / 16.0; /* 16-k steps of a run of 30 entries */
@@ -809,7 +820,7 @@ static int lxs_smm_rule(int datatype, int m, int n, int k, int stack_size, libsm
   config->split = 2;
   if (EXIT_SUCCESS != libsmm_acc_config_valid((libsmm_acc_data_t)datatype, m, n, k, config)) return EXIT_FAILURE;
   if (LXS_SMM_SPLIT_DEFAULT != lxs_cfg.split) config->split = 0; /* the caller's cut factor */
-  else if (0 != shortened) lxs_smm_pieces(datatype, m, n, k, stack_size, config, &config->bs, &config->split);
+  else if (0 != shortened) lxs_smm_pieces(datatype, m, n, k, stack_size, config, &config->bs, &config->split, piece);
   return EXIT_SUCCESS;
 }
 
@@ -819,7 +830,8 @@ static int lxs_smm_rule(int datatype, int m, int n, int k, int stack_size, libsm
    cut by lxs_smm_pieces where the configuration is this library's own choice: the rule or a row of the shipped file
    without a short-stack pair. What the caller chose (a file, libsmm_acc_config_set, OPENCL_LIBSMM_SMM_*,
    LIBXSTREAM_SMM_SPLIT) is launched as it is, bs scaled by its S. */
-static void lxs_smm_select(int datatype, int m, int n, int k, int stack_size, libsmm_acc_smm_config_t* config, int* source) {
+static void lxs_smm_select(int datatype, int m, int n, int k, int stack_size, libsmm_acc_smm_config_t* config, int* piece,
+  int* source) {
   const lxs_smm_slot_t* slot;
   libsmm_acc_smm_config_t env;
   int untuned, shipped;
@@ -828,10 +840,12 @@ static void lxs_smm_select(int datatype, int m, int n, int k, int stack_size, li
   untuned = (NULL == slot || libsmm_acc_config_learned == slot->source);
   shipped = (NULL != slot && 0 != slot->shipped);
   pthread_mutex_unlock(&lxs_smm_lock);
+  *piece = 0;
   *source = libsmm_acc_config_default;
-  if (0 != untuned && 0 != lxs_learned_is_shipped() && EXIT_SUCCESS == lxs_smm_rule(datatype, m, n, k, stack_size, config)) {
+  if (0 != untuned && 0 != lxs_learned_is_shipped() && EXIT_SUCCESS == lxs_smm_rule(datatype, m, n, k, stack_size, config, piece)) {
     env = *config;
     if (0 == lxs_smm_env(&env)) return;
+    *piece = 0;
   }
   lxs_smm_resolve(datatype, m, n, k, config, source);
   if (0 != shipped && libsmm_acc_config_tuned == *source && 0 == config->bs_short && 2 <= config->variant &&
@@ -844,7 +858,7 @@ static void lxs_smm_select(int datatype, int m, int n, int k, int stack_size, li
       config->kt = 16;
       if (EXIT_SUCCESS != libsmm_acc_config_valid((libsmm_acc_data_t)datatype, m, n, k, config)) config->nt = nt, config->kt = kt;
     }
-    lxs_smm_pieces(datatype, m, n, k, stack_size, config, &bs, &split);
+    lxs_smm_pieces(datatype, m, n, k, stack_size, config, &bs, &split, piece);
     config->bs = bs;
     config->split = split;
     config->s = 0; /* not scaled again */
@@ -852,7 +866,7 @@ static void lxs_smm_select(int datatype, int m, int n, int k, int stack_size, li
 }
 
 /* the launch arguments of one stack under a configuration (bs scaling, short-stack pair, cut length) */
-static void lxs_smm_fill(lxs_smm_args_t* out, const libsmm_acc_smm_config_t* config, const int* dev_param_stack,
+static void lxs_smm_fill(lxs_smm_args_t* out, const libsmm_acc_smm_config_t* config, int piece, const int* dev_param_stack,
   int stack_size, int datatype, const void* a, const void* b, void* c, int m, int n, int k, int param_format,
   int grouped) {
   lxs_smm_args_t args;
@@ -891,10 +905,11 @@ static void lxs_smm_fill(lxs_smm_args_t* out, const libsmm_acc_smm_config_t* con
   args.atomic = (1 == config->flush && 0 != grouped) ? 0 : 1;
   args.pfmt = param_format;
   args.tsplit = lxs_smm_tsplit(args.bs, split, stack_size);
+  args.piece = piece;
   *out = args;
 }
 
-static int lxs_smm_run(const libsmm_acc_smm_config_t* config, const int* dev_param_stack, int stack_size,
+static int lxs_smm_run(const libsmm_acc_smm_config_t* config, int piece, const int* dev_param_stack, int stack_size,
   int datatype, const void* a, const void* b, void* c, int m, int n, int k, void* stream, int param_format,
   int grouped) {
   const hipStream_t hs = lxs_stream_hip((const libxstream_stream_t*)stream);
@@ -902,7 +917,7 @@ static int lxs_smm_run(const libsmm_acc_smm_config_t* config, const int* dev_par
   void* token;
   int result = lxs_ensure_device();
   if (EXIT_SUCCESS != result) return result;
-  lxs_smm_fill(&args, config, dev_param_stack, stack_size, datatype, a, b, c, m, n, k, param_format, grouped);
+  lxs_smm_fill(&args, config, piece, dev_param_stack, stack_size, datatype, a, b, c, m, n, k, param_format, grouped);
   token = lxs_profile_begin(hs);
   result = lxs_smm_launch(&args, (void*)hs);
   lxs_profile_end(token, hs, "smm", 2.0 * stack_size * m * n * k,
@@ -917,10 +932,10 @@ int lxs_smm_enqueue(int datatype, const int* dev_param_stack, int stack_size, co
   int m, int n, int k, int shared, void* hip_stream) {
   libsmm_acc_smm_config_t config;
   lxs_smm_args_t args;
-  int source;
+  int piece, source;
   if (0 >= stack_size) return 0;
-  lxs_smm_select(datatype, m, n, k, stack_size, &config, &source);
-  lxs_smm_fill(&args, &config, dev_param_stack, stack_size, datatype, a, b, c, m, n, k, 0,
+  lxs_smm_select(datatype, m, n, k, stack_size, &config, &piece, &source);
+  lxs_smm_fill(&args, &config, piece, dev_param_stack, stack_size, datatype, a, b, c, m, n, k, 0,
     0 == shared ? lxs_cfg.grouped : 0);
   return lxs_smm_launch(&args, hip_stream);
 }
@@ -928,8 +943,8 @@ int lxs_smm_enqueue(int datatype, const int* dev_param_stack, int stack_size, co
 /* whether lxs_smm_enqueue has a kernel for the stack (resolves, and caches where that applies, its configuration) */
 int lxs_smm_enqueue_ok(int datatype, int stack_size, int m, int n, int k) {
   libsmm_acc_smm_config_t config;
-  int source;
-  lxs_smm_select(datatype, m, n, k, stack_size, &config, &source);
+  int piece, source;
+  lxs_smm_select(datatype, m, n, k, stack_size, &config, &piece, &source);
   return EXIT_SUCCESS == libsmm_acc_config_valid((libsmm_acc_data_t)datatype, m, n, k, &config);
 }
 
@@ -945,7 +960,7 @@ LIBXSTREAM_API int libsmm_acc_process_config(const libsmm_acc_smm_config_t* conf
     return lxs_error(EXIT_FAILURE, "libsmm_acc_process_config: configuration not valid for this shape");
   }
   /* an explicit configuration with flush 1 is the caller's statement that the stack is grouped by C */
-  result = lxs_smm_run(config, dev_param_stack, stack_size, (int)datatype, dev_a_data, dev_b_data, dev_c_data, m, n, k,
+  result = lxs_smm_run(config, 0, dev_param_stack, stack_size, (int)datatype, dev_a_data, dev_b_data, dev_c_data, m, n, k,
     stream, 0, 1);
   return (0 <= result ? lxs_hip((hipError_t)result, "stack kernel launch") : lxs_error(result, "stack kernel launch"));
 }
@@ -962,20 +977,20 @@ static int lxs_smm_process(const int* dev_param_stack, int stack_size, libsmm_ac
   const void* dev_a_data, const void* dev_b_data, void* dev_c_data, int m_max, int n_max, int k_max, int max_kernel_dim,
   c_dbcsr_acc_bool_t def_mnk, void* stack_stream, int param_format) {
   libsmm_acc_smm_config_t config;
-  int result;
+  int result, piece;
   if (0 == libsmm_acc_process_suitable(def_mnk, datatype, stack_size, m_max, n_max, k_max, max_kernel_dim)) {
     return (0 < stack_size ? -1 : EXIT_SUCCESS); /* smm_kernel.c:524-526 */
   }
   if (NULL == dev_param_stack || NULL == dev_a_data || NULL == dev_b_data || NULL == dev_c_data) {
     return lxs_error(EXIT_FAILURE, "libsmm_acc_process: NULL buffer");
   }
-  lxs_smm_select((int)datatype, m_max, n_max, k_max, stack_size, &config, &result);
+  lxs_smm_select((int)datatype, m_max, n_max, k_max, stack_size, &config, &piece, &result);
   if (0 >= config.nt) return -1; /* no compiled kernel covers this shape: host fallback */
-  result = lxs_smm_run(&config, dev_param_stack, stack_size, (int)datatype, dev_a_data, dev_b_data, dev_c_data, m_max,
+  result = lxs_smm_run(&config, piece, dev_param_stack, stack_size, (int)datatype, dev_a_data, dev_b_data, dev_c_data, m_max,
     n_max, k_max, stack_stream, param_format, lxs_cfg.grouped);
   if (LXS_ENOVARIANT == result || LXS_ELIMIT == result) {
     if (EXIT_SUCCESS != lxs_smm_default((int)datatype, m_max, n_max, k_max, &config)) return -1;
-    result = lxs_smm_run(&config, dev_param_stack, stack_size, (int)datatype, dev_a_data, dev_b_data, dev_c_data,
+    result = lxs_smm_run(&config, 0, dev_param_stack, stack_size, (int)datatype, dev_a_data, dev_b_data, dev_c_data,
       m_max, n_max, k_max, stack_stream, param_format, lxs_cfg.grouped);
     if (0 > result) return -1;
   }

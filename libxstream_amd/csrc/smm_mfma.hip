@@ -274,7 +274,8 @@ __global__ void __launch_bounds__(64 * NWI) smm_mfma(T* __restrict__ cdata, cons
  * the bits, do not depend on where the run lies in the work-group's share.
  * Run ownership and cuts as in smm_mfma: the work-group owns the runs whose first entry lies in
  * [w*bs, (w+1)*bs); a run continues past that range until its C block changes or a segment boundary
- * past it cuts the run (lxs_cut). The end of a run is found by a 64-wide ballot over the C indices
+ * past it cuts the run (lxs_cut), here one that lies on a multiple of piece, which is one of bs: short stacks take
+ * few entries per work-group and longer pieces. The end of a run is found by a 64-wide ballot over the C indices
  * (every wavefront computes it, so all take the same path through the barriers).
  * Barriers wait for LDS only (a fence restricted to the local address space).
  *
@@ -303,10 +304,11 @@ __global__ void __launch_bounds__(64 * NWI) smm_mfma(T* __restrict__ cdata, cons
  * l, l ^ 4, l ^ 8, l ^ 12, keeping element (i, j) in lane 16 i + j; FP32: lanes l ^ 4 .. l ^ 32, keeping row i
  * of column j in register i of lane j).
  */
+constexpr int SPREAD_CUS = 256;
 template <typename T, int TI, int TJ, int EP, int KB, int MC, int NC, int KC, int B4>
 __device__ __forceinline__ void ep_body(T* __restrict__ cdata, const T* __restrict__ adata,
   const T* __restrict__ bdata, const int* __restrict__ stack, int stack_size, int bs, int m_rt, int n_rt, int k_rt,
-  int kt_unused, int atomic, int ps, int pz, int tsplit) {
+  int kt_unused, int atomic, int ps, int pz, int tsplit, int piece) {
   typedef typename mfma<T>::acc_t acc_t;
   constexpr int SEG_LEN = 16; /* entries per matrix-core accumulation before the fold into the run total */
   constexpr int NTILE = TI * TJ; /* 16x16 tiles, or (B4) 4x4-block instructions per k-step */
@@ -328,7 +330,19 @@ __device__ __forceinline__ void ep_body(T* __restrict__ cdata, const T* __restri
   int tb;
   (void)kt_unused;
 
-  const int begin = blockIdx.x * bs;
+  /* this work-group's segment of the stack. Work-groups are placed in turn, so that w, w + 256, .. meet on one CU: where
+     one of them keeps a CU busy (blocks above one tile), they take neighbouring segments, of which a run longer than a
+     segment leaves only one work, and not two runs on one CU next to others without any. Five shapes above one tile,
+     both types, against segments in order, by stack size: 1000 to 7000 entries in runs of 30 1.07 to 1.35x, of 100 1.13
+     to 1.23, of 1000 1.05 to 1.19; runs of 1 to 4 0.98 to 1.04 (1.15 at 1000); 30000 in runs of 100 1.19;
+     from 100000 0.99 to 1.02. One stack lost more, FP64 64x64x64, 7000 entries in runs of 30 (114 -> 147 us). */
+  constexpr bool SPREAD = (2 != B4 && 1 < NTILE);
+  int seg = blockIdx.x;
+  if (SPREAD && SPREAD_CUS < gridDim.x) {
+    const int x = seg % SPREAD_CUS, share = gridDim.x / SPREAD_CUS;
+    seg = x * share + min(x, (int)gridDim.x % SPREAD_CUS) + seg / SPREAD_CUS;
+  }
+  const int begin = seg * bs;
   const int end = min(begin + bs, stack_size);
   /* WIN: the stack around the work-group's entries is held in registers: lane l has the C offset of
      entry begin + l and the C offset of entry begin - 64 + l (NONE outside the stack). The head and run-end
@@ -369,7 +383,7 @@ __device__ __forceinline__ void ep_body(T* __restrict__ cdata, const T* __restri
     /* C offset of the entry before each lane's: lanes 1..63 read lane l - 1 of wc, lane 0 reads lane 63 of
        the source, which holds entry begin - 1 (one shuffle, no lane-dependent select around a cross-lane read) */
     const int cprev = __shfl(63 == lane ? pc : wc, (lane + 63) & 63);
-    const int ccut = ((0 < tsplit && tsplit <= begin) ? c_uni(begin - tsplit) : NONE);
+    const int ccut = ((0 < tsplit && tsplit <= begin && 0 == begin % piece) ? c_uni(begin - tsplit) : NONE);
     const bool head = (wi < end) && (0 == wi || wc != cprev || (wi == begin && ccut == wc));
     const unsigned long long mask = __ballot(head);
     if (0 != mask) h = begin + __ffsll((long long)mask) - 1;
@@ -380,7 +394,7 @@ __device__ __forceinline__ void ep_body(T* __restrict__ cdata, const T* __restri
     bool head = false;
     if (i < end) {
       head = (0 == i) || (stack[ps * i + 2] != stack[ps * (i - 1) + 2]) ||
-             (i == begin && lxs_cut(stack, ps, i, stack[ps * i + 2], tsplit));
+             (i == begin && 0 == i % piece && lxs_cut(stack, ps, i, stack[ps * i + 2], tsplit));
     }
     const unsigned long long mask = __ballot(head);
     if (0 != mask) h = base + __ffsll((long long)mask) - 1;
@@ -393,7 +407,7 @@ __device__ __forceinline__ void ep_body(T* __restrict__ cdata, const T* __restri
     if constexpr (WIN) {
       if (h0 + 1 < begin + 64) {
         const int jc = wi - tsplit;
-        const bool bnd = (end <= wi && 0 == (wi - end) % bs && 0 < tsplit && tsplit <= wi);
+        const bool bnd = (end <= wi && 0 == wi % piece && 0 < tsplit && tsplit <= wi);
         const int x = __shfl(pc, (jc - begin + 64) & 63), y = __shfl(wc, (jc - begin) & 63);
         const bool need = (bnd && wc == c0); /* the cut test decides this lane */
         const bool inwin = (begin - 64 <= jc && jc < begin + 64);
@@ -409,7 +423,7 @@ __device__ __forceinline__ void ep_body(T* __restrict__ cdata, const T* __restri
       const int i = b0 + lane;
       bool stop = (i >= stack_size);
       if (!stop) {
-        stop = (stack[ps * i + 2] != c0) || (end <= i && 0 == (i - end) % bs && lxs_cut(stack, ps, i, c0, tsplit));
+        stop = (stack[ps * i + 2] != c0) || (end <= i && 0 == i % piece && lxs_cut(stack, ps, i, c0, tsplit));
       }
       const unsigned long long mask = __ballot(stop);
       if (0 != mask) return b0 + __ffsll((long long)mask) - 1;
@@ -702,8 +716,8 @@ __device__ __forceinline__ void ep_body(T* __restrict__ cdata, const T* __restri
 
 #define LXS_EP_ARGS \
   T* __restrict__ cdata, const T* __restrict__ adata, const T* __restrict__ bdata, const int* __restrict__ stack, \
-    int stack_size, int bs, int m_rt, int n_rt, int k_rt, int kt_unused, int atomic, int ps, int pz, int tsplit
-#define LXS_EP_PASS cdata, adata, bdata, stack, stack_size, bs, m_rt, n_rt, k_rt, kt_unused, atomic, ps, pz, tsplit
+    int stack_size, int bs, int m_rt, int n_rt, int k_rt, int kt_unused, int atomic, int ps, int pz, int tsplit, int piece
+#define LXS_EP_PASS cdata, adata, bdata, stack, stack_size, bs, m_rt, n_rt, k_rt, kt_unused, atomic, ps, pz, tsplit, piece
 
 template <typename T, int TI, int TJ, int EP, int KB, int MC, int NC, int KC>
 __global__ void __launch_bounds__(64 * EP, (TI * TJ <= 4 ? (2 == EP && 6 == KB ? 3 : 4) : (4 == sizeof(T) && TI * TJ <= 9 ? 4 : 1))) smm_mfma_ep(LXS_EP_ARGS) {

@@ -7,7 +7,7 @@
  *   get     TYPE M N K                        libsmm_acc_config_get
  *   clear                                     libsmm_acc_learned_set(NULL)
  * <configuration>: variant tm tn nt bs kt flush s split bs_short split_short. Output: for every launch
- *   launch <groups> <threads> <bs> <k> <kt> <tsplit> <atomic> <byte offset of A> <byte offset of B>
+ *   launch <groups> <threads> <bs> <k> <kt> <tsplit> <atomic> <byte offset of A> <byte offset of B> <piece>
  * for get "config <source> <configuration>", then "rc <result>" for every command.
  */
 #include <hip/hip_runtime.h>
@@ -38,8 +38,9 @@ hipError_t hipLaunchKernel(const void* fn, dim3 grid, dim3 block, void** args, s
   (void)fn;
   (void)lds;
   (void)stream;
-  printf("launch %u %u %d %d %d %d %d %ld %ld\n", grid.x, block.x, *(int*)args[5], *(int*)args[8], *(int*)args[9],
-    *(int*)args[13], *(int*)args[10], (long)(*(char**)args[1] - apool), (long)(*(char**)args[2] - bpool));
+  printf("launch %u %u %d %d %d %d %d %ld %ld %d\n", grid.x, block.x, *(int*)args[5], *(int*)args[8], *(int*)args[9],
+    *(int*)args[13], *(int*)args[10], (long)(*(char**)args[1] - apool), (long)(*(char**)args[2] - bpool),
+    *(int*)args[14]);
   return hipSuccess;
 }
 

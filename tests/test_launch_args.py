@@ -40,7 +40,7 @@ def launches(tmp_path_factory):
         for line in out.stdout.splitlines():
             word, *values = line.split()
             if word == "launch":
-                made.append(dict(zip(("groups", "nt", "bs", "k", "kt", "tsplit", "atomic", "a", "b"), map(int, values))))
+                made.append(dict(zip(("groups", "nt", "bs", "k", "kt", "tsplit", "atomic", "a", "b", "piece"), map(int, values))))
             elif word == "config":
                 config = tuple(map(int, values))
             elif word == "rc":
@@ -185,3 +185,20 @@ def test_configuration_reported_and_predictor_switches(launches, tid, shape):
         for (one,), _, rc in made:
             assert 0 == rc and (one["nt"], one["bs"]) == (nt, bs) and one["kt"] == (kt or one["kt"])
             assert one["tsplit"] == max((split or 2) * bs, 64)
+
+
+@pytest.mark.parametrize("tid", [lx.REAL_8, lx.REAL_4])
+@pytest.mark.parametrize("shape", [(23, 23, 23), (13, 13, 13), (5, 5, 5), (45, 45, 13), (17, 3, 40), (6, 7, 70)],
+                         ids=lambda s: "%dx%dx%d" % s)
+def test_short_stacks_in_pieces(launches, tid, shape):
+    """short stacks: few entries per work-group, which begin the pieces of longer runs"""
+    sizes = (30, 300, 1000, 2000, 4000, 7000, 10000, 15000, 16383)
+    runs = launches(["process %d %d %d %d %d" % (tid, *shape, s) for s in sizes])
+    for size, (made, _, rc) in zip(sizes, runs):
+        assert 0 == rc and 1 == len(made)
+        launch = made[0]
+        assert 1 <= launch["bs"] <= 8 and launch["groups"] == (size + launch["bs"] - 1) // launch["bs"]
+        assert 0 == launch["piece"] % launch["bs"] and 2 <= launch["piece"] <= 36 and 0 < launch["tsplit"] <= 48
+    # an explicit configuration's own segments
+    for made, _, rc in launches(["config %d %d %d %d 4000 2 2 2 256 12 16 2 2 0 0 0" % (tid, *shape)]):
+        assert rc or (12 == made[0]["bs"] == made[0]["piece"])
