@@ -44,6 +44,12 @@ __device__ __forceinline__ int oz_some_pairs(unsigned int oa, unsigned int ob, i
 }
 /* all pairs up to the cutoff s - 1 or 2 (s - 1) */
 __host__ __device__ constexpr int oz_all_pairs(int s, int cutoff) { return (2 * (s - 1) == cutoff ? s * s : s * (s + 1) / 2); }
+/* products without branches, of zero planes and all: faster than branches above 0.65 of the pairs (4096^3, ms: 8 slices,
+   triangle, 24 of 36 pairs 2.29 with branches, 2.16 without; all pairs, 36 of 64 2.77 and 3.06), for 3 slices above 0.7
+   (4 of 6 pairs 0.594 with, 0.641 without) */
+__device__ __forceinline__ bool oz_branch_free(int some, int s, int cutoff) {
+  return 20 * some > (3 < s ? 13 : 14) * oz_all_pairs(s, cutoff);
+}
 /*
  * 1 when oz_level_gemm and oz_recombine, which move and multiply only the planes with digits, are faster than oz_pairs,
  * which moves every plane of a tile: the products of the pairs with digits, and int32 partials per level that cost about
@@ -51,13 +57,19 @@ __host__ __device__ constexpr int oz_all_pairs(int s, int cutoff) { return (2 * 
  * plane per 7), oz_pairs / the other two: 8192^3, 8 slices, triangle: 7 bits 11.5 / 1.6, 21 13.2 / 5.6, 35 16.0 / 12.3, 42
  * 15.7 / 14.9; 4096^3 all pairs 7 1.64 / 0.42, 28 2.2 / 1.47, 42 2.8 / 2.66; 8192x8192x1024 all pairs 28 2.34 / 2.23, 35
  * 2.58 / 2.97, 6 slices 28 1.79 / 2.15. The partials cost more where all pairs share a tile's loads.
+ * A triangle of few slices has few products for the planes that oz_pairs moves for a tile of 128 x 64 (3 slices: 2 pairs a
+ * plane, 8: 4.5), 1.5 times the time of 8 slices per pair, and the other two win with all planes from K = 4000 on (3 slices)
+ * and 6000 (4): 3 slices 8192^3 4.32 / 3.51, 3000x3000x16000 1.60 / 1.35, 5000^3 1.14 / 1.14, 8192x8192x2048 1.36 / 1.40;
+ * 4 slices 8192^3 6.46 / 5.43, 5500x5500x8192 2.94 / 2.89, 6000x6000x3000 1.26 / 1.48; 5 slices with 4 planes 8192^3 8.0 /
+ * 7.2, with all 7.91 / 7.85.
  */
 __device__ __forceinline__ bool oz_few_pairs(unsigned int oa, unsigned int ob, int s, int cutoff, int Kp) {
   unsigned int levels;
-  const int some = oz_some_pairs(oa, ob, s, cutoff, levels);
+  const int some = oz_some_pairs(oa, ob, s, cutoff, levels), all = oz_all_pairs(s, cutoff);
+  long cost = (2 * (s - 1) == cutoff ? 75L : 92L); /* of a pair in oz_pairs, in hundredths */
+  if (s - 1 == cutoff && 5 >= s && 20 * some > 13 * all) cost = (3 >= s ? 138L : (4 == s ? 120L : 103L));
   /* whole numbers: the three kernels of a call have to agree */
-  return 100L * ((long)some * Kp + 3000L * __popc(levels)) <=
-    (2 * (s - 1) == cutoff ? 75L : 92L) * oz_all_pairs(s, cutoff) * Kp;
+  return 100L * ((long)some * Kp + 3000L * __popc(levels)) <= cost * all * Kp;
 }
 
 /*
@@ -104,10 +116,8 @@ __global__ void __launch_bounds__(256) oz_pairs(const int8_t* __restrict__ pa, c
   unsigned int oa = oz_occupied(occa, NS), ob = oz_occupied(occb, NS); /* the planes to move and multiply */
   if (0 != gate && oz_few_pairs(oa, ob, NS, CUT, Kp)) return; /* oz_level_gemm's */
   {
-    /* above 0.65 of the pairs the products without branches are faster, zero planes and all (4096^3, 8 slices, ms:
-       triangle, 24 of 36 pairs 2.29 with branches, 2.16 without; all pairs, 36 of 64 2.77 and 3.06) */
     unsigned int levels;
-    if (20 * oz_some_pairs(oa, ob, NS, CUT, levels) > 13 * oz_all_pairs(NS, CUT)) oa = ob = EVERY;
+    if (oz_branch_free(oz_some_pairs(oa, ob, NS, CUT, levels), NS, CUT)) oa = ob = EVERY;
   }
   i16_t acc[CUT + 1][WI];
 #pragma unroll
