@@ -743,42 +743,42 @@ static int lxs_smm_clamp(int v, int lo, int hi) { return (v < lo ? lo : (hi < v 
  * a shorter chain of k-steps than its run but its own atomic update of C, so pieces are short where the chain is long
  * against the stack: x = 1000 k (padded / useful area of C) / (wavefronts x entries). Few entries per work-group keep stacks
  * of short runs, which say nothing of themselves here, on many work-groups; a longer run leaves all but the first of
- * the work-groups of a piece without work.
- * The lines are the best of 12 choices of bs x 11 of pieces in each of 11 ranges of x, over 11 shapes, both types, 300 to
- * 15000 entries and runs of 1, 4, 10, 30, 100 and 1000 (902 stacks), a loss against one bs = entries / 1000 for every shape
- * counted five times. Against that (and the kernels it was for), geometric mean over 14 shapes, both types and 7 sizes, by
- * runs of 1, 2, 4, 10, 30, 100 and 1000: 1.37, 1.35, 1.32, 1.44, 1.47, 1.54 and 2.50; with 250 to 500 work-groups of pieces
- * that suit runs of about 30, whatever the stack: 1.05, 1.13, 1.19, 1.30, 1.41, 1.27 and 1.94, and 0.31 for single entries of
- * FP32 5x5x5 (S=10000: 15.9 -> 51.7 us; now 21.3, the most that this rule loses in a larger stack next to FP64 32x32x32
- * in runs of 100, S=7000: 23.5 -> 34.2).
+ * the work-groups of a piece without work, so their number grows slowly with the stack.
+ * The lines are a fit to 10 choices of bs x 10 of pieces timed over 576 stacks (380 of random shapes with extents 4 to 64, the
+ * others of 14 shapes from 4x9x22 to 64x64x64), both types, 300 to 16383 entries, in runs of 1, 4, 10, 30 and 100. Geometric
+ * mean of the speed against one bs = entries / 1000 for every shape (and the kernels that it was for), by runs: 1.29, 1.24,
+ * 1.33, 1.45 and 1.58; with 250 to 500 work-groups of pieces that suit runs of about 30, whatever the stack: 1.00, 1.12,
+ * 1.25, 1.37 and 1.31, and 0.31 for single entries of FP32 5x5x5 (S=10000: 15.9 -> 51.7 us; now 21.4). 35 of the 2880 times
+ * are below 0.85: stacks of single entries in small blocks, and launches of 4 to 7 us.
  */
+typedef struct lxs_smm_pieces_t {
+  double x[3];            /* piece and whole for x below x[0], x[1], x[2], and above */
+  int piece[4], whole[4]; /* runs up to whole entries are not cut */
+  int groups, most;       /* bs = entries / groups, at most so many and one piece */
+} lxs_smm_pieces_t;
+
 static void lxs_smm_pieces(int datatype, int m, int n, int k, int stack_size, const libsmm_acc_smm_config_t* config, int* bs,
   int* split, int* piece) {
+  static const lxs_smm_pieces_t rules[7] = {
+    {{1.0, 6.0, 40.0}, {24, 8, 4, 2}, {40, 8, 6, 2}, 400, 12},   /* 4x4 blocks in quadrants */
+    {{3.0, 16.0, 16.0}, {24, 8, 4, 4}, {40, 8, 4, 4}, 400, 16},  /* 16x16 tiles, C above one tile: FP32 */
+    {{1.5, 8.0, 35.0}, {24, 8, 4, 2}, {40, 8, 4, 2}, 400, 16},   /* FP64 */
+    {{1.6, 10.0, 10.0}, {24, 8, 4, 4}, {40, 8, 4, 4}, 550, 16},  /* one tile: FP32 */
+    {{0.3, 1.4, 11.0}, {16, 8, 4, 2}, {32, 12, 6, 2}, 450, 16},  /* FP64 */
+    {{7.5, 12.0, 12.0}, {24, 16, 4, 4}, {40, 32, 6, 6}, 900, 8}, /* 4x4 blocks splitting k: FP32 */
+    {{1.2, 10.0, 10.0}, {24, 8, 2, 2}, {40, 12, 2, 2}, 600, 8}}; /* FP64 */
   const int tile = (2 == config->variant ? 16 : (3 == config->variant ? 8 : 4)), ep = config->nt / 64;
   const double area = (double)(config->tm * tile) * (config->tn * tile) / ((double)m * n);
   const double x = 1000.0 * k * area / ((double)ep * stack_size);
   const int f64 = (dbcsr_type_real_8 == datatype);
-  int whole; /* runs up to this length */
-  if (16 < m || 16 < n) {
-    if (3 == config->variant) *piece = (x < 1 ? 32 : (x < 6 ? 8 : (x < 40 ? 4 : 2)));
-    else if (0 != f64) *piece = (x < 2 ? 16 : (x < 10 ? 8 : (x < 50 ? 4 : 2)));
-    else *piece = (x < 3 ? 24 : (x < 12 ? 8 : (x < 70 ? 4 : 2)));
-    *bs = (8 <= *piece ? lxs_smm_clamp(stack_size / 500, 2, 8) : 1);
-    whole = (24 == *piece || (16 == *piece && x < 0.7) ? 40 : (8 == *piece ? 12 : *piece));
-  }
-  else if (4 != config->variant) {
-    *piece = (x < 3 ? (0 != f64 ? 8 : 16) : (x < 8 ? 8 : (x < 30 && 0 == f64 ? 4 : 2)));
-    *bs = (x < 3 ? lxs_smm_clamp(stack_size / 500, 4, 8) : (8 <= x && x < 30 ? 2 : 1));
-    whole = (16 == *piece ? 32 : (8 == *piece ? 12 : *piece));
-  }
-  else {
-    *piece = (x < (0 != f64 ? 1.5 : 3.0) ? 24 : (x < 8 ? 16 : 2));
-    *bs = (24 == *piece ? (0 != f64 ? lxs_smm_clamp(stack_size / 650, 4, 8) : lxs_smm_clamp(stack_size / 1000, 2, 8))
-                        : (16 == *piece ? lxs_smm_clamp(stack_size / 500, 2, 8) : 1));
-    whole = (24 == *piece ? 40 : (16 == *piece ? 32 : 2));
-  }
-  *piece = (*piece + *bs / 2) / *bs * *bs; /* pieces begin where work-groups do */
-  *split = (whole + *bs / 2) / *bs;
+  const lxs_smm_pieces_t* const r =
+    rules + (3 == config->variant ? 0 : (4 == config->variant ? 5 : (16 < m || 16 < n ? 1 : 3)) + f64);
+  const int i = (x < r->x[0] ? 0 : (x < r->x[1] ? 1 : (x < r->x[2] ? 2 : 3)));
+  int most = r->most;
+  if (6 == r - rules && 9000 <= stack_size) most = 12; /* runs of 30: 0.97 of the speed with 8, those of 1 1.08 */
+  *bs = lxs_smm_clamp(stack_size / r->groups, 1, r->piece[i] < most ? r->piece[i] : most);
+  *piece = (r->piece[i] + *bs / 2) / *bs * *bs; /* pieces begin where work-groups do */
+  *split = lxs_smm_clamp(r->whole[i] / *bs, 1, r->whole[i]);
 }
 
 /*

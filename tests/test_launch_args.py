@@ -197,8 +197,8 @@ def test_short_stacks_in_pieces(launches, tid, shape):
     for size, (made, _, rc) in zip(sizes, runs):
         assert 0 == rc and 1 == len(made)
         launch = made[0]
-        assert 1 <= launch["bs"] <= 8 and launch["groups"] == (size + launch["bs"] - 1) // launch["bs"]
-        assert 0 == launch["piece"] % launch["bs"] and 2 <= launch["piece"] <= 36 and 0 < launch["tsplit"] <= 48
+        assert 1 <= launch["bs"] <= 16 and launch["groups"] == (size + launch["bs"] - 1) // launch["bs"]
+        assert 0 == launch["piece"] % launch["bs"] and 1 <= launch["piece"] <= 32 and 0 < launch["tsplit"] <= 40
     # an explicit configuration's own segments
     for made, _, rc in launches(["config %d %d %d %d 4000 2 2 2 256 12 16 2 2 0 0 0" % (tid, *shape)]):
         assert rc or (12 == made[0]["bs"] == made[0]["piece"])
