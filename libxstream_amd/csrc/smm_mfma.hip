@@ -304,7 +304,7 @@ __global__ void __launch_bounds__(64 * NWI) smm_mfma(T* __restrict__ cdata, cons
  * l, l ^ 4, l ^ 8, l ^ 12, keeping element (i, j) in lane 16 i + j; FP32: lanes l ^ 4 .. l ^ 32, keeping row i
  * of column j in register i of lane j).
  */
-constexpr int SPREAD_CUS = 256;
+constexpr int SPREAD_CUS = 256, SPREAD_MAX = 8 * SPREAD_CUS;
 template <typename T, int TI, int TJ, int EP, int KB, int MC, int NC, int KC, int B4>
 __device__ __forceinline__ void ep_body(T* __restrict__ cdata, const T* __restrict__ adata,
   const T* __restrict__ bdata, const int* __restrict__ stack, int stack_size, int bs, int m_rt, int n_rt, int k_rt,
@@ -334,11 +334,12 @@ __device__ __forceinline__ void ep_body(T* __restrict__ cdata, const T* __restri
      one of them keeps a CU busy (blocks above one tile), they take neighbouring segments, of which a run longer than a
      segment leaves only one work, and not two runs on one CU next to others without any. Five shapes above one tile,
      both types, against segments in order, by stack size: 1000 to 7000 entries in runs of 30 1.07 to 1.35x, of 100 1.13
-     to 1.23, of 1000 1.05 to 1.19; runs of 1 to 4 0.98 to 1.04 (1.15 at 1000); 30000 in runs of 100 1.19;
-     from 100000 0.99 to 1.02. One stack lost more, FP64 64x64x64, 7000 entries in runs of 30 (114 -> 147 us). */
+     to 1.23, of 1000 1.05 to 1.19; runs of 1 to 4 0.98 to 1.04 (1.15 at 1000); 30000 in runs of 100 1.19. One stack lost
+     more, FP64 64x64x64, 7000 entries in runs of 30 (114 -> 147 us). Above 8 work-groups per CU they even out by
+     themselves: 100000 entries 0.96 to 1.05, FP32 45x45x13 in runs of 30 106.4 -> 107.9 us. */
   constexpr bool SPREAD = (2 != B4 && 1 < NTILE);
   int seg = blockIdx.x;
-  if (SPREAD && SPREAD_CUS < gridDim.x) {
+  if (SPREAD && SPREAD_CUS < gridDim.x && gridDim.x <= SPREAD_MAX) {
     const int x = seg % SPREAD_CUS, share = gridDim.x / SPREAD_CUS;
     seg = x * share + min(x, (int)gridDim.x % SPREAD_CUS) + seg / SPREAD_CUS;
   }

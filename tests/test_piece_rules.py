@@ -4,21 +4,21 @@ import numpy as np
 
 from tests.test_cut_rules import check, cut, stacks
 
-CUS = 256
+CUS, MOST = 256, 2048
 
 
 def segment(w, groups, spread):
     """the segment of work-group w of groups"""
-    if not spread or groups <= CUS:
+    if not spread or groups <= CUS or MOST < groups:
         return w
     x, share = w % CUS, groups // CUS
     return x * share + min(x, groups % CUS) + w // CUS
 
 
 def test_every_segment_once():
-    for groups in list(range(1, 600, 7)) + [255, 256, 257, 511, 512, 513, 4095, 8191, 8192, 8193]:
+    for groups in list(range(1, 600, 7)) + [255, 256, 257, 511, 512, 513, 2047, 2048, 2049, 4095]:
         assert sorted(segment(w, groups, True) for w in range(groups)) == list(range(groups))
-    for groups in (300, 1000, 8192):  # neighbours meet on one CU: w, w + 256, ..
+    for groups in (300, 1000, 2048):  # neighbours meet on one CU: w, w + 256, ..
         for x in range(0, CUS, 17):
             mine = [segment(w, groups, True) for w in range(x, groups, CUS)]
             assert mine == list(range(mine[0], mine[0] + len(mine)))
